@@ -1343,9 +1343,12 @@ k_restore(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         a.dst[q][s] = a.src[q][s];
     a.id_dst[s] = a.id_src[s];
     a.key_dst[s] = a.key_src[s];
-    if (blk * kTPB == P.poff)
-        for (unsigned c = threadIdx.x; c <= P.ncells; c += kTPB)
-            a.start_dst[P.cell_base + c] = a.start_src[P.cell_base + c];
+    // the scene's cell starts, shared by all of its workgroups: one workgroup
+    // copying them alone is a chain of ncells / 256 dependent rounds (920 us
+    // for the 960,000 cells of the 1M dam break, against 17 us shared)
+    const unsigned wg = blk - P.poff / kTPB, nwg = ((unsigned)P.n + P.pad) / kTPB;
+    for (unsigned long long c = wg * kTPB + threadIdx.x; c <= P.ncells; c += nwg * kTPB)
+        a.start_dst[P.cell_base + c] = a.start_src[P.cell_base + c];
 }
 
 __global__ void __launch_bounds__(kTPB)
