@@ -388,12 +388,15 @@ int sph_scene_lattice(fluid_particle *out, int nx, int ny, float x0, float y0, f
 
 /* Self-check of the kernels' correctly rounded square root (no counterpart
  * in the reference): counts the float bit patterns in [lo_bits, hi_bits)
- * whose sqrt differs from IEEE sqrtf (all NaNs count as equal). */
+ * whose sqrt differs from IEEE sqrtf (all NaNs count as equal), in either of
+ * the kernels' two forms (the pairs' common one over 2^-96..2^120). */
 int sph_selftest_sqrt(unsigned lo_bits, unsigned hi_bits, unsigned long long *mismatches);
 
 /* The same for the kernels' correctly rounded reciprocal against IEEE
  * division 1.0f / x over its domain (+-0, +-inf, NaN and 2^-126 <= |x| <=
- * 2^125; patterns outside it are skipped); no counterpart in the reference. */
+ * 2^125; patterns outside it are skipped), and for the pairs' common
+ * reciprocal of a root against 1.0f / sqrtf(x) over 2^-96..2^120; no
+ * counterpart in the reference. */
 int sph_selftest_rcp(unsigned lo_bits, unsigned hi_bits, unsigned long long *mismatches);
 
 /* ------------------------------------------------------------------------

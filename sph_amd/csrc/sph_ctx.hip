@@ -97,6 +97,8 @@ void derive_params(sph_ctx *c)
         p.bucket_cap = c->bucket_cap;
         int e = 0;
         p.h_pow2 = std::frexp(p.h, &e) == 0.5f && std::fpclassify(p.h_recip) == FP_NORMAL;
+        const float near_h2 = p.h2 * (1.0f - 0x1p-19f);
+        memcpy(&p.near_h2, &near_h2, sizeof near_h2);
     }
 }
 

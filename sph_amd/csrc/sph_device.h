@@ -37,6 +37,7 @@ struct sph_dev_params {
     int frozen;        // 1: the fused step leaves this scene's state unchanged
     int h_pow2;        // 1: h is a power of two with a normal reciprocal, so that
                        //    x / h == x * h_recip for every x (both round x 2^-k once)
+    unsigned near_h2;  // bits of a float a little below h^2 (sph_common_pair)
     unsigned bucket_cap; // 0, or the reference's per-cell bucket cap: a particle
                          // ranked bucket_cap or later by id in its cell is in
                          // no neighbour set of the hash (src/hash.c:153-164)
@@ -159,6 +160,67 @@ __device__ __forceinline__ bool sph_rcp_domain(float x)
     return !(ax > 0.0f && ax < 0x1p-126f) && !(ax > 0x1p125f && ax < __builtin_inff());
 }
 
+// Which instructions the pair terms are made of matters as much as how many.
+// A SIMD feeds two VALU pipes, each taking a wave64 instruction every 4
+// cycles: one takes all of them, the other only float add, multiply and FMA,
+// moves, bitwise logic, integer add and right shifts whose operands are VGPRs
+// or inline constants (measured: 0.9 ns an instruction against 1.8 for
+// compares, selects, min / max / med3, left shifts, bit counts, conversions,
+// double precision, DPP and anything with an SGPR operand, and 3.6 for the
+// reciprocal, the roots and exp2).  So the common path of a pair is written in
+// the first kind: uniform factors held in VGPRs (sph_vgpr), one root whose
+// refinement also gives the reciprocal, and one range test in the place of
+// every compare and select that only unusual pairs need.
+__device__ __forceinline__ float sph_vgpr(float x)
+{
+    asm("" : "+v"(x));
+    return x;
+}
+
+// Correctly rounded square root r of x and correctly rounded 1/r, for
+// 2^-96 <= x <= 2^120.  v_rsq_f32 gives y within an ulp of x^-1/2; g = x y is
+// corrected by its residual x - g^2 times y / 2, 1/r as in sph_rcp (each
+// residual formed by an FMA with one rounding).  Both equal IEEE sqrtf and
+// 1.0f / sqrtf for every x of the domain: checked exhaustively
+// (sph_selftest_sqrt, sph_selftest_rcp).  Two transcendentals and six cheap
+// instructions, where sph_sqrt and sph_rcp need eleven dear ones besides.
+// (Taking y as the reciprocal's seed as well saves v_rcp_f32, but misses the
+// r whose mantissa is all ones, and testing for those costs more.)
+struct sph_root {
+    float r, rinv;
+};
+
+__device__ __forceinline__ float sph_sqrt_common(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y, h = 0.5f * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+
+__device__ __forceinline__ sph_root sph_root_common(float x)
+{
+    sph_root q;
+    q.r = sph_sqrt_common(x);
+    const float z = __builtin_amdgcn_rcpf(q.r);
+    q.rinv = __builtin_fmaf(__builtin_fmaf(-q.r, z, 1.0f), z, z);
+    return q;
+}
+
+// Is a pair an uncommon one: not lo <= r2 < about h^2 (as bits; near_h2: h^2
+// (1 - 2^-19), so that r / h < 1 whatever the roundings)?  One unsigned
+// compare, true for zero, tiny, NaN and (h <= 2^60) too large r2.  Every pair
+// is evaluated the common way, with no compare but this one; when any lane of
+// the wave holds an uncommon pair - coincident particles, a pair at the very
+// edge of h, NaN - the wave evaluates its pairs again by the whole
+// expressions.
+constexpr unsigned kPairLoRoot = 0x0f800000u;  // 2^-96: the domain of sph_root_common
+constexpr unsigned kPairLoNudge = 0x2c000000u; // 2^-39 > (1e-6)^2: no nudge above
+__device__ __forceinline__ bool sph_uncommon_pair(float r2, unsigned lo, const sph_dev_params &P)
+{
+    const unsigned span = P.near_h2 > lo ? P.near_h2 - lo : 0u;
+    return __float_as_uint(r2) - lo >= span;
+}
+
 // src/fluid.c:613-625 without branches: the median of (v, -5, 5) is v
 // clamped to [-5, 5] (v_med3_f32); a NaN passes through unchanged, as in
 // the reference's if / else if.
@@ -221,36 +283,56 @@ __device__ __forceinline__ void sph_boundary(float &px, float &py, const sph_dev
 
 // src/fluid.c:591.  The literal 0.5 is a double, so the spring term, its
 // sum with the pressure terms and the product with dt*dt are double
-// operations, rounded to float once.
-__device__ __forceinline__ float sph_relax_D(float dt, float Psum, float Pnsum, float OmR,
+// operations, rounded to float once.  (double)s * 0.5 is exact, so that the
+// FMA rounds as the reference's sum does.
+__device__ __forceinline__ float sph_relax_D(double dt2, float Psum, float Pnsum, float OmR,
                                              float k_spring, float h, float r)
 {
     float a = Psum * OmR + Pnsum * OmR * OmR;
     float s = k_spring * (h - r);
-    float dt2 = dt * dt;
-    return (float)((double)dt2 * ((double)a + (double)s * 0.5));
+    return (float)(dt2 * __builtin_fma((double)s, 0.5, (double)a));
 }
 
-// src/fluid.c:442-459: impulse of pair (p, q) with p in the owner role.
-// Exactly antisymmetric in (p, q), so a particle in either role subtracts
-// half of the impulse computed with itself as p.
-// Evaluated unconditionally and returned with the test u > 0, so that the
-// caller applies it with selects (no branch in the pair loop).
-__device__ __forceinline__ bool sph_visc_impulse(float px, float py, float pvx, float pvy, float qx,
-                                                 float qy, float qvx, float qvy,
-                                                 const sph_dev_params &P, float &ix, float &iy)
+// src/fluid.c:442-478: impulse of pair (p, q) with p in the owner role, and
+// what p subtracts of it: half the clamped impulse if u > 0, else +0 (v - 0 ==
+// v).  Exactly antisymmetric in (p, q), so a particle in either role
+// subtracts half of the impulse computed with itself as p.  The common way
+// makes u <= 0 an impulse of zero (max) in the place of three selects; the
+// FMA with +0 halves it and turns -0 into +0.
+struct sph_visc_consts {
+    float h_recip, dt, sigma, beta;
+};
+
+__device__ __forceinline__ float2 sph_visc_half(float px, float py, float pvx, float pvy, float qx,
+                                                float qy, float qvx, float qvy,
+                                                const sph_visc_consts &V, const sph_dev_params &P)
 {
-    float QmP_x = qx - px;
-    float QmP_y = qy - py;
-    float r = sph_sqrt(QmP_x * QmP_x + QmP_y * QmP_y);
-    float r_recip = sph_rcp(r); // 1.0f / r
-    float ratio = r * P.h_recip;
-    float u = ((pvx - qvx) * QmP_x + (pvy - qvy) * QmP_y) * r_recip;
-    float imp = P.dt * (1.0f - ratio) * (P.sigma * u + P.beta * u * u);
-    ix = imp * QmP_x * r_recip;
-    iy = imp * QmP_y * r_recip;
-    sph_check_velocity(ix, iy);
-    return u > 0.0f;
+    const float QmP_x = qx - px;
+    const float QmP_y = qy - py;
+    const float r2 = QmP_x * QmP_x + QmP_y * QmP_y;
+    const float along = (pvx - qvx) * QmP_x + (pvy - qvy) * QmP_y;
+    const sph_root q = sph_root_common(r2);
+    const float u = __builtin_fmaxf(along * q.rinv, 0.0f);
+    const float imp = V.dt * (1.0f - q.r * V.h_recip) * (V.sigma * u + V.beta * u * u);
+    const float ix = imp * QmP_x * q.rinv;
+    const float iy = imp * QmP_y * q.rinv;
+    float hx = __builtin_fmaf(__builtin_amdgcn_fmed3f(ix, -5.0f, 5.0f), 0.5f, 0.0f);
+    float hy = __builtin_fmaf(__builtin_amdgcn_fmed3f(iy, -5.0f, 5.0f), 0.5f, 0.0f);
+    // a NaN passes through the clamp, and follows from no common u <= 0
+    if (__builtin_expect((__ballot(sph_uncommon_pair(r2, kPairLoRoot, P)) |
+                          __ballot(__builtin_isunordered(ix, iy))) != 0ull, 0)) {
+        const float r = sph_sqrt(r2);
+        const float r_recip = sph_rcp(r); // 1.0f / r
+        const float ratio = r * V.h_recip;
+        const float uu = along * r_recip;
+        const float im = V.dt * (1.0f - ratio) * (V.sigma * uu + V.beta * uu * uu);
+        float jx = im * QmP_x * r_recip;
+        float jy = im * QmP_y * r_recip;
+        sph_check_velocity(jx, jy);
+        hx = uu > 0.0f ? jx * 0.5f : 0.0f;
+        hy = uu > 0.0f ? jy * 0.5f : 0.0f;
+    }
+    return make_float2(hx, hy);
 }
 
 // Half-list owner rule of src/hash.c:176-237 for the pair (self at sorted
@@ -378,16 +460,17 @@ struct sph_masks_replay {
 // exactly the order of one lane per particle.
 struct sph_pair_term {
     float a, b; // the term's two components (zero: no update)
-    int f;      // an extra flag of the term (the relaxation's 1e-6 nudge)
 };
 
-// A pair body split in two for LP = 4: term(idx, own, rec) evaluates one
-// pair's contribution, apply(t) adds it to the particle's sums; apply of a
-// zero term with f = 0 must leave the sums unchanged bit for bit.
-template <class Term, class Apply>
+// A pair body split for LP = 4: term(idx, rec, own, nudged) evaluates one
+// pair's contribution, apply(t) adds it to the particle's sums (apply of a
+// zero term must leave them unchanged bit for bit), and where a term sets
+// nudged (the relaxation's coincident pairs), nudge(true) goes before it.
+template <class Term, class Apply, class Nudge>
 struct sph_split_body {
     Term term;
     Apply apply;
+    Nudge nudge;
 };
 
 __device__ __forceinline__ unsigned sph_quad_lane() { return __lane_id() & 3u; }
@@ -404,8 +487,7 @@ __device__ __forceinline__ sph_pair_term sph_quad_term(const sph_pair_term &t)
 {
     constexpr int kCtrl = J * 0x55;
     return sph_pair_term{__uint_as_float(sph_dpp<kCtrl>(__float_as_uint(t.a))),
-                         __uint_as_float(sph_dpp<kCtrl>(__float_as_uint(t.b))),
-                         (int)sph_dpp<kCtrl>((unsigned)t.f)};
+                         __uint_as_float(sph_dpp<kCtrl>(__float_as_uint(t.b)))};
 }
 
 // The same walk in two passes, for SIMD efficiency.  Pass 1 tests the
@@ -446,11 +528,11 @@ __device__ __forceinline__ sph_pair_term sph_quad_term(const sph_pair_term &t)
 // gives lane q the q-th pending pair of the head chunk, and the four terms
 // are applied by every lane in pair order.  Same chunks, same masks, same
 // sums as LP = 1, with a quarter of the serial work per lane.
-template <bool OWN = false, bool CAP = false, int DY0 = -1, int DY1 = 1, int LP = 1, class Src,
-          class Dist2, class Body, class Masks>
+template <bool CAP = false, int DY0 = -1, int DY1 = 1, int LP = 1, class Src, class Dist2,
+          class Body, class Masks, class Rows>
 __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R, const Src &src,
                                                float h2, unsigned cap, Dist2 &&dist2, Body &&body,
-                                               Masks &mk, unsigned &ci)
+                                               Masks &mk, Rows &&rows, unsigned &ci)
 {
     // bits t of a chunk starting at c with c + t < x
     auto below = [](unsigned c, unsigned x) {
@@ -459,21 +541,32 @@ __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R,
     const bool dropped = CAP && self - R.b1[1] >= cap;
     unsigned m0 = 0, m1 = 0, m2 = 0; // pending masks, m0 drained first
     unsigned x0 = 0, x1 = 0, x2 = 0; // source index of each mask's bit 0
-    unsigned t0 = 0, t1 = 0, t2 = 0; // owner threshold, source index space
     unsigned nq = 0;
     unsigned full = 0, half = 0;
+    // is the pair with source index idx in self's half list?
+    auto owns = [&](unsigned idx) {
+        const sph_rows Q = rows();
+        bool own = false;
+#pragma unroll
+        for (int dy = DY0; dy <= DY1; dy++) {
+            const unsigned off = (unsigned)src.row(dy);
+            const unsigned b0 = Q.b0[dy + 1], b3 = Q.b3[dy + 1];
+            const unsigned thr = dy == 1 ? Q.b1[dy + 1] : dy == 0 ? self + 1u : Q.b2[dy + 1];
+            own = idx - (b0 + off) < b3 - b0 ? idx >= thr + off : own;
+        }
+        return own;
+    };
     auto drain = [&]() {
         // the queue in locals: selects between captured variables can be
         // folded into a load from a selected address, which puts the queue
         // in scratch memory
-        unsigned q0 = m0, q1 = m1, q2 = m2, y0 = x0, y1 = x1, y2 = x2, u0 = t0, u1 = t1,
-                 u2 = t2;
+        unsigned q0 = m0, q1 = m1, q2 = m2, y0 = x0, y1 = x1, y2 = x2;
         while (q0) {
             if constexpr (LP == 1) {
                 const unsigned t = (unsigned)__builtin_ctz(q0);
                 q0 &= q0 - 1u;
                 const unsigned idx = y0 + t;
-                body(idx, OWN && idx >= u0, src.at(idx));
+                body(idx, src.at(idx), [&] { return owns(idx); });
             } else {
                 // lane q: the q-th lowest pending pair of the head chunk
                 const unsigned q = sph_quad_lane();
@@ -483,14 +576,27 @@ __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R,
                 r = q >= 3u ? r & (r - 1u) : r;
                 const bool have = r != 0u;
                 const unsigned idx = y0 + (have ? (unsigned)__builtin_ctz(r) : 0u);
-                sph_pair_term tm = body.term(idx, OWN && idx >= u0, src.at(idx));
+                bool nudged = false;
+                sph_pair_term tm =
+                    body.term(idx, src.at(idx), [&] { return owns(idx); }, nudged);
                 tm.a = have ? tm.a : 0.0f;
                 tm.b = have ? tm.b : 0.0f;
-                tm.f = have ? tm.f : 0;
-                body.apply(sph_quad_term<0>(tm));
-                body.apply(sph_quad_term<1>(tm));
-                body.apply(sph_quad_term<2>(tm));
-                body.apply(sph_quad_term<3>(tm));
+                if (__builtin_expect(__ballot(nudged) == 0ull, 1)) {
+                    body.apply(sph_quad_term<0>(tm));
+                    body.apply(sph_quad_term<1>(tm));
+                    body.apply(sph_quad_term<2>(tm));
+                    body.apply(sph_quad_term<3>(tm));
+                } else {
+                    const unsigned f = have && nudged ? 1u : 0u;
+                    body.nudge(sph_dpp<0x00>(f) != 0u);
+                    body.apply(sph_quad_term<0>(tm));
+                    body.nudge(sph_dpp<0x55>(f) != 0u);
+                    body.apply(sph_quad_term<1>(tm));
+                    body.nudge(sph_dpp<0xAA>(f) != 0u);
+                    body.apply(sph_quad_term<2>(tm));
+                    body.nudge(sph_dpp<0xFF>(f) != 0u);
+                    body.apply(sph_quad_term<3>(tm));
+                }
                 q0 &= q0 - 1u;
                 q0 &= q0 - 1u;
                 q0 &= q0 - 1u;
@@ -499,10 +605,8 @@ __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R,
             const bool next = q0 == 0; // chunk done: the queue moves up
             q0 = next ? q1 : q0;
             y0 = next ? y1 : y0;
-            u0 = next ? u1 : u0;
             q1 = next ? q2 : q1;
             y1 = next ? y2 : y1;
-            u1 = next ? u2 : u1;
             q2 = next ? 0u : q2;
         }
         m0 = m1 = m2 = 0u;
@@ -592,15 +696,12 @@ __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R,
                 if (nq == 0u) {
                     m0 = mask;
                     x0 = x;
-                    t0 = tt;
                 } else if (nq == 1u) {
                     m1 = mask;
                     x1 = x;
-                    t1 = tt;
                 } else {
                     m2 = mask;
                     x2 = x;
-                    t2 = tt;
                 }
                 nq++;
             }
@@ -611,12 +712,11 @@ __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R,
 }
 
 // All three candidate rows in one call.
-template <bool OWN = false, bool CAP = false, int LP = 1, class Src, class Dist2, class Body,
-          class Masks>
+template <bool CAP = false, int LP = 1, class Src, class Dist2, class Body, class Masks, class Rows>
 __device__ __forceinline__ uint2 sph_walk_masked(unsigned self, const sph_rows &R, const Src &src,
                                                  float h2, unsigned cap, Dist2 &&dist2,
-                                                 Body &&body, Masks &mk)
+                                                 Body &&body, Masks &mk, Rows &&rows)
 {
     unsigned ci = 0; // chunks of this lane so far (all rows, walk order)
-    return sph_walk_rows<OWN, CAP, -1, 1, LP>(self, R, src, h2, cap, dist2, body, mk, ci);
+    return sph_walk_rows<CAP, -1, 1, LP>(self, R, src, h2, cap, dist2, body, mk, rows, ci);
 }

@@ -48,15 +48,16 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kTPB = 256;
 // The gathers ask the compiler for at least 6 resident workgroups per CU
-// (6 waves per SIMD, at most 80 VGPRs): it then schedules them in 62-80
+// (6 waves per SIMD, at most 80 VGPRs): it then schedules them in 67-80
 // VGPRs without scratch, where left alone it took 72-84 (5-6 waves).  LDS
 // tiles allow 7 workgroups.  Measured on the 1M dam break at steps 221-230:
 // density -2%, relaxation -4%, the capped variants -3 to -7%, viscosity
-// unchanged.  The uncapped relaxation asks for 7, which keeps it at 72 VGPRs
-// (7 waves) with its row-by-row staging path; 6 let it grow to 74 (6 waves).
+// unchanged.  The capped relaxation asks for 5 (86-94 VGPRs): with 6 its
+// uncommon-pair path spills 60 bytes, and the capped 513k-particle dam break
+// takes 11.89 ms for 64 steps and their download against 11.59.
 // The four-lanes-per-particle variants (contexts of at most two tiles per
 // CU, so at most eight of their 64-particle workgroups per CU) set no bound:
-// their 66-88 VGPRs still allow 5-7 waves per SIMD, without scratch.
+// their 74-98 VGPRs still allow 4-6 waves per SIMD, without scratch.
 constexpr int kGatherMinBlocks = 6;
 #ifndef SPH_TILE_CAP
 #define SPH_TILE_CAP 1280
@@ -340,13 +341,14 @@ __device__ __forceinline__ void stage_row(const TilePlan &T, int dy, const Mem &
 }
 
 // Candidate source reading the LDS tile: the tile index of sorted position
-// k of row dy is k + row(dy).
+// k of row dy is k + row(dy).  The offsets stay in the plan, in LDS: each is
+// needed once per row, and registers decide how many waves run.
 template <class Mem>
 struct LdsSrc {
     Mem tile;
-    int offA[3], offB[3];
-    bool rowB;
-    __device__ int row(int dy) const { return rowB ? offB[dy + 1] : offA[dy + 1]; }
+    const TilePlan *T;
+    int seg; // 0, or 3 for a lane in the group's second cell row
+    __device__ int row(int dy) const { return T->off[seg + dy + 1]; }
     __device__ typename Mem::Rec at(unsigned idx) const { return tile.get(idx); }
 };
 
@@ -354,30 +356,29 @@ template <class Mem>
 __device__ __forceinline__ LdsSrc<Mem> lds_src(const Mem &tile, const TilePlan &T, unsigned key,
                                               const sph_dev_params &P)
 {
-    LdsSrc<Mem> r;
-    r.tile = tile;
-    for (int q = 0; q < 3; q++) {
-        r.offA[q] = T.off[q];
-        r.offB[q] = T.off[3 + q];
-    }
-    r.rowB = (key - P.cell_base) / P.sx != T.jA;
-    return r;
+    return LdsSrc<Mem>{tile, &T, (key - P.cell_base) / P.sx != T.jA ? 3 : 0};
 }
 
-// The source of a tile staged by stage_row(dy): only row dy's offsets matter.
+// The source of a tile staged by stage_row(dy): its first cell row's segment
+// begins at index 0, its second one's follows.
 template <class Mem>
-__device__ __forceinline__ LdsSrc<Mem> lds_row_src(const Mem &tile, const TilePlan &T, int dy,
-                                                  unsigned key, const sph_dev_params &P)
-{
-    LdsSrc<Mem> r;
-    r.tile = tile;
-    const int qa = dy + 1, qb = dy + 4;
-    for (int q = 0; q < 3; q++) {
-        r.offA[q] = -(int)T.g0[qa];
-        r.offB[q] = (int)T.len[qa] - (int)T.g0[qb];
+struct LdsRowSrc {
+    Mem tile;
+    const TilePlan *T;
+    bool rowB;
+    __device__ int row(int dy) const
+    {
+        const int qa = dy + 1, qb = dy + 4;
+        return rowB ? (int)T->len[qa] - (int)T->g0[qb] : -(int)T->g0[qa];
     }
-    r.rowB = (key - P.cell_base) / P.sx != T.jA;
-    return r;
+    __device__ typename Mem::Rec at(unsigned idx) const { return tile.get(idx); }
+};
+
+template <class Mem>
+__device__ __forceinline__ LdsRowSrc<Mem> lds_row_src(const Mem &tile, const TilePlan &T,
+                                                      unsigned key, const sph_dev_params &P)
+{
+    return LdsRowSrc<Mem>{tile, &T, (key - P.cell_base) / P.sx != T.jA};
 }
 
 // Candidate source reading global memory.
@@ -398,20 +399,22 @@ __device__ __forceinline__ GlobalSrc<Rec, Load> global_src(Load l)
 // plan staged one, else from global memory (same order, same results).  Every
 // thread of the workgroup calls this (the staging and its barrier need all of
 // them); `live` lanes walk.
-template <bool OWN, bool CAP, int CAPACITY, int LP = 1, class Rec, class Load, class Test,
-          class Body, class Masks>
+template <bool CAP, int CAPACITY, int LP = 1, class Rec, class Load, class Test, class Body,
+          class Masks>
 __device__ __forceinline__ uint2 walk_group(const TilePlan &T, Rec *tile, Load load, bool live,
                                             unsigned self, const sph_rows &R, unsigned key,
-                                            const sph_dev_params &P, Test &test, Body &body,
-                                            Masks &mk)
+                                            const sph_dev_params &P,
+                                            const unsigned *__restrict__ start, Test &test,
+                                            Body &body, Masks &mk)
 {
     uint2 fh = make_uint2(0u, 0u);
     const auto mem = tile_mem<CAPACITY>(tile);
+    auto rows = [&] { return sph_row_bounds(key, P, start); };
     if (T.ok) {
         stage_tile<CAPACITY>(T, mem, load);
         if (live)
-            fh = sph_walk_masked<OWN, CAP, LP>(self, R, lds_src(mem, T, key, P), P.h2,
-                                               P.bucket_cap, test, body, mk);
+            fh = sph_walk_masked<CAP, LP>(self, R, lds_src(mem, T, key, P), P.h2, P.bucket_cap,
+                                          test, body, mk, rows);
     } else if (T.rows_ok) {
         // one candidate row at a time: same chunks, same order
         unsigned ci = 0;
@@ -419,9 +422,10 @@ __device__ __forceinline__ uint2 walk_group(const TilePlan &T, Rec *tile, Load l
             constexpr int dy = decltype(row)::value;
             stage_row<CAPACITY>(T, dy, mem, load);
             if (live) {
-                const uint2 r = sph_walk_rows<OWN, CAP, dy, dy, LP>(
-                    self, R, lds_row_src(mem, T, dy, key, P), P.h2, P.bucket_cap, test, body,
-                    mk, ci);
+                const uint2 r = sph_walk_rows<CAP, dy, dy, LP>(self, R,
+                                                               lds_row_src(mem, T, key, P), P.h2,
+                                                               P.bucket_cap, test, body, mk, rows,
+                                                               ci);
                 fh.x += r.x;
                 fh.y += r.y;
             }
@@ -431,8 +435,8 @@ __device__ __forceinline__ uint2 walk_group(const TilePlan &T, Rec *tile, Load l
         pass(std::integral_constant<int, 0>{});
         pass(std::integral_constant<int, 1>{});
     } else if (live) {
-        fh = sph_walk_masked<OWN, CAP, LP>(self, R, global_src<Rec>(load), P.h2, P.bucket_cap,
-                                           test, body, mk);
+        fh = sph_walk_masked<CAP, LP>(self, R, global_src<Rec>(load), P.h2, P.bucket_cap, test,
+                                      body, mk, rows);
     }
     return fh;
 }
@@ -520,33 +524,35 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
             const float dx = b.x - a.x, ddy = b.y - a.y;
             return dx * dx + ddy * ddy;
         };
-        auto body = [&](unsigned, bool, float4 b) {
-            float ix, iy;
-            const bool push = sph_visc_impulse(a.x, a.y, avx, avy, b.x, b.y, b.z, b.w, P, ix, iy);
-            nvx = push ? nvx - ix * 0.5f : nvx;
-            nvy = push ? nvy - iy * 0.5f : nvy;
+        const sph_visc_consts V{sph_vgpr(P.h_recip), sph_vgpr(P.dt), sph_vgpr(P.sigma),
+                                sph_vgpr(P.beta)};
+        auto half_impulse = [&](float4 b) {
+            return sph_visc_half(a.x, a.y, avx, avy, b.x, b.y, b.z, b.w, V, P);
         };
         plan_tile_par(kf0, s1 - s0 == kPer ? kl0 : K[s1 - 1], start, P, T, kTileCap);
         sph_masks_none mk;
         uint2 fh;
         if constexpr (LP == 1) {
-            fh = walk_group<false, CAP, kTileCap>(T, tile, load, live, s, R, key, P, test, body,
-                                                  mk);
+            auto body = [&](unsigned, float4 b, auto &&) {
+                const float2 t = half_impulse(b);
+                nvx = nvx - t.x;
+                nvy = nvy - t.y;
+            };
+            fh = walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, P, start, test, body,
+                                           mk);
         } else {
-            // the same impulse as a term (zero when not pushed: nv - 0 == nv)
-            auto term = [&](unsigned, bool, float4 b) {
-                float ix, iy;
-                const bool push =
-                    sph_visc_impulse(a.x, a.y, avx, avy, b.x, b.y, b.z, b.w, P, ix, iy);
-                return sph_pair_term{push ? ix : 0.0f, push ? iy : 0.0f, 0};
+            auto term = [&](unsigned, float4 b, auto &&, bool &) {
+                const float2 t = half_impulse(b);
+                return sph_pair_term{t.x, t.y};
             };
             auto apply = [&](const sph_pair_term &t) {
-                nvx = nvx - t.a * 0.5f;
-                nvy = nvy - t.b * 0.5f;
+                nvx = nvx - t.a;
+                nvy = nvy - t.b;
             };
-            sph_split_body<decltype(term), decltype(apply)> sb{term, apply};
-            fh = walk_group<false, CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, test, sb,
-                                                      mk);
+            auto never = [](bool) {};
+            sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply, never};
+            fh = walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb,
+                                               mk);
         }
         full = fh.x;
         half = lead ? fh.y : 0u; // a particle's half list counted once
@@ -938,37 +944,46 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         const float dx = a.x - b.x, ddy = a.y - b.y;
         return dx * dx + ddy * ddy;
     };
-    auto body = [&](unsigned, bool, float2 b) {
+    const float h_recip = sph_vgpr(P.h_recip);
+    // the pair's (1 - r/h)^2 and ^3, or zero outside h (rho + 0 == rho, as
+    // rho >= +0)
+    auto pair = [&](float2 b) {
         const float dx = a.x - b.x, ddy = a.y - b.y;
         const float r2 = dx * dx + ddy * ddy;
-        const float ratio = sph_sqrt(r2) * P.h_recip;
-        const float OmR2 = (1.0f - ratio) * (1.0f - ratio);
-        const bool in = ratio < 1.0f;
-        rho = in ? rho + OmR2 : rho;
-        rhon = in ? rhon + OmR2 * (1.0f - ratio) : rhon;
+        const float OmR = 1.0f - sph_sqrt_common(r2) * h_recip;
+        const float OmR2 = OmR * OmR;
+        float2 t = make_float2(OmR2, OmR2 * OmR);
+        if (__builtin_expect(__ballot(sph_uncommon_pair(r2, kPairLoRoot, P)) != 0ull, 0)) {
+            const float ratio = sph_sqrt(r2) * h_recip;
+            const float w = (1.0f - ratio) * (1.0f - ratio);
+            const bool in = ratio < 1.0f;
+            t = make_float2(in ? w : 0.0f, in ? w * (1.0f - ratio) : 0.0f);
+        }
+        return t;
     };
     sph_masks_record mk;
     uint2 fh;
     if constexpr (LP == 1) {
-        fh = walk_group<false, CAP, 2 * kTileCap>(T, tile, load, live, s, R, key, P, test, body,
-                                                  mk);
+        auto body = [&](unsigned, float2 b, auto &&) {
+            const float2 t = pair(b);
+            rho = rho + t.x;
+            rhon = rhon + t.y;
+        };
+        fh = walk_group<CAP, 2 * kTileCap>(T, tile, load, live, s, R, key, P, start, test, body,
+                                           mk);
     } else {
-        // the same sums as terms (zero outside h: rho + 0 == rho, as rho >= +0)
-        auto term = [&](unsigned, bool, float2 b) {
-            const float dx = a.x - b.x, ddy = a.y - b.y;
-            const float r2 = dx * dx + ddy * ddy;
-            const float ratio = sph_sqrt(r2) * P.h_recip;
-            const float OmR2 = (1.0f - ratio) * (1.0f - ratio);
-            const bool in = ratio < 1.0f;
-            return sph_pair_term{in ? OmR2 : 0.0f, in ? OmR2 * (1.0f - ratio) : 0.0f, 0};
+        auto term = [&](unsigned, float2 b, auto &&, bool &) {
+            const float2 t = pair(b);
+            return sph_pair_term{t.x, t.y};
         };
         auto apply = [&](const sph_pair_term &t) {
             rho = rho + t.a;
             rhon = rhon + t.b;
         };
-        sph_split_body<decltype(term), decltype(apply)> sb{term, apply};
-        fh = walk_group<false, CAP, 2 * kTileCap, LP>(T, tile, load, live, s, R, key, P, test, sb,
-                                                      mk);
+        auto never = [](bool) {};
+        sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply, never};
+        fh = walk_group<CAP, 2 * kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb,
+                                               mk);
     }
     if (live && lead) {
         RHO[s] = make_float2(rho, rhon);
@@ -1067,63 +1082,58 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         const float dx = a.x - b.x, ddy = a.y - b.y;
         return dx * dx + ddy * ddy;
     };
-    auto body = [&](unsigned, bool own, float4 b) {
+    const float h_recip = sph_vgpr(P.h_recip), h = sph_vgpr(P.h), k_spring = sph_vgpr(P.k_spring);
+    const double dt2 = (double)(P.dt * P.dt);
+    // the pair's displacement (zero when not pushed: n - 0 == n); on_nudge
+    // hears whether an uncommon pair takes the 1e-6 nudge, before it
+    auto pair = [&](float4 b, auto &&own, auto &&on_nudge) {
         const float dx = a.x - b.x, ddy = a.y - b.y;
         const float r2 = dx * dx + ddy * ddy;
-        const float rr = sph_sqrt(r2);
-        const float r_recip = sph_rcp(rr); // 1.0f / rr
-        const float ratio = rr * P.h_recip;
-        const float OmR = 1.0f - ratio;
-        // both updates as selects (no branch in the pair loop)
-        const bool nudge = rr <= 0.000001f && own;
-        nx = nudge ? nx + 0.000001f : nx;
-        ny = nudge ? ny + 0.000001f : ny;
-        const float D = sph_relax_D(P.dt, aP + b.z, aPn + b.w, OmR, P.k_spring, P.h, rr);
         // b - a = -(a - b) exactly in IEEE arithmetic
-        const float Dx = D * -dx * r_recip;
-        const float Dy = D * -ddy * r_recip;
-        const bool push = ratio < 1.0f && rr > 0.0f;
-        nx = push ? nx - Dx : nx;
-        ny = push ? ny - Dy : ny;
-    };
-    if constexpr (LP == 1) {
-        if (FUSED) { // the density pass of this step walked the same neighbour set
-            sph_masks_replay mk{live ? masks[s] : make_uint4(0u, 0u, 0u, 0u)};
-            walk_group<true, CAP, kTileCap>(T, tile, load, live, s, R, key, P, test, body, mk);
-        } else {
-            sph_masks_none mk;
-            walk_group<true, CAP, kTileCap>(T, tile, load, live, s, R, key, P, test, body, mk);
-        }
-    } else {
-        // the same updates as terms: the displacement (zero when not pushed:
-        // n - 0 == n) and the nudge flag, applied nudge first as in body
-        auto term = [&](unsigned, bool own, float4 b) {
-            const float dx = a.x - b.x, ddy = a.y - b.y;
-            const float r2 = dx * dx + ddy * ddy;
+        const sph_root q = sph_root_common(r2);
+        const float D = sph_relax_D(dt2, aP + b.z, aPn + b.w, 1.0f - q.r * h_recip, k_spring, h,
+                                    q.r);
+        sph_pair_term t{D * -dx * q.rinv, D * -ddy * q.rinv};
+        if (__builtin_expect(__ballot(sph_uncommon_pair(r2, kPairLoNudge, P)) != 0ull, 0)) {
             const float rr = sph_sqrt(r2);
             const float r_recip = sph_rcp(rr); // 1.0f / rr
-            const float ratio = rr * P.h_recip;
-            const float OmR = 1.0f - ratio;
-            const bool nudge = rr <= 0.000001f && own;
-            const float D = sph_relax_D(P.dt, aP + b.z, aPn + b.w, OmR, P.k_spring, P.h, rr);
-            const float Dx = D * -dx * r_recip;
-            const float Dy = D * -ddy * r_recip;
+            const float ratio = rr * h_recip;
             const bool push = ratio < 1.0f && rr > 0.0f;
-            return sph_pair_term{push ? Dx : 0.0f, push ? Dy : 0.0f, nudge ? 1 : 0};
-        };
-        auto apply = [&](const sph_pair_term &t) {
-            nx = t.f ? nx + 0.000001f : nx;
-            ny = t.f ? ny + 0.000001f : ny;
-            nx = nx - t.a;
-            ny = ny - t.b;
-        };
-        sph_split_body<decltype(term), decltype(apply)> sb{term, apply};
-        if (FUSED) {
+            const float E = sph_relax_D(dt2, aP + b.z, aPn + b.w, 1.0f - ratio, k_spring, h, rr);
+            t.a = push ? E * -dx * r_recip : 0.0f;
+            t.b = push ? E * -ddy * r_recip : 0.0f;
+            on_nudge(rr <= 0.000001f && own());
+        }
+        return t;
+    };
+    auto nudge = [&](bool yes) {
+        nx = yes ? nx + 0.000001f : nx;
+        ny = yes ? ny + 0.000001f : ny;
+    };
+    auto apply = [&](const sph_pair_term &t) {
+        nx = nx - t.a;
+        ny = ny - t.b;
+    };
+    if constexpr (LP == 1) {
+        auto body = [&](unsigned, float4 b, auto &&own) { apply(pair(b, own, nudge)); };
+        if (FUSED) { // the density pass of this step walked the same neighbour set
             sph_masks_replay mk{live ? masks[s] : make_uint4(0u, 0u, 0u, 0u)};
-            walk_group<true, CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, test, sb, mk);
+            walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, P, start, test, body, mk);
         } else {
             sph_masks_none mk;
-            walk_group<true, CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, test, sb, mk);
+            walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, P, start, test, body, mk);
+        }
+    } else {
+        auto term = [&](unsigned, float4 b, auto &&own, bool &nudged) {
+            return pair(b, own, [&](bool yes) { nudged = yes; });
+        };
+        sph_split_body<decltype(term), decltype(apply), decltype(nudge)> sb{term, apply, nudge};
+        if (FUSED) {
+            sph_masks_replay mk{live ? masks[s] : make_uint4(0u, 0u, 0u, 0u)};
+            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb, mk);
+        } else {
+            sph_masks_none mk;
+            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb, mk);
         }
     }
     if (!live || !lead)
@@ -1145,7 +1155,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 }
 
 template <bool FUSED, bool CAP>
-__global__ void __launch_bounds__(kTPB, CAP ? kGatherMinBlocks : kGatherMinBlocks + 1)
+__global__ void __launch_bounds__(kTPB, CAP ? kGatherMinBlocks - 1 : kGatherMinBlocks)
 k_relax(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
         const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
@@ -1284,9 +1294,9 @@ void launch(F kernel, dim3 grid, dim3 block, hipStream_t st, Args... args)
 } // namespace
 
 // Exhaustive checks of sph_sqrt (FN 0) against sqrtf and sph_rcp (FN 1)
-// against IEEE division: every float with bit pattern in [lo, hi)
-// (grid-stride; for sph_rcp, every one in its domain), bit for bit (any NaN
-// equals any NaN).
+// against IEEE division, and of sph_root_common's root (FN 0) and reciprocal
+// root (FN 1): every float with bit pattern in [lo, hi) (grid-stride; the
+// last three over their domains), bit for bit (any NaN equals any NaN).
 __device__ __attribute__((noinline)) float ieee_sqrt(float x) { return sqrtf(x); }
 __device__ __attribute__((noinline)) float ieee_rcp(float x) { return 1.0f / x; }
 
@@ -1299,13 +1309,20 @@ k_selftest_math(unsigned lo, unsigned hi, unsigned long long *__restrict__ bad)
     for (unsigned long long b = lo + (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
          b < hi; b += stride) {
         const float x = __uint_as_float((unsigned)b);
-        if (FN == 1 && !sph_rcp_domain(x))
-            continue;
-        const float got = FN == 0 ? sph_sqrt(x) : sph_rcp(x);
-        const float want = FN == 0 ? ieee_sqrt(x) : ieee_rcp(x);
-        const bool same = __float_as_uint(got) == __float_as_uint(want) ||
-                          (got != got && want != want);
-        nbad += same ? 0u : 1u;
+        auto differ = [](float got, float want) {
+            return __float_as_uint(got) != __float_as_uint(want) && !(got != got && want != want);
+        };
+        bool bad_x = false;
+        if (FN == 0)
+            bad_x = differ(sph_sqrt(x), ieee_sqrt(x));
+        else if (sph_rcp_domain(x))
+            bad_x = differ(sph_rcp(x), ieee_rcp(x));
+        if (x >= 0x1p-96f && x <= 0x1p120f) {
+            const sph_root q = sph_root_common(x);
+            const float r = ieee_sqrt(x);
+            bad_x = bad_x || differ(FN == 0 ? q.r : q.rinv, FN == 0 ? r : ieee_rcp(r));
+        }
+        nbad += bad_x ? 1u : 0u;
     }
     for (int o = 32; o > 0; o >>= 1)
         nbad += __shfl_xor(nbad, o, 64);
