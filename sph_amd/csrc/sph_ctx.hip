@@ -187,7 +187,7 @@ void enqueue_fused_step(sph_ctx *c, bool visc)
     const bool cap = c->bucket_cap != 0;
     {
         Tick t(c, KV);
-        sph_launch_visc_predict(c->st, S, true, visc, true, cap, c->dPA, c->BS, c->POS0, c->VEL,
+        sph_launch_visc_predict(c->st, S, true, visc, true, cap, c->dPA, c->BS, c->plans, c->POS0, c->VEL,
                                 c->K0, c->start, c->UPOS, c->ukey, c->uslot, c->cnt, c->dC,
                                 c->dclock, c->UVEL, c->lanes);
     }
@@ -196,16 +196,16 @@ void enqueue_fused_step(sph_ctx *c, bool visc)
         Tick t(c, KRO);
         sph_reorder_fields<2> f{{c->UPOS, c->POS0}, {c->POS1, c->PREV}};
         sph_launch_reorder2(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K1,
-                            f, c->ID1, c->dC);
+                            f, c->ID1, c->plans, c->dC);
     }
     {
         Tick t(c, KDE);
-        sph_launch_density(c->st, S, cap, c->dP, c->BS, c->POS1, c->K1, c->start, c->RHO,
+        sph_launch_density(c->st, S, cap, c->dP, c->BS, c->plans, c->POS1, c->K1, c->start, c->RHO,
                            c->MASK, c->dC, c->lanes);
     }
     {
         Tick t(c, KRE);
-        sph_launch_relax(c->st, S, true, cap, c->dP, c->BS, c->POS1, c->PREV, c->RHO, c->K1,
+        sph_launch_relax(c->st, S, true, cap, c->dP, c->BS, c->plans, c->POS1, c->PREV, c->RHO, c->K1,
                          c->start, c->UPOS, c->UVEL, c->ukey, c->uslot, c->cnt, c->MASK, c->dC,
                          c->dclock, c->lanes);
     }
@@ -214,7 +214,7 @@ void enqueue_fused_step(sph_ctx *c, bool visc)
         Tick t(c, KRO);
         sph_reorder_fields<2> f{{c->UPOS, c->UVEL}, {c->POS0, c->VEL}};
         sph_launch_reorder2(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K0,
-                            f, c->ID0, c->dC);
+                            f, c->ID0, c->plans, c->dC);
     }
 }
 
@@ -276,6 +276,14 @@ int dalloc(T **p, size_t count)
         return set_err(SPH_ENOMEM, "hipMalloc(%zu x %zu B) failed: %s", count, sizeof(T),
                        hipGetErrorString(e));
     return SPH_OK;
+}
+
+// The four-lane gathers' plans exist in the contexts that use them.
+int ensure_plans(sph_ctx *c)
+{
+    if (c->lanes != 4 || c->plans.t64)
+        return SPH_OK;
+    return dalloc(&c->plans.t64, (size_t)c->slots / 64);
 }
 
 int check_scene_desc(const sph_scene_desc &d, int idx)
@@ -364,10 +372,14 @@ int sph_create_batch(sph_ctx **out, const sph_scene_desc *scenes, int nscenes)
     A(POS1, N + kSphWalkPad); A(UPOS, N); A(UVEL, N); A(T2a, N); A(T2b, N);
     A(ID0, N); A(ID1, N); A(perm_src, N); A(perm_id, N); A(pos_of_id, N);
     A(K0, N); A(K1, N); A(ukey, N); A(uslot, N);
-    A(cnt, MP); A(start, MP); A(bsum, sph_scan_blocks((unsigned)M));
+    A(cnt, MP); A(start_mem, MP + 8); A(plans.t256, N / kSphTPB); A(bsum, sph_scan_blocks((unsigned)M));
     A(coords, 2 * N); A(MASK, N); A(dP, (size_t)nscenes); A(dPA, (size_t)nscenes); A(ACC, N);
     A(BS, N / kSphTPB); A(dC, 1); A(dclock, 1);
 #undef A
+    if (!rc) {
+        c->start = c->start_mem + 4; // a spare entry before, 16-byte aligned for the scans
+        rc = ensure_plans(c);
+    }
     if (!rc) {
         hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
         if (e != hipSuccess)
@@ -382,7 +394,7 @@ int sph_create_batch(sph_ctx **out, const sph_scene_desc *scenes, int nscenes)
         if (e == hipSuccess)
             e = hipMemset(c->cnt, 0, sizeof(unsigned) * MP);
         if (e == hipSuccess)
-            e = hipMemset(c->start, 0, sizeof(unsigned) * MP);
+            e = hipMemset(c->start_mem, 0, sizeof(unsigned) * (MP + 8));
         if (e == hipSuccess)
             e = hipMemset(c->dC, 0, sizeof(sph_dev_counters));
         if (e == hipSuccess)
@@ -423,10 +435,10 @@ void sph_destroy(sph_ctx *c)
     void *ptrs[] = {c->POS0, c->VEL,  c->PREV,     c->RHO,     c->POS1,      c->UPOS,
                     c->UVEL, c->T2a,  c->T2b,      c->ID0,     c->ID1,       c->perm_src,
                     c->perm_id, c->pos_of_id, c->K0, c->K1,    c->ukey,      c->uslot,
-                    c->cnt,  c->start, c->bsum,    c->coords,  c->dP,        c->BS,
+                    c->cnt,  c->start_mem, c->bsum,    c->coords,  c->dP,        c->BS,
                     c->dC,   c->dclock, c->SPOS,    c->SVEL,    c->SPREV,     c->SRHO,
                     c->SID,  c->SK,    c->Sstart,  c->Sclock,  c->dflags, c->MASK,
-                    c->dPA,  c->XY,    c->ACC,     c->AOS};
+                    c->dPA,  c->XY,    c->ACC,     c->AOS,     c->plans.t256, c->plans.t64};
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);
@@ -659,6 +671,12 @@ int sph_set_gather_lanes(sph_ctx *c, int lanes)
     if (want != c->lanes)
         free_graphs(c); // the captured steps launch the other kernel variants
     c->lanes = want;
+    if (int rc = ensure_plans(c))
+        return rc;
+    if (c->lists_valid && c->n_total) { // the current hash's plans for these lanes
+        sph_launch_plan(c->st, c->slots, c->dP, c->BS, c->start, c->K0, c->plans);
+        HIPCHK(hipGetLastError());
+    }
     return SPH_OK;
 }
 
@@ -803,7 +821,7 @@ int sph_phase_viscosity(sph_ctx *c)
     if (!c->lists_valid || c->n_total == 0)
         return SPH_OK; // empty lists (src/fluid.c:202)
     sph_launch_visc_predict(c->st, c->slots, false, true, false, c->bucket_cap != 0, c->dP, c->BS,
-                            c->POS0, c->VEL, c->K0, c->start, c->UVEL, nullptr, nullptr, c->cnt,
+                            c->plans, c->POS0, c->VEL, c->K0, c->start, c->UVEL, nullptr, nullptr, c->cnt,
                             c->dC, c->dclock, nullptr, c->lanes);
     HIPCHK(hipMemcpyAsync(c->VEL, c->UVEL, sizeof(float2) * (size_t)c->slots,
                           hipMemcpyDeviceToDevice, c->st));
@@ -837,7 +855,7 @@ int sph_phase_hash(sph_ctx *c, int compute_density)
     sph_reorder_fields<4> f{{c->POS0, c->VEL, c->PREV, c->RHO},
                             {c->POS1, c->UVEL, c->T2a, c->T2b}};
     sph_launch_reorder4(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K1, f,
-                        c->ID1, c->dC);
+                        c->ID1, c->plans, c->dC);
     const size_t b = sizeof(float2) * (size_t)S;
     for (int k = 0; k < 4; k++)
         HIPCHK(hipMemcpyAsync((void *)f.src[k], f.dst[k], b, hipMemcpyDeviceToDevice, c->st));
@@ -845,7 +863,7 @@ int sph_phase_hash(sph_ctx *c, int compute_density)
     HIPCHK(hipMemcpyAsync(c->K0, c->K1, sizeof(unsigned) * (size_t)S, hipMemcpyDeviceToDevice,
                           c->st));
     if (compute_density)
-        sph_launch_density(c->st, S, c->bucket_cap != 0, c->dP, c->BS, c->POS0, c->K0, c->start,
+        sph_launch_density(c->st, S, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->K0, c->start,
                            c->RHO, c->MASK, c->dC, c->lanes);
     HIPCHK(hipGetLastError());
     c->lists_valid = true;
@@ -863,7 +881,7 @@ int sph_phase_relax(sph_ctx *c)
         return SPH_OK;
     if (!c->lists_valid)
         return set_err(SPH_ESTATE, "sph_phase_relax: no hash since upload");
-    sph_launch_relax(c->st, c->slots, false, c->bucket_cap != 0, c->dP, c->BS, c->POS0, c->PREV,
+    sph_launch_relax(c->st, c->slots, false, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->PREV,
                      c->RHO, c->K0, c->start, c->UPOS, nullptr, nullptr, nullptr, nullptr,
                      nullptr, c->dC, c->dclock, c->lanes);
     HIPCHK(hipMemcpyAsync(c->POS0, c->UPOS, sizeof(float2) * (size_t)c->slots,
@@ -943,6 +961,7 @@ int sph_snapshot_restore(sph_ctx *c, const int *scene_flags)
                        {c->POS0, c->VEL, c->PREV, c->RHO},
                        c->SID, c->ID0, c->SK, c->Sstart, c->K0, c->start};
     sph_launch_restore(c->st, c->slots, c->dP, c->BS, c->dflags, a);
+    sph_launch_plan(c->st, c->slots, c->dP, c->BS, c->start, c->K0, c->plans);
     HIPCHK(hipMemcpyAsync(c->dclock, c->Sclock, sizeof(unsigned long long),
                           hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());

@@ -54,6 +54,8 @@ struct sph_ctx {
         *pos_of_id = nullptr;
     unsigned *K0 = nullptr, *K1 = nullptr, *ukey = nullptr, *uslot = nullptr, *cnt = nullptr,
              *start = nullptr, *bsum = nullptr;
+    unsigned *start_mem = nullptr; // start's allocation (start has a spare entry before it)
+    sph_tile_plans plans;          // of the hash that K0 or K1 and start describe
     short *coords = nullptr;
     uint4 *MASK = nullptr; // per slot: the density pass's first accepted-candidate masks
     float2 *ACC = nullptr;  // (a_x, a_y) by caller index: carried, never changed (src/fluid.c)

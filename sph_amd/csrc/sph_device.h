@@ -384,35 +384,58 @@ __device__ __forceinline__ void sph_walk(unsigned s, unsigned key, const sph_dev
     }
 }
 
+// The plan of a tile of consecutive sorted particles (sph_make_plan), made
+// once per sort by the reorder kernel, for every gather that follows.  The
+// candidate rows of the tile's (at most two) cell rows are six segments of
+// the sorted arrays: segment 3 rho + dy + 1 holds, for the particles in cell
+// row jA + rho, the cells c0 - 1 .. c1 + 1 of row jA + rho + dy (empty outside
+// the grid).  A gather reads its plan with one scalar load.  (Made by the
+// gathers themselves it was two dependent loads, two barriers and a serial
+// stretch on one thread in every workgroup, before the first record could be
+// staged.  viscosity / relaxation / density of the 1M dam break, steps 21-220:
+// 42.2 / 36.6 / 31.9 -> 40.6 / 33.8 / 30.8 us, the reorder 10.6 -> 11.1 us; of
+// 16k particles, late: 19.7 / 20.5 / 15.6 -> 18.9 / 19.3 / 15.3 us.)
+struct alignas(64) sph_tile_plan {
+    unsigned g0[6], len[6]; // begin and length of the segments
+    unsigned jA;            // cell row of the first particle
+    unsigned split;         // sorted position where row jA + 1 begins
+    int scene;
+    unsigned wide;          // 1: more than two cell rows, no segments
+};
+
 // The candidate rows of a particle in global cell `key`: row dy = -1, 0, 1
 // holds its cells i-1 / i / i+1 (clipped to the grid) at sorted positions
 // [b0,b1) / [b1,b2) / [b2,b3); a row outside the grid is empty.  Kernels
 // load them as soon as the key is known, so that the walk itself reads no
-// global memory but its candidates.
+// global memory but its candidates.  The four starts of a row are consecutive:
+// one 16-byte load a row (start has a spare entry before the first and after
+// the last).  j: the particle's cell row.
 struct sph_rows {
     unsigned b0[3], b1[3], b2[3], b3[3];
 };
 
-__device__ __forceinline__ sph_rows sph_row_bounds(unsigned key, const sph_dev_params &P,
+struct sph_starts4 {
+    unsigned v[4];
+};
+
+__device__ __forceinline__ sph_rows sph_row_bounds(unsigned key, unsigned j,
+                                                   const sph_dev_params &P,
                                                    const unsigned *__restrict__ start)
 {
     sph_rows R;
     const unsigned sx = P.sx, sy = P.sy;
-    const unsigned local = key - P.cell_base;
-    const unsigned i = local % sx, j = local / sx;
-    const unsigned i0 = i > 0 ? i - 1 : 0;
-    const unsigned i1 = i + 1 < sx ? i + 1 : sx - 1;
+    const unsigned i = key - P.cell_base - j * sx;
+    const bool left = i > 0, right = i + 1 < sx;
 #pragma unroll
     for (int dy = -1; dy <= 1; dy++) {
-        const long r = (long)j + dy;
-        const bool in = r >= 0 && r < (long)sy;
-        const unsigned base = P.cell_base + (in ? (unsigned)r : j) * sx;
-        const unsigned b0 = start[base + i0], b1 = start[base + i];
-        const unsigned b2 = start[base + i + 1], b3 = start[base + i1 + 1];
-        R.b0[dy + 1] = in ? b0 : 0;
-        R.b1[dy + 1] = in ? b1 : 0;
-        R.b2[dy + 1] = in ? b2 : 0;
-        R.b3[dy + 1] = in ? b3 : 0;
+        const bool in = dy < 0 ? j > 0 : dy > 0 ? j + 1 < sy : true;
+        const size_t c = (size_t)(in ? key + (unsigned)dy * sx : key);
+        sph_starts4 q;
+        __builtin_memcpy(&q, start + c - 1, sizeof q);
+        R.b0[dy + 1] = in ? (left ? q.v[0] : q.v[1]) : 0;
+        R.b1[dy + 1] = in ? q.v[1] : 0;
+        R.b2[dy + 1] = in ? q.v[2] : 0;
+        R.b3[dy + 1] = in ? (right ? q.v[3] : q.v[2]) : 0;
     }
     return R;
 }

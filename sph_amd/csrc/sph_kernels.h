@@ -11,6 +11,12 @@ struct sph_reorder_fields {
     float2 *dst[NF];
 };
 
+// The tile plans of the current sort: of 256 sorted particles each, and of 64
+// (the four-lane gathers' tiles; null unless the context uses those).
+struct sph_tile_plans {
+    sph_tile_plan *t256 = nullptr, *t64 = nullptr;
+};
+
 // Workgroup size of every particle kernel; scenes are padded to multiples.
 constexpr unsigned kSphTPB = 256;
 
@@ -22,8 +28,8 @@ int sph_gather_lanes(unsigned slots);
 // lanes: lanes per particle of the gathers, 1 or 4 (sph_gather_lanes); 4
 // applies to the fused step's variants (grav, visc and pred; fused relax).
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
-                             bool cap, const sph_dev_params *P, const int *BS, const float2 *POS,
-                             const float2 *VEL, const unsigned *K, const unsigned *start,
+                             bool cap, const sph_dev_params *P, const int *BS,
+                             const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,
                              float2 *opos, unsigned *okey, unsigned *oslot, unsigned *cnt,
                              sph_dev_counters *C, const unsigned long long *clock,
                              float2 *held_vel, int lanes);
@@ -53,18 +59,21 @@ void sph_launch_scatter(hipStream_t st, unsigned slots, const sph_dev_params *P,
 void sph_launch_reorder2(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                          const unsigned *start, const int *perm_src, const int *perm_id,
                          const unsigned *skey, sph_reorder_fields<2> f, int *id_dst,
-                         sph_dev_counters *C);
+                         const sph_tile_plans &plans, sph_dev_counters *C);
 void sph_launch_reorder4(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                          const unsigned *start, const int *perm_src, const int *perm_id,
                          const unsigned *skey, sph_reorder_fields<4> f, int *id_dst,
-                         sph_dev_counters *C);
+                         const sph_tile_plans &plans, sph_dev_counters *C);
+// The tile plans alone, of sorted keys that no reorder has just placed.
+void sph_launch_plan(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
+                     const unsigned *start, const unsigned *skey, const sph_tile_plans &plans);
 void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_params *P,
-                        const int *BS, const float2 *POS, const unsigned *K,
+                        const int *BS, const sph_tile_plans &plans, const float2 *POS, const unsigned *K,
                         const unsigned *start, float2 *RHO, uint4 *masks, sph_dev_counters *C,
                         int lanes);
 void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
-                      const sph_dev_params *P, const int *BS, const float2 *POS,
-                      const float2 *PREV, const float2 *RHO, const unsigned *K,
+                      const sph_dev_params *P, const int *BS, const sph_tile_plans &plans,
+                      const float2 *POS, const float2 *PREV, const float2 *RHO, const unsigned *K,
                       const unsigned *start, float2 *opos, float2 *ovel, unsigned *okey,
                       unsigned *oslot, unsigned *cnt, const uint4 *masks, sph_dev_counters *C,
                       unsigned long long *clock, int lanes);

@@ -89,9 +89,10 @@ __device__ __forceinline__ bool lane0() { return (threadIdx.x & (kWave - 1)) == 
 
 // Logical workgroup index: runs of kXcdChunk consecutive tiles go to one
 // XCD, and consecutive runs to consecutive XCDs.
-__device__ __forceinline__ unsigned xcd_block()
+// `skip` workgroups (a multiple of the XCDs) before them do something else.
+__device__ __forceinline__ unsigned xcd_block(unsigned skip = 0)
 {
-    const unsigned b = blockIdx.x, nb = gridDim.x;
+    const unsigned b = blockIdx.x - skip, nb = gridDim.x - skip;
     const unsigned full = nb / (kXcds * kXcdChunk) * (kXcds * kXcdChunk);
     if (b >= full)
         return b; // the last, partial round keeps dispatch order
@@ -131,18 +132,92 @@ __device__ __forceinline__ void add_pad(const sph_dev_params &P, unsigned s0, un
 }
 
 // ---------------------------------------------------------------------------
-// Tiles: the candidate ranges of one workgroup of sorted particles.
-struct TilePlan {
-    int ok;           // 1: staged in LDS; 0: read candidates from global memory
-    int rows_ok;      // 1 (when not ok): each candidate row (dy) fits on its own
-    unsigned jA;      // first cell row of the group
-    unsigned g0[6];   // segment sorted begin, segment = (row - jA) * 3 + dy + 1
-    unsigned len[6];  // segment length
-    int off[6];       // LDS index = k + off[segment]
-    unsigned tb[6];   // LDS index of the segment's first record (~0u: no segment)
+// Tiles: the candidate ranges of one workgroup of sorted particles.  The plan
+// (sph_tile_plan) is uniform over the workgroup, so all of this stays in
+// scalar registers.
+struct Tile {
+    int off[6];       // LDS index = sorted position + off[segment]
+    unsigned tb[6];   // LDS index of the segment's first record
+    unsigned g0[6], len[6];
     unsigned total;   // staged records
-    unsigned sv[12];  // the segments' bounding cell starts, read by 12 threads
+    bool ok;          // staged in LDS; else read candidates from global memory
+    bool rows_ok;     // (when not ok) each candidate row (dy) fits on its own
 };
+
+// A group is staged when its rows hold at most `cap` records.
+__device__ __forceinline__ Tile make_tile(const sph_tile_plan &p, unsigned cap)
+{
+    Tile T;
+    T.total = 0;
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+        T.g0[q] = p.g0[q];
+        T.len[q] = p.len[q];
+        T.tb[q] = T.total;
+        T.off[q] = (int)T.total - (int)p.g0[q];
+        T.total += p.len[q];
+    }
+    T.ok = !p.wide && T.total <= cap;
+    T.rows_ok = !p.wide && T.len[0] + T.len[3] <= cap && T.len[1] + T.len[4] <= cap &&
+                T.len[2] + T.len[5] <= cap;
+    return T;
+}
+
+// Plan p of a context of `tiles` 256-slot tiles, by the eight lanes of a wave
+// that share p: plans 0 .. tiles - 1 are the whole tiles', the rest those of
+// their quarters (where the context has them).  Lane q < 6 makes segment q,
+// lane 6 the rest.
+__device__ __forceinline__ void make_plan(unsigned p, unsigned tiles,
+                                          const sph_dev_params *__restrict__ Pp,
+                                          const int *__restrict__ BS,
+                                          const unsigned *__restrict__ skey,
+                                          const unsigned *__restrict__ start,
+                                          const sph_tile_plans &plans)
+{
+    const unsigned q = threadIdx.x % 8u;
+    const bool quarter = p >= tiles;
+    const unsigned n = quarter ? p - tiles : p, size = quarter ? 64u : (unsigned)kTPB;
+    if (quarter && (!plans.t64 || n >= 4u * tiles))
+        return;
+    const int scene = BS[quarter ? n / 4u : n];
+    const sph_dev_params &P = Pp[scene];
+    const unsigned f = n * size, end = P.poff + (unsigned)P.n; // f: the plan's first particle
+    if (f >= end)
+        return;
+    sph_tile_plan *out = (quarter ? plans.t64 : plans.t256) + n;
+    const unsigned sx = P.sx, sy = P.sy;
+    const unsigned kf = skey[f] - P.cell_base, kl = skey[min(f + size, end) - 1u] - P.cell_base;
+    const unsigned jA = kf / sx, jB = kl / sx;
+    const bool wide = jB > jA + 1;
+    if (q < 6u) {
+        const unsigned rho = q / 3u, j = jA + rho;
+        const long r = (long)j + (long)(q % 3u) - 1;
+        unsigned a = 0, b = 0;
+        if (!wide && j <= jB && r >= 0 && r < (long)sy) {
+            const unsigned lo = rho == 0 ? kf - jA * sx : 0;
+            const unsigned hi = j == jB ? kl - jB * sx : sx - 1;
+            const unsigned row = P.cell_base + (unsigned)r * sx;
+            a = start[row + (lo > 0 ? lo - 1 : 0)];
+            b = start[row + (hi + 1 < sx ? hi + 1 : sx - 1) + 1];
+        }
+        out->g0[q] = a;
+        out->len[q] = b - a;
+    } else if (q == 6u) {
+        out->jA = jA;
+        out->split = jB > jA ? start[P.cell_base + (jA + 1) * sx] : ~0u;
+        out->scene = scene;
+        out->wide = wide ? 1u : 0u;
+    }
+}
+
+// Workgroups that make all plans, eight lanes each; a multiple of the XCDs.
+constexpr unsigned kPlansPerGroup = kTPB / 8;
+unsigned plan_groups(unsigned slots, const sph_tile_plans &plans)
+{
+    const unsigned n = slots / kTPB * (plans.t64 ? 5u : 1u);
+    const unsigned g = (n + kPlansPerGroup - 1) / kPlansPerGroup;
+    return (g + kXcds - 1) / kXcds * kXcds;
+}
 
 // Slot of this lane's particle within its cell `key` for the counting sort.
 // The wavefront's live lanes are grouped by key first (ballots, no memory),
@@ -172,69 +247,6 @@ __device__ __forceinline__ unsigned wave_slot(unsigned *cnt, unsigned key)
     if ((int)lane == leader)
         base = atomicAdd(&cnt[key], (unsigned)__popcll(mine));
     return __shfl(base, leader, 64) + rank;
-}
-
-// The tile plan of the sorted particles [s0, s1) of a workgroup, given the
-// keys of s0 and s1 - 1 (the caller reads them early): the segments of the
-// candidate rows of its (at most two) cell rows, i.e. for each row the
-// sorted range of cells c0-1 .. c1+1.  Made by the whole workgroup: threads
-// 0..11 read one segment-bounding cell start each, and thread 0 assembles
-// the plan from those with no memory access of its own.  Ends with a
-// barrier.  The group is staged when its rows hold at most `cap` records.
-__device__ void plan_tile_par(unsigned key_first, unsigned key_last,
-                              const unsigned *__restrict__ start, const sph_dev_params &P,
-                              TilePlan &T, unsigned cap)
-{
-    const unsigned sx = P.sx, sy = P.sy;
-    const unsigned kf = key_first - P.cell_base, kl = key_last - P.cell_base;
-    const unsigned jA = kf / sx, jB = kl / sx;
-    const unsigned t = threadIdx.x;
-    if (t < 12u && jB <= jA + 1) {
-        const unsigned q = t / 2u, rho = q / 3u;
-        const long r = (long)(jA + rho) + (long)(q % 3u) - 1;
-        if (rho <= jB - jA && r >= 0 && r < (long)sy) {
-            const unsigned j = jA + rho;
-            const unsigned lo = rho == 0 ? kf % sx : 0;
-            const unsigned hi = j == jB ? kl % sx : sx - 1;
-            const unsigned c0 = lo > 0 ? lo - 1 : 0;
-            const unsigned c1 = hi + 1 < sx ? hi + 1 : sx - 1;
-            T.sv[t] = start[P.cell_base + (unsigned)r * sx + ((t & 1u) ? c1 + 1 : c0)];
-        }
-    }
-    __syncthreads();
-    if (t == 0) {
-        T.jA = jA;
-        T.ok = 0;
-        T.rows_ok = 0;
-        for (int q = 0; q < 6; q++) {
-            T.g0[q] = 0;
-            T.len[q] = 0;
-            T.off[q] = 0;
-            T.tb[q] = ~0u;
-        }
-        T.total = 0;
-        if (jB <= jA + 1) {
-            unsigned total = 0;
-            for (unsigned rho = 0; rho <= jB - jA; rho++)
-                for (int dy = -1; dy <= 1; dy++) {
-                    const long r = (long)(jA + rho) + dy;
-                    if (r < 0 || r >= (long)sy)
-                        continue;
-                    const int q = (int)rho * 3 + dy + 1;
-                    const unsigned a = T.sv[2 * q], b = T.sv[2 * q + 1];
-                    T.g0[q] = a;
-                    T.len[q] = b - a;
-                    T.off[q] = (int)total - (int)a;
-                    T.tb[q] = total;
-                    total += b - a;
-                }
-            T.ok = total <= cap;
-            T.total = total;
-            T.rows_ok = T.len[0] + T.len[3] <= cap && T.len[1] + T.len[4] <= cap &&
-                        T.len[2] + T.len[5] <= cap;
-        }
-    }
-    __syncthreads();
 }
 
 // LDS storage of a tile of CAPACITY records (plus the walk's padding): as
@@ -287,7 +299,7 @@ __device__ __forceinline__ auto tile_mem(float4 *tile)
 // or before it), issues all of its loads, and only then stores them - one
 // memory round trip per workgroup, not one per segment.
 template <int CAPACITY, class Mem, class Load>
-__device__ __forceinline__ void stage_tile(const TilePlan &T, const Mem &tile, Load load)
+__device__ __forceinline__ void stage_tile(const Tile &T, const Mem &tile, Load load)
 {
     using Rec = typename Mem::Rec;
     constexpr int kPer = (CAPACITY + kTPB - 1) / kTPB;
@@ -317,7 +329,7 @@ __device__ __forceinline__ void stage_tile(const TilePlan &T, const Mem &tile, L
 // dy + 4 of the second, back to back) into the tile, then barrier: for groups
 // whose rows fit one at a time but not all together.
 template <int CAPACITY, class Mem, class Load>
-__device__ __forceinline__ void stage_row(const TilePlan &T, int dy, const Mem &tile, Load load)
+__device__ __forceinline__ void stage_row(const Tile &T, int dy, const Mem &tile, Load load)
 {
     using Rec = typename Mem::Rec;
     constexpr int kPer = (CAPACITY + kTPB - 1) / kTPB;
@@ -341,22 +353,20 @@ __device__ __forceinline__ void stage_row(const TilePlan &T, int dy, const Mem &
 }
 
 // Candidate source reading the LDS tile: the tile index of sorted position
-// k of row dy is k + row(dy).  The offsets stay in the plan, in LDS: each is
-// needed once per row, and registers decide how many waves run.
+// k of row dy is k + row(dy).
 template <class Mem>
 struct LdsSrc {
     Mem tile;
-    const TilePlan *T;
-    int seg; // 0, or 3 for a lane in the group's second cell row
-    __device__ int row(int dy) const { return T->off[seg + dy + 1]; }
+    const Tile &T;
+    bool rowB; // the lane is in the group's second cell row
+    __device__ int row(int dy) const { return rowB ? T.off[dy + 4] : T.off[dy + 1]; }
     __device__ typename Mem::Rec at(unsigned idx) const { return tile.get(idx); }
 };
 
 template <class Mem>
-__device__ __forceinline__ LdsSrc<Mem> lds_src(const Mem &tile, const TilePlan &T, unsigned key,
-                                              const sph_dev_params &P)
+__device__ __forceinline__ LdsSrc<Mem> lds_src(const Mem &tile, const Tile &T, bool rowB)
 {
-    return LdsSrc<Mem>{tile, &T, (key - P.cell_base) / P.sx != T.jA ? 3 : 0};
+    return LdsSrc<Mem>{tile, T, rowB};
 }
 
 // The source of a tile staged by stage_row(dy): its first cell row's segment
@@ -364,21 +374,20 @@ __device__ __forceinline__ LdsSrc<Mem> lds_src(const Mem &tile, const TilePlan &
 template <class Mem>
 struct LdsRowSrc {
     Mem tile;
-    const TilePlan *T;
+    const Tile &T;
     bool rowB;
     __device__ int row(int dy) const
     {
         const int qa = dy + 1, qb = dy + 4;
-        return rowB ? (int)T->len[qa] - (int)T->g0[qb] : -(int)T->g0[qa];
+        return rowB ? (int)T.len[qa] - (int)T.g0[qb] : -(int)T.g0[qa];
     }
     __device__ typename Mem::Rec at(unsigned idx) const { return tile.get(idx); }
 };
 
 template <class Mem>
-__device__ __forceinline__ LdsRowSrc<Mem> lds_row_src(const Mem &tile, const TilePlan &T,
-                                                      unsigned key, const sph_dev_params &P)
+__device__ __forceinline__ LdsRowSrc<Mem> lds_row_src(const Mem &tile, const Tile &T, bool rowB)
 {
-    return LdsRowSrc<Mem>{tile, &T, (key - P.cell_base) / P.sx != T.jA};
+    return LdsRowSrc<Mem>{tile, T, rowB};
 }
 
 // Candidate source reading global memory.
@@ -395,25 +404,37 @@ __device__ __forceinline__ GlobalSrc<Rec, Load> global_src(Load l)
     return GlobalSrc<Rec, Load>{l};
 }
 
+// The cell row of the lane's particle (a pad lane's: row 0, its stand-in
+// cell's), from the plan unless the tile spans more than two.
+__device__ __forceinline__ unsigned cell_row(const sph_tile_plan &T, bool live, unsigned s,
+                                             unsigned key, const sph_dev_params &P)
+{
+    if (T.wide)
+        return (key - P.cell_base) / P.sx;
+    return live ? T.jA + (s >= T.split ? 1u : 0u) : 0u;
+}
+
 // Walk a workgroup's candidates from its LDS tile (CAPACITY records) if the
 // plan staged one, else from global memory (same order, same results).  Every
 // thread of the workgroup calls this (the staging and its barrier need all of
 // them); `live` lanes walk.
 template <bool CAP, int CAPACITY, int LP = 1, class Rec, class Load, class Test, class Body,
           class Masks>
-__device__ __forceinline__ uint2 walk_group(const TilePlan &T, Rec *tile, Load load, bool live,
-                                            unsigned self, const sph_rows &R, unsigned key,
-                                            const sph_dev_params &P,
+__device__ __forceinline__ uint2 walk_group(const sph_tile_plan &plan, Rec *tile, Load load,
+                                            bool live, unsigned self, const sph_rows &R,
+                                            unsigned key, unsigned j, const sph_dev_params &P,
                                             const unsigned *__restrict__ start, Test &test,
                                             Body &body, Masks &mk)
 {
+    const Tile T = make_tile(plan, CAPACITY);
+    const bool rowB = self >= plan.split;
     uint2 fh = make_uint2(0u, 0u);
     const auto mem = tile_mem<CAPACITY>(tile);
-    auto rows = [&] { return sph_row_bounds(key, P, start); };
+    auto rows = [&] { return sph_row_bounds(key, j, P, start); };
     if (T.ok) {
         stage_tile<CAPACITY>(T, mem, load);
         if (live)
-            fh = sph_walk_masked<CAP, LP>(self, R, lds_src(mem, T, key, P), P.h2, P.bucket_cap,
+            fh = sph_walk_masked<CAP, LP>(self, R, lds_src(mem, T, rowB), P.h2, P.bucket_cap,
                                           test, body, mk, rows);
     } else if (T.rows_ok) {
         // one candidate row at a time: same chunks, same order
@@ -423,7 +444,7 @@ __device__ __forceinline__ uint2 walk_group(const TilePlan &T, Rec *tile, Load l
             stage_row<CAPACITY>(T, dy, mem, load);
             if (live) {
                 const uint2 r = sph_walk_rows<CAP, dy, dy, LP>(self, R,
-                                                               lds_row_src(mem, T, key, P), P.h2,
+                                                               lds_row_src(mem, T, rowB), P.h2,
                                                                P.bucket_cap, test, body, mk, rows,
                                                                ci);
                 fh.x += r.x;
@@ -457,15 +478,14 @@ __device__ __forceinline__ uint2 walk_group(const TilePlan &T, Rec *tile, Load l
 template <bool GRAV, bool VISC, bool PRED, bool CAP, int LP = 1>
 __device__ __forceinline__ void
 visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-                  const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
-                  const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+                  const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+                  const float2 *__restrict__ VEL, const unsigned *__restrict__ K, const unsigned *__restrict__ start,
                   float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                   unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                   sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                   float2 *__restrict__ held_vel)
 {
 
-    __shared__ TilePlan T;
     __shared__ float4 tile[VISC ? kTileCap + kSphWalkPad : 1];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
     const unsigned blk = xcd_block();
@@ -476,7 +496,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     // is live)
     const float2 a0 = POS[s], av0 = VEL[s];
     const unsigned ks = VISC ? K[s] : 0u;
-    const unsigned kf0 = VISC ? K[s0] : 0u, kl0 = VISC ? K[s0 + kPer - 1] : 0u;
+    const sph_tile_plan T = VISC ? plans[blk] : sph_tile_plan{};
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -507,7 +527,8 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     const float2 a = a0, av = av0;
     const bool live = s < s1;
     const unsigned key = VISC && live ? ks : P.cell_base; // pad lanes: any valid cell
-    const sph_rows R = VISC ? sph_row_bounds(key, P, start) : sph_rows{};
+    const unsigned j = VISC ? cell_row(T, live, s, key, P) : 0u;
+    const sph_rows R = VISC ? sph_row_bounds(key, j, P, start) : sph_rows{};
     const float avx = slosh ? av.x + sdt : av.x;
     const float avy = GRAV ? av.y + gdt : av.y;
     float nvx = avx, nvy = avy;
@@ -529,7 +550,6 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
         auto half_impulse = [&](float4 b) {
             return sph_visc_half(a.x, a.y, avx, avy, b.x, b.y, b.z, b.w, V, P);
         };
-        plan_tile_par(kf0, s1 - s0 == kPer ? kl0 : K[s1 - 1], start, P, T, kTileCap);
         sph_masks_none mk;
         uint2 fh;
         if constexpr (LP == 1) {
@@ -538,7 +558,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
                 nvx = nvx - t.x;
                 nvy = nvy - t.y;
             };
-            fh = walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, P, start, test, body,
+            fh = walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body,
                                            mk);
         } else {
             auto term = [&](unsigned, float4 b, auto &&, bool &) {
@@ -551,7 +571,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
             };
             auto never = [](bool) {};
             sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply, never};
-            fh = walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb,
+            fh = walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb,
                                                mk);
         }
         full = fh.x;
@@ -577,14 +597,14 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
 template <bool GRAV, bool VISC, bool PRED, bool CAP>
 __global__ void __launch_bounds__(kTPB, kGatherMinBlocks)
 k_visc_predict(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-               const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
+               const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
                const unsigned *__restrict__ K, const unsigned *__restrict__ start,
                float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                float2 *__restrict__ held_vel)
 {
-    visc_predict_tile<GRAV, VISC, PRED, CAP, 1>(Pp, BS, POS, VEL, K, start, out_pos, out_key,
+    visc_predict_tile<GRAV, VISC, PRED, CAP, 1>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
                                                 out_slot, cnt, C, clock, held_vel);
 }
 
@@ -592,14 +612,14 @@ k_visc_predict(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
 k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-                    const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
+                    const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
                     const unsigned *__restrict__ K, const unsigned *__restrict__ start,
                     float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                     unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                     sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                     float2 *__restrict__ held_vel)
 {
-    visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, POS, VEL, K, start, out_pos, out_key,
+    visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
                                                 out_slot, cnt, C, clock, held_vel);
 }
 
@@ -815,16 +835,26 @@ k_scatter(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 // holds more than the reference's 100 bucket slots (src/fluid.c:174).
 constexpr unsigned kRankBatch = 8;
 constexpr unsigned kRankHalo = 64; // staged ids either side of a workgroup's positions
-
+// The launch's first `planners` workgroups make the tile plans of the sorted
+// positions for the gathers that follow, beside the others, which rank and
+// move the particles.  (Made by the ranking workgroups themselves, by some of
+// their lanes or by a fifth wave, the plans lengthened the 10.6 us of a
+// reorder of 1M particles to 11.2 - 13.0.)
 template <int NF>
 __global__ void __launch_bounds__(kTPB)
 k_reorder(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
           const unsigned *__restrict__ start, const int *__restrict__ perm_src,
           const int *__restrict__ perm_id, const unsigned *__restrict__ skey,
-          sph_reorder_fields<NF> f, int *__restrict__ id_dst, sph_dev_counters *__restrict__ C)
+          sph_reorder_fields<NF> f, int *__restrict__ id_dst, unsigned planners,
+          sph_tile_plans plans, sph_dev_counters *__restrict__ C)
 {
     __shared__ int wid[kTPB + 2 * kRankHalo];
-    const unsigned blk = xcd_block();
+    if (blockIdx.x < planners) {
+        make_plan(blockIdx.x * kPlansPerGroup + threadIdx.x / 8u, gridDim.x - planners, Pp, BS,
+                  skey, start, plans);
+        return;
+    }
+    const unsigned blk = xcd_block(planners);
     const sph_dev_params &P = Pp[BS[blk]];
     const unsigned s0 = blk * kTPB;
     const unsigned end = P.poff + (unsigned)P.n;
@@ -904,18 +934,26 @@ k_reorder(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         raise_max(&C->max_cell_count, m);
 }
 
+// The tile plans alone (sph_launch_plan).
+__global__ void __launch_bounds__(kTPB)
+k_plan(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned tiles,
+       const unsigned *__restrict__ start, const unsigned *__restrict__ skey,
+       sph_tile_plans plans)
+{
+    make_plan(blockIdx.x * kPlansPerGroup + threadIdx.x / 8u, tiles, Pp, BS, skey, start, plans);
+}
+
 // ---------------------------------------------------------------------------
 // Density (src/hash.c:190-194, 225-229 with src/fluid.c:527-539) in gather
 // form: each particle sums (1-r/h)^2 and (1-r/h)^3 over its neighbours.
 template <bool CAP, int LP = 1>
 __device__ __forceinline__ void
 density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-             const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+             const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
              const unsigned *__restrict__ start, float2 *__restrict__ RHO,
              uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
 
-    __shared__ TilePlan T;
     // positions only: twice the candidates of the other gathers' float4
     // tiles in the same LDS bytes, so denser rows stay in LDS at no cost in
     // occupancy (registers allow 7 workgroups per CU either way)
@@ -924,10 +962,11 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
     const unsigned s = s0 + threadIdx.x / LP;
-    // the lane's own particle and the tile's end keys, before the scene
+    // the lane's own particle and the tile's plan, before the scene
     // parameters (every slot of the grid is inside the arrays)
     const float2 a = POS[s];
-    const unsigned ks = K[s], kf0 = K[s0], kl0 = K[s0 + kPer - 1];
+    const unsigned ks = K[s];
+    const sph_tile_plan T = plans[blk];
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -936,8 +975,8 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // the candidate rows, before the barriers
     const bool live = s < s1;
     const unsigned key = live ? ks : P.cell_base; // pad lanes: any valid cell
-    const sph_rows R = sph_row_bounds(key, P, start);
-    plan_tile_par(kf0, s1 - s0 == kPer ? kl0 : K[s1 - 1], start, P, T, 2 * kTileCap);
+    const unsigned j = cell_row(T, live, s, key, P);
+    const sph_rows R = sph_row_bounds(key, j, P, start);
     float rho = 0.0f, rhon = 0.0f;
     auto load = [&](unsigned g) { return POS[g]; };
     auto test = [&](float2 b) {
@@ -969,7 +1008,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             rho = rho + t.x;
             rhon = rhon + t.y;
         };
-        fh = walk_group<CAP, 2 * kTileCap>(T, tile, load, live, s, R, key, P, start, test, body,
+        fh = walk_group<CAP, 2 * kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body,
                                            mk);
     } else {
         auto term = [&](unsigned, float2 b, auto &&, bool &) {
@@ -982,7 +1021,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         };
         auto never = [](bool) {};
         sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply, never};
-        fh = walk_group<CAP, 2 * kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb,
+        fh = walk_group<CAP, 2 * kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb,
                                                mk);
     }
     if (live && lead) {
@@ -996,22 +1035,22 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, kGatherMinBlocks)
 k_density(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-          const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+          const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
           const unsigned *__restrict__ start, float2 *__restrict__ RHO,
           uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
-    density_tile<CAP, 1>(Pp, BS, POS, K, start, RHO, masks, C);
+    density_tile<CAP, 1>(Pp, BS, plans, POS, K, start, RHO, masks, C);
 }
 
 // Four lanes per particle.
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
 k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-               const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+               const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
                const unsigned *__restrict__ start, float2 *__restrict__ RHO,
                uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
-    density_tile<CAP, 4>(Pp, BS, POS, K, start, RHO, masks, C);
+    density_tile<CAP, 4>(Pp, BS, plans, POS, K, start, RHO, masks, C);
 }
 
 // Double-density relaxation (src/fluid.c:541-611) in gather form.
@@ -1021,7 +1060,7 @@ k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS
 template <bool FUSED, bool CAP, int LP = 1>
 __device__ __forceinline__ void
 relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-           const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+           const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
            const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
            const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
            float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
@@ -1030,15 +1069,15 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
            unsigned long long *__restrict__ clock)
 {
 
-    __shared__ TilePlan T;
     __shared__ float4 tile[kTileCap + kSphWalkPad];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
     const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
     const unsigned s = s0 + threadIdx.x / LP;
-    // the lane's own key and the tile's end keys, before the scene
+    // the lane's own key and the tile's plan, before the scene
     // parameters (every slot of the grid is inside the arrays)
-    const unsigned ks = K[s], kf0 = K[s0], kl0 = K[s0 + kPer - 1];
+    const unsigned ks = K[s];
+    const sph_tile_plan T = plans[blk];
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -1067,8 +1106,8 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const float2 ar = RHO[s];
     const bool live = s < s1;
     const unsigned key = live ? ks : P.cell_base; // pad lanes: any valid cell
-    const sph_rows R = sph_row_bounds(key, P, start);
-    plan_tile_par(kf0, s1 - s0 == kPer ? kl0 : K[s1 - 1], start, P, T, kTileCap);
+    const unsigned j = cell_row(T, live, s, key, P);
+    const sph_rows R = sph_row_bounds(key, j, P, start);
     // a neighbour's record carries its pressure and near-pressure
     // (src/fluid.c:563-564), evaluated once per record rather than per pair
     auto load = [&](unsigned g) {
@@ -1118,10 +1157,10 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         auto body = [&](unsigned, float4 b, auto &&own) { apply(pair(b, own, nudge)); };
         if (FUSED) { // the density pass of this step walked the same neighbour set
             sph_masks_replay mk{live ? masks[s] : make_uint4(0u, 0u, 0u, 0u)};
-            walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, P, start, test, body, mk);
+            walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body, mk);
         } else {
             sph_masks_none mk;
-            walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, P, start, test, body, mk);
+            walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body, mk);
         }
     } else {
         auto term = [&](unsigned, float4 b, auto &&own, bool &nudged) {
@@ -1130,10 +1169,10 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         sph_split_body<decltype(term), decltype(apply), decltype(nudge)> sb{term, apply, nudge};
         if (FUSED) {
             sph_masks_replay mk{live ? masks[s] : make_uint4(0u, 0u, 0u, 0u)};
-            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb, mk);
+            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb, mk);
         } else {
             sph_masks_none mk;
-            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, P, start, test, sb, mk);
+            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb, mk);
         }
     }
     if (!live || !lead)
@@ -1157,7 +1196,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool FUSED, bool CAP>
 __global__ void __launch_bounds__(kTPB, CAP ? kGatherMinBlocks - 1 : kGatherMinBlocks)
 k_relax(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-        const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+        const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
         const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
         const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
         float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
@@ -1165,7 +1204,7 @@ k_relax(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
         unsigned long long *__restrict__ clock)
 {
-    relax_tile<FUSED, CAP, 1>(Pp, BS, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
+    relax_tile<FUSED, CAP, 1>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
                               cnt, masks, C, clock);
 }
 
@@ -1173,7 +1212,7 @@ k_relax(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
 k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-             const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+             const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
              const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
              const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
              float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
@@ -1181,7 +1220,7 @@ k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
              const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
              unsigned long long *__restrict__ clock)
 {
-    relax_tile<true, CAP, 4>(Pp, BS, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
+    relax_tile<true, CAP, 4>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
                              cnt, masks, C, clock);
 }
 
@@ -1479,17 +1518,17 @@ int sph_gather_lanes(unsigned slots)
 }
 
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
-                             bool cap, const sph_dev_params *P, const int *BS, const float2 *POS,
-                             const float2 *VEL, const unsigned *K, const unsigned *start,
+                             bool cap, const sph_dev_params *P, const int *BS,
+                             const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,
                              float2 *opos, unsigned *okey, unsigned *oslot, unsigned *cnt,
                              sph_dev_counters *C, const unsigned long long *clock,
                              float2 *held_vel, int lanes)
 {
 #define VP(G, V, R, CAP)                                                                         \
-    launch(k_visc_predict<G, V, R, CAP>, GRID(slots), kTPB, st, P, BS, POS, VEL, K, start, opos, \
+    launch(k_visc_predict<G, V, R, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, VEL, K, start, opos, \
            okey, oslot, cnt, C, clock, held_vel)
 #define VP4(CAP)                                                                                 \
-    launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, POS,    \
+    launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS,    \
            VEL, K, start, opos, okey, oslot, cnt, C, clock, held_vel)
 #define VPC(G, V, R)                                                                             \
     do {                                                                                         \
@@ -1592,50 +1631,59 @@ void sph_launch_scatter(hipStream_t st, unsigned slots, const sph_dev_params *P,
 void sph_launch_reorder2(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                          const unsigned *start, const int *perm_src, const int *perm_id,
                          const unsigned *skey, sph_reorder_fields<2> f, int *id_dst,
-                         sph_dev_counters *C)
+                         const sph_tile_plans &plans, sph_dev_counters *C)
 {
-    launch(k_reorder<2>, GRID(slots), kTPB, st, P, BS, start, perm_src, perm_id, skey, f, id_dst,
-                                               C);
+    const unsigned planners = plan_groups(slots, plans);
+    launch(k_reorder<2>, dim3(planners + slots / kTPB), kTPB, st, P, BS, start, perm_src, perm_id,
+           skey, f, id_dst, planners, plans, C);
 }
 
 void sph_launch_reorder4(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                          const unsigned *start, const int *perm_src, const int *perm_id,
                          const unsigned *skey, sph_reorder_fields<4> f, int *id_dst,
-                         sph_dev_counters *C)
+                         const sph_tile_plans &plans, sph_dev_counters *C)
 {
-    launch(k_reorder<4>, GRID(slots), kTPB, st, P, BS, start, perm_src, perm_id, skey, f, id_dst,
-                                               C);
+    const unsigned planners = plan_groups(slots, plans);
+    launch(k_reorder<4>, dim3(planners + slots / kTPB), kTPB, st, P, BS, start, perm_src, perm_id,
+           skey, f, id_dst, planners, plans, C);
+}
+
+void sph_launch_plan(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
+                     const unsigned *start, const unsigned *skey, const sph_tile_plans &plans)
+{
+    launch(k_plan, dim3(plan_groups(slots, plans)), kTPB, st, P, BS, slots / kTPB, start, skey,
+           plans);
 }
 
 void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_params *P,
-                        const int *BS, const float2 *POS, const unsigned *K,
+                        const int *BS, const sph_tile_plans &plans, const float2 *POS, const unsigned *K,
                         const unsigned *start, float2 *RHO, uint4 *masks, sph_dev_counters *C,
                         int lanes)
 {
     if (lanes == 4 && cap)
-        launch(k_density_quad<true>, GRID(4 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
+        launch(k_density_quad<true>, GRID(4 * slots), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
                C);
     else if (lanes == 4)
-        launch(k_density_quad<false>, GRID(4 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
+        launch(k_density_quad<false>, GRID(4 * slots), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
                C);
     else if (cap)
-        launch(k_density<true>, GRID(slots), kTPB, st, P, BS, POS, K, start, RHO, masks, C);
+        launch(k_density<true>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO, masks, C);
     else
-        launch(k_density<false>, GRID(slots), kTPB, st, P, BS, POS, K, start, RHO, masks, C);
+        launch(k_density<false>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO, masks, C);
 }
 
 void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
-                      const sph_dev_params *P, const int *BS, const float2 *POS,
-                      const float2 *PREV, const float2 *RHO, const unsigned *K,
+                      const sph_dev_params *P, const int *BS, const sph_tile_plans &plans,
+                      const float2 *POS, const float2 *PREV, const float2 *RHO, const unsigned *K,
                       const unsigned *start, float2 *opos, float2 *ovel, unsigned *okey,
                       unsigned *oslot, unsigned *cnt, const uint4 *masks, sph_dev_counters *C,
                       unsigned long long *clock, int lanes)
 {
 #define RL(F, CAP)                                                                               \
-    launch(k_relax<F, CAP>, GRID(slots), kTPB, st, P, BS, POS, PREV, RHO, K, start, opos, ovel,   \
+    launch(k_relax<F, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, start, opos, ovel,   \
            okey, oslot, cnt, masks, C, clock)
 #define RL4(CAP)                                                                                 \
-    launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, POS, PREV, RHO, K, start,  \
+    launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, PREV, RHO, K, start,  \
            opos, ovel, okey, oslot, cnt, masks, C, clock)
     // four lanes per particle for the fused step's variant only
     if (fused && lanes == 4 && cap)
