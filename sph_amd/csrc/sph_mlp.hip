@@ -17,10 +17,15 @@
 // Precision: weights and activations bf16, MFMA 16x16x16 bf16 with fp32
 // accumulation, SiLU / sums / losses / Adam in fp32 (fp32 master weights).
 //
-// Work layout: one wavefront per particle for the edge passes (its
-// neighbours are compacted into LDS, 16 edges per MFMA tile), one wavefront
-// per 16 consecutive particles for the node passes, split-K MFMA reductions
-// for the weight gradients.  Particles are the solver context's sorted slots.
+// Work layout: one wavefront per 16 consecutive particles everywhere (the
+// solver context's sorted slots).  The edge passes compact the group's edges
+// into LDS, 16 per MFMA tile.  Every product is taken with the weights as the
+// A operand and the particles (or the edge sums) as columns, because the
+// 16x16x16 MFMA returns, per lane, rows 4 (l / 16) .. + 3 of column l % 16: the
+// very layout its B operand takes.  So the layers chain in registers, forward
+// and backward, and where a product needs the other layout (the weight
+// gradients sum over particles) the values are turned by an MFMA with the
+// identity, exactly, on otherwise idle matrix cores.
 #include "sph_ctx_internal.h"
 
 #include <math.h>
@@ -34,7 +39,6 @@
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) short bf16x4;
-typedef __attribute__((ext_vector_type(4))) __bf16 bfx4;
 
 namespace {
 
@@ -42,7 +46,8 @@ constexpr int kH = 64;      // hidden width
 constexpr int kKE = 16;     // edge input width (6 used)
 constexpr int kKN = 80;     // node input width (64 + 4 + bias, padded)
 constexpr unsigned kGroup = 16;         // consecutive slots per wavefront in the edge passes
-constexpr unsigned kEdgeBuf = 256;      // LDS edge rows per wavefront (flushed as it fills)
+constexpr unsigned kEdgeBuf = 176;      // LDS edge rows per wavefront (flushed as it fills)
+constexpr unsigned kNoOwner = 16;       // owner of a padding row: no particle of the group
 constexpr float kVScale = 0.2f, kAScale = 0.1f, kDScale = 0.05f;
 constexpr int kTrendRefresh = 16; // forced plain macro-step per scene every this many
 
@@ -78,11 +83,20 @@ __device__ __forceinline__ float silu_grad(float x)
     return s * (1.0f + x * (1.0f - s));
 }
 
+// Two conversions an instruction (the four-wide conversion compiles to one
+// each and two byte permutes).
 __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d)
 {
-    const f32x4 v = {a, b, c, d};
-    return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, bfx4));
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 bfx2;
+    const f32x2 lo = {a, b}, hi = {c, d};
+    uint2 r;
+    r.x = __builtin_bit_cast(unsigned, __builtin_convertvector(lo, bfx2));
+    r.y = __builtin_bit_cast(unsigned, __builtin_convertvector(hi, bfx2));
+    return __builtin_bit_cast(bf16x4, r);
 }
+
+__device__ __forceinline__ bf16x4 pack4(f32x4 v) { return pack4(v[0], v[1], v[2], v[3]); }
 
 __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c)
 {
@@ -106,158 +120,208 @@ __device__ __forceinline__ NodeCtx node_ctx(const sph_dev_params &P, unsigned lo
     return c;
 }
 
+// This wavefront's index in its workgroup, as a scalar: what follows from it
+// (the group, its scene's parameters) is uniform and stays in scalar registers.
+__device__ __forceinline__ unsigned wave_index()
+{
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64u));
+}
+
 // LDS edge list of one wavefront's group of kGroup consecutive slots:
 // features (dx/h, dy/h, 0.2 dvx, 0.2 dvy, r/h, 1, 0, 0) as two bf16x4, and
-// the owning particle (0..15 within the group; 0xff for padding rows).
+// the owning particle (0..15 within the group; kNoOwner for padding rows).
 struct EdgeBuf {
     bf16x4 f[kEdgeBuf][2];
     unsigned char owner[kEdgeBuf];
 };
 
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+}
+
 // Stream every edge of the particles [n0, n0 + 16) through L (one
-// wavefront).  Lane l tests particle l % 16 against every fourth candidate
-// (offset l / 16) of each of the particle's three candidate rows (cells
-// i-1..i+1 of rows j-1..j+1, contiguous in the sorted arrays), so all 64
-// lanes test useful pairs.  Accepted edges are appended to L in arbitrary
-// order; whenever L is nearly full, flush(nedges) consumes its first nedges
-// (a multiple of 16) and the remainder moves to the front.  The final call
-// gets the rest, padded to a multiple of 16 with zero rows owned by 0xff.
-// Lanes 0..15 get the degree and, with DENS, the density sum
-// (src/fluid.c:527-539: (1 - r/h)^2 for r/h < 1) of particle n0 + lane.
-template <bool DENS, class Flush>
-__device__ void walk_group(unsigned n0, const sph_dev_params &P, const float2 *POS,
-                           const float2 *VEL, const unsigned *K, const unsigned *start,
-                           EdgeBuf &L, Flush &&flush, float &deg_out, float &rho_out)
+// wavefront).  Lane l takes every fourth candidate (from l / 16 on) of
+// particle l % 16's three candidate rows (cells i-1..i+1 of rows j-1..j+1,
+// contiguous in the sorted arrays) taken as one list, so that a wave runs as
+// many rounds as its longest list needs; a round's records are loaded one
+// round ahead, position and velocity together.  Accepted edges are appended
+// to L in arbitrary order; whenever L is nearly full, flush(nedges) consumes
+// its first nedges (a multiple of 16) and the remainder moves to the front.
+// The final call gets the rest, padded to a multiple of 16 with zero rows of
+// no owner.  Returns the degree of particle l % 16.
+template <class Flush>
+__device__ __forceinline__ float walk_group(unsigned n0, const sph_dev_params &P,
+                                            const float2 *__restrict__ POS,
+                                            const float2 *__restrict__ VEL,
+                                            const unsigned *__restrict__ K,
+                                            const unsigned *__restrict__ start, EdgeBuf &L,
+                                            Flush &&flush)
 {
     const unsigned l = lane(), p = l % 16u, sub = l / 16u;
     const unsigned me = n0 + p;
     const bool valid = me < P.poff + (unsigned)P.n;
-    float2 a = make_float2(0, 0), av = make_float2(0, 0);
-    unsigned i = 0, j = 0;
-    if (valid) {
-        a = POS[me];
-        av = VEL[me];
-        const unsigned key = K[me] - P.cell_base;
-        i = key % P.sx;
-        j = key / P.sx;
-    }
+    const unsigned mc = valid ? me : n0; // n0 is a live slot
+    const float2 a = POS[mc], av = VEL[mc];
+    const unsigned key = K[mc] - P.cell_base;
+    const unsigned j = key / P.sx, i = key - j * P.sx;
     const unsigned lo = i > 0 ? i - 1 : 0, hi = i + 1 < P.sx ? i + 1 : P.sx - 1;
+    unsigned b0[3], n[3]; // begin and length of the candidate rows
+#pragma unroll
+    for (int dy = 0; dy < 3; dy++) {
+        const bool in = valid && (dy == 0 ? j > 0 : dy == 2 ? j + 1 < P.sy : true);
+        const unsigned base = P.cell_base + (in ? j + (unsigned)dy - 1u : j) * P.sx;
+        const unsigned s0 = start[base + lo], s3 = start[base + hi + 1];
+        b0[dy] = s0;
+        n[dy] = in ? s3 - s0 : 0u;
+    }
+    const unsigned n01 = n[0] + n[1], total = n01 + n[2];
+    // candidate t of the lane's list (its own slot past the end)
+    auto at = [&](unsigned t) {
+        unsigned c = b0[0] + t;
+        c = t >= n[0] ? b0[1] + (t - n[0]) : c;
+        c = t >= n01 ? b0[2] + (t - n01) : c;
+        return t < total ? c : mc;
+    };
     unsigned count = 0, mine = 0;
-    float dens = 0.0f;
-    for (int dy = -1; dy <= 1; dy++) {
-        const long r = (long)j + dy;
-        unsigned b0 = 0, b3 = 0;
-        if (valid && r >= 0 && r < (long)P.sy) {
-            const unsigned base = P.cell_base + (unsigned)r * P.sx;
-            b0 = start[base + lo];
-            b3 = start[base + hi + 1];
+    unsigned t = sub, c = at(t);
+    float2 q = POS[c], qv = VEL[c];
+    while (__ballot(t < total) != 0ull) {
+        const unsigned tn = t + 4u, cn = at(tn);
+        const float2 qn = POS[cn], qvn = VEL[cn];
+        const float dx = q.x - a.x, dy = q.y - a.y;
+        const float r2 = dx * dx + dy * dy;
+        const bool acc = t < total && c != me && !(r2 > P.h2);
+        const unsigned long long m = __ballot(acc);
+        const float rr = sph_sqrt(r2);
+        if (acc) {
+            const unsigned pos =
+                __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, count));
+            L.f[pos][0] = pack4(dx * P.h_recip, dy * P.h_recip, (qv.x - av.x) * kVScale,
+                                (qv.y - av.y) * kVScale);
+            L.f[pos][1] = pack4(rr * P.h_recip, 1.0f, 0.0f, 0.0f);
+            L.owner[pos] = (unsigned char)p;
+            mine++;
         }
-        for (unsigned c = b0 + sub;; c += 4) {
-            const bool act = c < b3;
-            if (__ballot(act) == 0ull)
-                break;
-            bool acc = false;
-            float dx = 0, dyy = 0, r2 = 0;
-            if (act && c != me) {
-                const float2 q = POS[c];
-                dx = q.x - a.x;
-                dyy = q.y - a.y;
-                r2 = dx * dx + dyy * dyy;
-                acc = !(r2 > P.h2);
+        count += (unsigned)__popcll(m);
+        if (count > kEdgeBuf - 64u) { // the next round might not fit: flush full tiles
+            wave_lds_order();
+            const unsigned full = count & ~15u, rem = count - full;
+            flush(full);
+            wave_lds_order();
+            bf16x4 f0 = pack4(0, 0, 0, 0), f1 = f0;
+            unsigned char ow = kNoOwner;
+            if (l < rem) {
+                f0 = L.f[full + l][0];
+                f1 = L.f[full + l][1];
+                ow = L.owner[full + l];
             }
-            const unsigned long long m = __ballot(acc);
-            if (acc) {
-                const unsigned pos = count + (unsigned)__popcll(m & ((1ull << l) - 1ull));
-                const float rr = sqrtf(r2);
-                if (DENS) {
-                    const float ratio = rr * P.h_recip;
-                    if (ratio < 1.0f)
-                        dens += (1.0f - ratio) * (1.0f - ratio);
-                }
-                mine++;
-                const float2 qv = VEL[c];
-                L.f[pos][0] = pack4(dx * P.h_recip, dyy * P.h_recip, (qv.x - av.x) * kVScale,
-                                    (qv.y - av.y) * kVScale);
-                L.f[pos][1] = pack4(rr * P.h_recip, 1.0f, 0.0f, 0.0f);
-                L.owner[pos] = (unsigned char)p;
+            wave_lds_order();
+            if (l < rem) {
+                L.f[l][0] = f0;
+                L.f[l][1] = f1;
+                L.owner[l] = ow;
             }
-            count += (unsigned)__popcll(m);
-            if (count > kEdgeBuf - 64u) { // the next batch might not fit: flush full tiles
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                const unsigned full = count & ~15u, rem = count - full;
-                flush(full);
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                bf16x4 f0 = pack4(0, 0, 0, 0), f1 = f0;
-                unsigned char ow = 0xffu;
-                if (l < rem) {
-                    f0 = L.f[full + l][0];
-                    f1 = L.f[full + l][1];
-                    ow = L.owner[full + l];
-                }
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                if (l < rem) {
-                    L.f[l][0] = f0;
-                    L.f[l][1] = f1;
-                    L.owner[l] = ow;
-                }
-                count = rem;
-            }
+            count = rem;
         }
+        t = tn;
+        c = cn;
+        q = qn;
+        qv = qvn;
     }
     // the rest, padded to a whole 16-edge tile
     const unsigned padded = (count + 15u) & ~15u;
     if (count + l < padded) {
         L.f[count + l][0] = pack4(0, 0, 0, 0);
         L.f[count + l][1] = pack4(0, 0, 0, 0);
-        L.owner[count + l] = 0xffu;
+        L.owner[count + l] = kNoOwner;
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    wave_lds_order();
     if (padded)
         flush(padded);
     float fm = (float)mine;
     fm += __shfl_xor(fm, 16, 64);
     fm += __shfl_xor(fm, 32, 64);
-    deg_out = fm;
-    if (DENS) {
-        dens += __shfl_xor(dens, 16, 64);
-        dens += __shfl_xor(dens, 32, 64);
-        rho_out = dens;
-    }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
+    return fm;
 }
 
-// A-operand of an edge tile: lane l holds edge e0 + l%16, features
-// 4*(l/16) .. +3 (features 8..15 are zero).
+// A operand of an edge tile: lane l holds edge e0 + l%16, features 4*(l/16)
+// .. +3.  Features 8..15 stand against zero weights: those lanes read the
+// first eight again.
 __device__ __forceinline__ bf16x4 edge_tile_a(const EdgeBuf &L, unsigned e0)
 {
-    const unsigned sub = lane() / 16u;
-    return sub < 2u ? L.f[e0 + lane() % 16u][sub] : pack4(0, 0, 0, 0);
+    return L.f[e0 + lane() % 16u][(lane() / 16u) & 1u];
 }
 
-// A-operand of the group membership matrix of an edge tile: lane l holds
-// row (particle) l%16, columns (edges) e0 + 4*(l/16) .. +3: 1 where the edge
-// belongs to the particle.
-__device__ __forceinline__ bf16x4 member_a(const EdgeBuf &L, unsigned e0)
+// Membership of the tile's edges e0 + 4*(l/16) .. +3 in particle l%16 (1 or
+// 0): the B operand of the sum over edges.  The four owners are compared as
+// one word (they and the particle are at most 16, so no byte carries into the
+// next): z has 0x80 in the bytes that match, and 0x3f80, bf16 1, follows from
+// it by shifts.
+__device__ __forceinline__ bf16x4 member(const EdgeBuf &L, unsigned e0)
 {
-    const unsigned p = lane() % 16u, e = e0 + 4u * (lane() / 16u);
-    bf16x4 r;
-    for (int q = 0; q < 4; q++)
-        r[q] = L.owner[e + q] == p ? (short)0x3f80 : (short)0;
-    return r;
+    const unsigned w = *(const unsigned *)&L.owner[e0 + 4u * (lane() / 16u)];
+    const unsigned x = w ^ (lane() % 16u) * 0x01010101u;
+    const unsigned z = ((x + 0x7f7f7f7fu) & 0x80808080u) ^ 0x80808080u;
+    const unsigned h = (z >> 1) - (z >> 7);
+    uint2 r;
+    r.x = __builtin_amdgcn_perm(h, z, 0x05010400u);
+    r.y = __builtin_amdgcn_perm(h, z, 0x07030602u);
+    return __builtin_bit_cast(bf16x4, r);
 }
 
-// B-operand of W1^T for hidden-unit tile t: B[k][c] = W1[16t + c][k].
+// One-hot A operand of the expansion of particles to a tile's edges: lane l
+// holds edge e0 + l%16, particles 4*(l/16) .. +3.
+__device__ __forceinline__ bf16x4 one_hot(unsigned own)
+{
+    const unsigned k = own - 4u * (lane() / 16u); // 0..3 when the owner is one of them
+    uint2 r;
+    r.x = k < 2u ? 0x3f80u << (16u * k) : 0u;
+    r.y = k - 2u < 2u ? 0x3f80u << (16u * (k - 2u)) : 0u;
+    return __builtin_bit_cast(bf16x4, r);
+}
+
+// The identity as a B operand, and a tile turned by it: x holds, per lane,
+// rows 4*(l/16) .. +3 of column l%16; the result columns 4*(l/16) .. +3 of row
+// l%16, of the same (bf16) values.
+__device__ __forceinline__ bf16x4 identity_b() { return one_hot(lane() % 16u); }
+
+__device__ __forceinline__ bf16x4 turn(bf16x4 x, bf16x4 eye)
+{
+    f32x4 d = {0, 0, 0, 0};
+    return pack4(mfma(x, eye, d));
+}
+
+// B operand of W1^T for hidden-unit tile t: B[k][c] = W1[16t + c][k].
 __device__ __forceinline__ bf16x4 w1_b(const unsigned short *W1b, int t)
 {
     const unsigned c = 16u * t + lane() % 16u, k = 4u * (lane() / 16u);
-    bf16x4 r;
-    for (int q = 0; q < 4; q++)
-        r[q] = (short)W1b[c * kKE + k + q];
-    return r;
+    return *(const bf16x4 *)(W1b + c * kKE + k);
+}
+
+// The edge sums of a group: acc[t] += SiLU(W1 f)^T over the first ne edges,
+// per lane hidden units 16t + 4*(l/16) .. +3 of particle l%16.  A tile's four
+// pre-activations come first, so that their SiLUs interleave.
+__device__ __forceinline__ void edge_sums(const EdgeBuf &L, unsigned ne, const bf16x4 B[4],
+                                          f32x4 acc[4])
+{
+    for (unsigned e0 = 0; e0 < ne; e0 += 16) {
+        const bf16x4 a = edge_tile_a(L, e0);
+        const bf16x4 mem = member(L, e0);
+        const f32x4 zero = {0, 0, 0, 0};
+        f32x4 d[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            d[t] = mfma(a, B[t], zero);
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            // D (edges 4*(l/16)+q, unit 16t + l%16) is the A layout of the sum
+            acc[t] = mfma(pack4(silu(d[t][0]), silu(d[t][1]), silu(d[t][2]), silu(d[t][3])), mem,
+                          acc[t]);
+    }
 }
 
 } // namespace
@@ -266,8 +330,11 @@ struct sph_surrogate {
     size_t slots = 0;
     float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
     unsigned short *W1b = nullptr, *W2b = nullptr, *W3b = nullptr;
-    float *S = nullptr, *deg = nullptr, *dS = nullptr, *disp = nullptr, *tgt = nullptr;
-    unsigned short *U = nullptr, *dP3 = nullptr, *dM = nullptr; // tile-major bf16
+    float *deg = nullptr, *disp = nullptr, *tgt = nullptr;
+    // training, bf16 as the products take them, [group][tile][lane]: the edge
+    // sums (particles as columns) and their gradients (particles as rows)
+    bf16x4 *S = nullptr, *dS = nullptr;
+    float *part = nullptr; // the workgroups' partial gradients
     float *loss = nullptr;
     float2 *tmp2 = nullptr;
     int adam_t = 0;
@@ -319,21 +386,23 @@ __global__ void k_mfma_selftest(float *D)
         D[(4u * (l / 16u) + q) * 16u + l % 16u] = d[q];
 }
 
-// Edge forward: S_i = sum_j SiLU(W1 f_ij) and deg_i (and, with DENS, the
-// density sum of the judge).  One wavefront per group of 16 slots: the
-// group's edges are compacted into LDS, each 16-edge tile runs
-// W1 on MFMA (4 hidden tiles), SiLU, and the per-particle sum as a second
-// MFMA against the tile's membership matrix.
-template <bool DENS>
-__global__ void __launch_bounds__(256)
+// Edge forward of training: S_i = sum_j SiLU(W1 f_ij) and deg_i.  One
+// wavefront per group of 16 slots: the group's edges are compacted into LDS,
+// each 16-edge tile runs W1 on MFMA (4 hidden tiles), SiLU, and the
+// per-particle sum as a second MFMA against the tile's membership matrix.
+// Bound by VALU issue (per tile 16 SiLUs a lane: two transcendentals and three
+// instructions each); a launch bound of more than one workgroup keeps the
+// MFMA results out of accumulation registers, which cost a read each.  A
+// million particles of 17 neighbours: 0.82 -> 0.41 ms.
+__global__ void __launch_bounds__(256, 4)
 k_edge_fwd(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned slots,
            const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
            const unsigned *__restrict__ K, const unsigned *__restrict__ start,
-           const unsigned short *__restrict__ W1b, float *__restrict__ S,
-           float *__restrict__ deg, float *__restrict__ rho)
+           const unsigned short *__restrict__ W1b, bf16x4 *__restrict__ S,
+           float *__restrict__ deg)
 {
-    __shared__ EdgeBuf Lb[4];
-    const unsigned w = threadIdx.x / 64u, l = lane(), p = l % 16u, sub = l / 16u;
+    __shared__ __align__(16) EdgeBuf Lb[4];
+    const unsigned w = wave_index(), l = lane();
     EdgeBuf &L = Lb[w];
     bf16x4 B[4];
     for (int t = 0; t < 4; t++)
@@ -341,166 +410,130 @@ k_edge_fwd(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, un
     const unsigned ngroups = slots / kGroup, nw = gridDim.x * 4u;
     for (unsigned g = blockIdx.x * 4u + w; g < ngroups; g += nw) {
         const unsigned n0 = g * kGroup;
-        const sph_dev_params &P = Pp[BS[n0 / kSphTPB]];
+        const sph_dev_params P = Pp[BS[n0 / kSphTPB]];
+        if (n0 >= P.poff + (unsigned)P.n)
+            continue;
         f32x4 acc[4];
         for (int t = 0; t < 4; t++)
             acc[t] = {0, 0, 0, 0};
-        float dg = 0.0f, rh = 0.0f;
-        if (n0 < P.poff + (unsigned)P.n) {
-            auto tiles = [&](unsigned ne) {
-                for (unsigned e0 = 0; e0 < ne; e0 += 16) {
-                    const bf16x4 a = edge_tile_a(L, e0);
-                    const bf16x4 mem = member_a(L, e0);
-                    for (int t = 0; t < 4; t++) {
-                        f32x4 d = {0, 0, 0, 0};
-                        d = mfma(a, B[t], d);
-                        // D layout (edge 4*sub+q, unit 16t+p) is the B layout of the sum
-                        acc[t] = mfma(mem, pack4(silu(d[0]), silu(d[1]), silu(d[2]), silu(d[3])),
-                                      acc[t]);
-                    }
-                }
-            };
-            walk_group<DENS>(n0, P, POS, VEL, K, start, L, tiles, dg, rh);
-        }
+        const float dg = walk_group(n0, P, POS, VEL, K, start, L,
+                                    [&](unsigned ne) { edge_sums(L, ne, B, acc); });
         for (int t = 0; t < 4; t++)
-            for (int q = 0; q < 4; q++)
-                S[(size_t)(n0 + 4u * sub + q) * kH + 16u * t + p] = acc[t][q];
-        if (l < 16u) {
+            S[((size_t)g * 4u + t) * 64u + l] = pack4(acc[t]);
+        if (l < 16u)
             deg[n0 + l] = dg;
-            if (DENS)
-                rho[n0 + l] = rh;
-        }
-        __builtin_amdgcn_wave_barrier();
     }
 }
 
 namespace {
 
-// Node-pass state of one 16-particle tile held by one wavefront.
-struct NodeTile {
-    f32x4 pre3[4]; // D layout: row 4*(l/16)+q, unit 16t + l%16
-    float out[4][2];
-};
-
-// Node-layer weights staged in LDS once per workgroup: the B operands of
-// every tile's MFMAs are read from here as 8-byte rows.
+// Node-layer weights staged in LDS once per workgroup.  A lane reads 8-byte
+// pieces of row l%16 of a weight matrix; the rows are 4 shorts longer than the
+// matrix, so that a wave's reads fall on different banks.
+constexpr unsigned kS2 = kH + 4, kS3 = kKN + 4; // row strides
 struct NodeW {
-    unsigned short W2[kH * kH];
-    unsigned short W3[kH * kKN];
+    unsigned short W2[kH * kS2];
+    unsigned short W3[kH * kS3];
     float b2[kH], W4[2 * kH], b4[2];
 };
+// W2 and the first 64 columns of W3 with rows and columns exchanged.
+struct NodeWT {
+    unsigned short W2[kH * kS2];
+    unsigned short W3[kH * kS2];
+};
 
+// Ends without a barrier.
 __device__ void stage_node_weights(NodeW &sw, const unsigned short *W2b,
                                    const unsigned short *W3b, const float *params)
 {
     for (unsigned i = threadIdx.x; i < kH * kH / 4u; i += blockDim.x)
-        ((uint2 *)sw.W2)[i] = ((const uint2 *)W2b)[i];
+        *(uint2 *)&sw.W2[i / (kH / 4u) * kS2 + i % (kH / 4u) * 4u] = ((const uint2 *)W2b)[i];
     for (unsigned i = threadIdx.x; i < kH * kKN / 4u; i += blockDim.x)
-        ((uint2 *)sw.W3)[i] = ((const uint2 *)W3b)[i];
+        *(uint2 *)&sw.W3[i / (kKN / 4u) * kS3 + i % (kKN / 4u) * 4u] = ((const uint2 *)W3b)[i];
     for (unsigned i = threadIdx.x; i < kH; i += blockDim.x)
         sw.b2[i] = params[ob2 + i];
     for (unsigned i = threadIdx.x; i < 2u * kH; i += blockDim.x)
         sw.W4[i] = params[oW4 + i];
     if (threadIdx.x < 2u)
         sw.b4[threadIdx.x] = params[ob4 + threadIdx.x];
-    __syncthreads();
 }
 
-__device__ __forceinline__ bf16x4 lds_row4(const unsigned short *base)
+__device__ void stage_turned_weights(NodeWT &sw, const unsigned short *W2b,
+                                     const unsigned short *W3b)
 {
-    return *(const bf16x4 *)base;
-}
-
-// Build u = [m, feats, 1, 0..] for a tile in LDS (bf16 [16][80]) and run the
-// node forward.  Rows of invalid slots are zero.
-// A operands of a tile's S rows (row l%16, columns 16kc + 4(l/16) ..) from
-// the fp32 S array, and the degrees of rows 4(l/16) + q.
-__device__ __forceinline__ void load_s_tile(unsigned n0, unsigned vend, const float *S,
-                                            const float *deg, bf16x4 A[4], float degv[4])
-{
-    const unsigned l = lane();
-    const unsigned row = n0 + l % 16u;
-    for (int kc = 0; kc < 4; kc++) {
-        const unsigned k = 16u * kc + 4u * (l / 16u);
-        if (row < vend) {
-            const float4 sv = *(const float4 *)(S + (size_t)row * kH + k);
-            A[kc] = pack4(sv.x, sv.y, sv.z, sv.w);
-        } else {
-            A[kc] = pack4(0, 0, 0, 0);
-        }
-    }
-    for (int q = 0; q < 4; q++) {
-        const unsigned r = n0 + 4u * (l / 16u) + q;
-        degv[q] = r < vend ? deg[r] : 0.0f;
+    for (unsigned i = threadIdx.x; i < kH * kH; i += blockDim.x) {
+        const unsigned r = i / kH, c = i % kH;
+        sw.W2[c * kS2 + r] = W2b[r * kH + c];
+        sw.W3[c * kS2 + r] = W3b[r * kKN + c];
     }
 }
 
-__device__ __forceinline__ void node_forward(unsigned n0, const sph_dev_params &P,
-                                             unsigned long long clock, const float2 *VEL,
-                                             const bf16x4 A[4], const float degv[4],
-                                             const NodeW &sw, unsigned short (*ul)[kKN],
-                                             NodeTile &T)
+// A operand: row 16t + l%16, columns 16kc + 4*(l/16) .. +3.
+template <unsigned STRIDE>
+__device__ __forceinline__ bf16x4 weight_a(const unsigned short *W, int t, int kc)
 {
-    const unsigned l = lane();
-    const unsigned nvalid_end = P.poff + (unsigned)P.n;
-    const NodeCtx nc = node_ctx(P, clock);
-    // m = S W2^T + deg b2
+    return *(const bf16x4 *)(W + (16u * t + lane() % 16u) * STRIDE + 16u * kc +
+                             4u * (lane() / 16u));
+}
+
+// Four floats of units 16t + 4*(l/16) .. +3.
+__device__ __forceinline__ f32x4 unit4(const float *v, int t)
+{
+    return *(const f32x4 *)(v + 16u * t + 4u * (lane() / 16u));
+}
+
+// Node-pass state of one 16-particle group held by one wavefront: per lane
+// units 16t + 4*(l/16) .. +3 of particle l%16.
+struct NodeTile {
+    bf16x4 u[5];   // node input [m, 0.2 v, 0.1 a, 1, 0 ..]
+    f32x4 pre3[4];
+    float out[2];  // every lane of the particle
+};
+
+// The node forward from the edge sums S and degree of particle l%16 (velocity
+// v; not ok: no particle, all zero).
+__device__ __forceinline__ void node_forward(const bf16x4 S[4], float deg, bool ok, float2 v,
+                                             const NodeCtx &nc, const NodeW &sw, NodeTile &T)
+{
+    const unsigned sub = lane() / 16u;
+    // m = W2 S + deg b2
+#pragma unroll
     for (int t = 0; t < 4; t++) {
         f32x4 d = {0, 0, 0, 0};
-        for (int kc = 0; kc < 4; kc++) {
-            // B[k][c] = W2[16t + c][k]
-            const unsigned c = 16u * t + l % 16u, k = 16u * kc + 4u * (l / 16u);
-            d = mfma(A[kc], lds_row4(&sw.W2[c * kH + k]), d);
-        }
-        const float b2 = sw.b2[16u * t + l % 16u];
-        for (int q = 0; q < 4; q++) {
-            const unsigned r = 4u * (l / 16u) + q;
-            const unsigned row = n0 + r;
-            const float m = row < nvalid_end ? d[q] + degv[q] * b2 : 0.0f;
-            ul[r][16u * t + l % 16u] = f2bf(m);
-        }
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++)
+            d = mfma(weight_a<kS2>(sw.W2, t, kc), S[kc], d);
+        const f32x4 b2 = unit4(sw.b2, t);
+        T.u[t] = pack4(ok ? d[0] + deg * b2[0] : 0.0f, ok ? d[1] + deg * b2[1] : 0.0f,
+                       ok ? d[2] + deg * b2[2] : 0.0f, ok ? d[3] + deg * b2[3] : 0.0f);
     }
     // node features, bias column, padding
-    if (l < 16u) {
-        const unsigned row = n0 + l;
-        const bool ok = row < nvalid_end;
-        const float2 v = ok ? VEL[row] : make_float2(0, 0);
-        ul[l][64] = f2bf(v.x * kVScale);
-        ul[l][65] = f2bf(v.y * kVScale);
-        ul[l][66] = f2bf(ok ? nc.fx * kAScale : 0.0f);
-        ul[l][67] = f2bf(ok ? nc.g_neg * kAScale : 0.0f);
-        ul[l][68] = f2bf(ok ? 1.0f : 0.0f);
-        for (int q = 69; q < kKN; q++)
-            ul[l][q] = 0;
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    // pre3 = u W3^T
-    bf16x4 Au[5];
-    for (int kc = 0; kc < 5; kc++) {
-        const unsigned k = 16u * kc + 4u * (l / 16u);
-        for (int q = 0; q < 4; q++)
-            Au[kc][q] = (short)ul[l % 16u][k + q];
-    }
+    const bool f0 = ok && sub == 0u;
+    T.u[4] = pack4(f0 ? v.x * kVScale : ok && sub == 1u ? 1.0f : 0.0f, f0 ? v.y * kVScale : 0.0f,
+                   f0 ? nc.fx * kAScale : 0.0f, f0 ? nc.g_neg * kAScale : 0.0f);
+    // pre3 = W3 u; out = W4 SiLU(pre3) + b4
+    float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
     for (int t = 0; t < 4; t++) {
         f32x4 d = {0, 0, 0, 0};
-        for (int kc = 0; kc < 5; kc++) {
-            // B[k][c] = W3[16t + c][k]
-            const unsigned c = 16u * t + l % 16u, k = 16u * kc + 4u * (l / 16u);
-            d = mfma(Au[kc], lds_row4(&sw.W3[c * kKN + k]), d);
-        }
+#pragma unroll
+        for (int kc = 0; kc < 5; kc++)
+            d = mfma(weight_a<kS3>(sw.W3, t, kc), T.u[kc], d);
         T.pre3[t] = d;
-    }
-    // out = W4 SiLU(pre3) + b4, reduced over the 16 lanes of each row group
-    for (int q = 0; q < 4; q++)
-        for (int o = 0; o < 2; o++) {
-            float p = 0.0f;
-            for (int t = 0; t < 4; t++)
-                p += silu(T.pre3[t][q]) * sw.W4[o * kH + 16u * t + l % 16u];
-            for (int x = 1; x < 16; x <<= 1)
-                p += __shfl_xor(p, x, 64);
-            T.out[q][o] = p + sw.b4[o];
+        const f32x4 w0 = unit4(sw.W4, t), w1 = unit4(sw.W4 + kH, t);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float z = silu(d[q]);
+            o0 += z * w0[q];
+            o1 += z * w1[q];
         }
+    }
+    o0 += __shfl_xor(o0, 16, 64);
+    o1 += __shfl_xor(o1, 16, 64);
+    o0 += __shfl_xor(o0, 32, 64);
+    o1 += __shfl_xor(o1, 32, 64);
+    T.out[0] = o0 + sw.b4[0];
+    T.out[1] = o1 + sw.b4[1];
 }
 
 __device__ __forceinline__ float2 ballistic(const NodeCtx &nc, float2 v)
@@ -513,19 +546,14 @@ __device__ __forceinline__ float2 ballistic(const NodeCtx &nc, float2 v)
 } // namespace
 
 // Inference: the edge pass and the node MLP of each 16-slot group in one
-// kernel (the group is one node tile).  S and deg stay on chip: the edge
-// pass's per-particle sums are transposed through LDS into the node MLP's A
-// operands, in the LDS the edge buffer used.
-union InferLds {
-    EdgeBuf e;
-    struct {
-        unsigned short ul[16][kKN];
-        unsigned short sS[16][kH];
-        float deg[16];
-    } n;
-};
-
-__global__ void __launch_bounds__(256)
+// kernel; everything between the edge list and the displacement stays in
+// registers.  Bound by VALU issue, of which the edges' SiLUs are the largest
+// part; 64 scenes of 16,384 particles (17 neighbours each) take 0.49 ms, 0.82
+// with the layers' values turned through LDS (weight rows on the same banks,
+// 32 lane permutes for the output layer), half-width conversions, the MFMA
+// results in accumulation registers, two dependent global loads a round, and
+// eight groups a wave.
+__global__ void __launch_bounds__(256, 3)
 k_infer(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned slots,
         const unsigned long long *__restrict__ clock, const float2 *__restrict__ POS,
         const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
@@ -533,11 +561,12 @@ k_infer(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsig
         const unsigned short *__restrict__ W2b, const float *__restrict__ params,
         const unsigned short *__restrict__ W3b, float2 *__restrict__ disp)
 {
-    __shared__ __align__(16) InferLds Lb[4];
+    __shared__ __align__(16) EdgeBuf Lb[4];
     __shared__ __align__(16) NodeW sw;
     stage_node_weights(sw, W2b, W3b, params);
-    const unsigned w = threadIdx.x / 64u, l = lane(), p = l % 16u, sub = l / 16u;
-    InferLds &L = Lb[w];
+    __syncthreads();
+    const unsigned w = wave_index(), l = lane(), p = l % 16u;
+    EdgeBuf &L = Lb[w];
     bf16x4 B[4];
     for (int t = 0; t < 4; t++)
         B[t] = w1_b(W1b, t);
@@ -545,350 +574,300 @@ k_infer(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsig
     const unsigned long long ck = *clock;
     for (unsigned g = blockIdx.x * 4u + w; g < ngroups; g += nw) {
         const unsigned n0 = g * kGroup;
-        const sph_dev_params &P = Pp[BS[n0 / kSphTPB]];
+        const sph_dev_params P = Pp[BS[n0 / kSphTPB]];
         const unsigned vend = P.poff + (unsigned)P.n;
         if (n0 >= vend)
             continue;
         f32x4 acc[4];
         for (int t = 0; t < 4; t++)
             acc[t] = {0, 0, 0, 0};
-        float dg = 0.0f, rh = 0.0f;
-        auto tiles = [&](unsigned ne) {
-            for (unsigned e0 = 0; e0 < ne; e0 += 16) {
-                const bf16x4 a = edge_tile_a(L.e, e0);
-                const bf16x4 mem = member_a(L.e, e0);
-                for (int t = 0; t < 4; t++) {
-                    f32x4 d = {0, 0, 0, 0};
-                    d = mfma(a, B[t], d);
-                    acc[t] = mfma(mem, pack4(silu(d[0]), silu(d[1]), silu(d[2]), silu(d[3])),
-                                  acc[t]);
-                }
-            }
-        };
-        walk_group<false>(n0, P, POS, VEL, K, start, L.e, tiles, dg, rh);
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        // S tile (rows 4*sub+q, units 16t+p) -> LDS, transposed on read below
+        const float dg = walk_group(n0, P, POS, VEL, K, start, L,
+                                    [&](unsigned ne) { edge_sums(L, ne, B, acc); });
+        bf16x4 S[4];
         for (int t = 0; t < 4; t++)
-            for (int q = 0; q < 4; q++)
-                L.n.sS[4u * sub + q][16u * t + p] = f2bf(acc[t][q]);
-        if (l < 16u)
-            L.n.deg[l] = dg;
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        bf16x4 A[4];
-        for (int kc = 0; kc < 4; kc++)
-            A[kc] = lds_row4(&L.n.sS[p][16u * kc + 4u * sub]);
-        float degv[4];
-        for (int q = 0; q < 4; q++)
-            degv[q] = L.n.deg[4u * sub + q];
-        NodeTile T;
-        node_forward(n0, P, ck, VEL, A, degv, sw, L.n.ul, T);
+            S[t] = pack4(acc[t]);
+        const bool ok = n0 + p < vend;
+        const float2 v = ok ? VEL[n0 + p] : make_float2(0, 0);
         const NodeCtx nc = node_ctx(P, ck);
-        if (p == 0)
-            for (int q = 0; q < 4; q++) {
-                const unsigned row = n0 + 4u * sub + q;
-                if (row < vend) {
-                    const float2 b = ballistic(nc, VEL[row]);
-                    disp[row] = make_float2(b.x + kDScale * T.out[q][0],
-                                            b.y + kDScale * T.out[q][1]);
-                }
-            }
-        __builtin_amdgcn_wave_barrier();
+        NodeTile T;
+        node_forward(S, dg, ok, v, nc, sw, T);
+        if (l < 16u && ok) {
+            const float2 b = ballistic(nc, v);
+            disp[n0 + p] = make_float2(b.x + kDScale * T.out[0], b.y + kDScale * T.out[1]);
+        }
     }
 }
 
-// Node backward: loss, dout, dW4/db4 (+ atomics), and per particle dS (fp32),
-// dPre3, dM, U (tile-major bf16 [tile][col][16]) for the weight-gradient
-// reduction.  tgt holds the target displacement per slot.
-__global__ void __launch_bounds__(256)
-k_node_bwd(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned slots,
-           const unsigned long long *__restrict__ clock, const float2 *__restrict__ VEL,
-           const float *__restrict__ S, const float *__restrict__ deg,
-           const unsigned short *__restrict__ W2b, const float *__restrict__ params,
-           const unsigned short *__restrict__ W3b, const float2 *__restrict__ tgt, float inv_n,
-           float *__restrict__ dS, unsigned short *__restrict__ U,
-           unsigned short *__restrict__ dP3, unsigned short *__restrict__ dM,
-           float *__restrict__ grads, float *__restrict__ loss)
+// Node backward: loss, and the gradients of W2, b2, W3, W4, b4 and of the edge
+// sums.  One wavefront per group runs the node forward again and the layers
+// back, all in registers; the weight gradients dW3 (64x80) = sum dPre3^T U and
+// dW2 (64x64) = sum dM^T S sum over particles, so each wave leaves its group's
+// four factors, turned, in LDS, and then takes 9 of the 36 output tiles over
+// the workgroup's four groups.  (With the factors written to memory, 350 bytes
+// a particle, and a second kernel for the products: 0.84 ms for a million
+// particles, 0.18 now.)  tgt holds the target displacement per slot.
+constexpr int kFactors = 4 + 5 + 4 + 4; // dPre3, U, dM, S tiles of a group
+constexpr unsigned kNodeTiles = 36 * 256;    // partial dW3 and dW2 of a workgroup, by tile and lane
+constexpr unsigned kNodeRest = 3 * kH + 4;   // dW4 (two rows), db2, db4, loss, 0
+constexpr unsigned kNodePart = kNodeTiles + kNodeRest;
+__global__ void __launch_bounds__(256, 2)
+k_node_grad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned slots,
+            const unsigned long long *__restrict__ clock, const float2 *__restrict__ VEL,
+            const bf16x4 *__restrict__ S, const float *__restrict__ deg,
+            const unsigned short *__restrict__ W2b, const float *__restrict__ params,
+            const unsigned short *__restrict__ W3b, const float2 *__restrict__ tgt, float inv_n,
+            bf16x4 *__restrict__ dS, float *__restrict__ part)
 {
-    __shared__ unsigned short ul[4][16][kKN];
-    __shared__ unsigned short dl[4][16][kH];
-    __shared__ float du_l[4][16][kH];
     __shared__ __align__(16) NodeW sw;
+    __shared__ __align__(16) NodeWT st;
+    __shared__ bf16x4 fac[4][kFactors][64];
     stage_node_weights(sw, W2b, W3b, params);
-    const unsigned w = threadIdx.x / 64u, l = lane();
-    const unsigned ntiles = slots / 16u, nw = gridDim.x * 4u;
+    stage_turned_weights(st, W2b, W3b);
+    __syncthreads();
+    const unsigned w = wave_index(), l = lane(), p = l % 16u, sub = l / 16u;
+    const unsigned ngroups = slots / kGroup; // a multiple of 16
     const unsigned long long ck = *clock;
-    float gW4[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-    float gb4[2] = {0, 0}, gb2[4] = {0, 0, 0, 0}, lsum = 0.0f;
-    for (unsigned tile = blockIdx.x * 4u + w; tile < ntiles; tile += nw) {
-        const unsigned n0 = tile * 16u;
-        const sph_dev_params &P = Pp[BS[n0 / kSphTPB]];
-        const unsigned vend = P.poff + (unsigned)P.n;
-        unsigned short *Ut = U + (size_t)tile * kKN * 16u;
-        unsigned short *Pt = dP3 + (size_t)tile * kH * 16u;
-        unsigned short *Mt = dM + (size_t)tile * kH * 16u;
-        if (n0 >= vend) { // padding tile: zero operands for the reduction
-            for (unsigned x = l; x < kKN * 16u; x += 64)
-                Ut[x] = 0;
-            for (unsigned x = l; x < kH * 16u; x += 64) {
-                Pt[x] = 0;
-                Mt[x] = 0;
-            }
-            continue;
-        }
-        NodeTile T;
-        bf16x4 A[4];
-        float degv[4];
-        load_s_tile(n0, vend, S, deg, A, degv);
-        node_forward(n0, P, ck, VEL, A, degv, sw, ul[w], T);
-        const NodeCtx nc = node_ctx(P, ck);
-        // dout for the 4 rows of this lane group
-        float dout[4][2];
-        for (int q = 0; q < 4; q++) {
-            const unsigned row = n0 + 4u * (l / 16u) + q;
-            const bool ok = row < vend;
-            float2 pred = make_float2(0, 0), y = make_float2(0, 0);
-            if (ok) {
-                const float2 b = ballistic(nc, VEL[row]);
-                pred = make_float2(b.x + kDScale * T.out[q][0], b.y + kDScale * T.out[q][1]);
-                y = tgt[row];
-            }
-            // loss = mean over particles of |d - y|^2 / kDScale^2
-            const float ex = (pred.x - y.x) / kDScale, ey = (pred.y - y.y) / kDScale;
-            dout[q][0] = ok ? 2.0f * ex * inv_n : 0.0f;
-            dout[q][1] = ok ? 2.0f * ey * inv_n : 0.0f;
-            if (ok && l % 16u == 0)
-                lsum += (ex * ex + ey * ey) * inv_n;
-        }
-        // dW4, db4, dz, dpre3
-        for (int t = 0; t < 4; t++) {
-            const unsigned c = 16u * t + l % 16u;
-            for (int q = 0; q < 4; q++) {
-                const float x = T.pre3[t][q];
-                const float z = silu(x);
-                gW4[0][t] += dout[q][0] * z;
-                gW4[1][t] += dout[q][1] * z;
-                const float dz = dout[q][0] * sw.W4[c] + dout[q][1] * sw.W4[kH + c];
-                const float dp = dz * silu_grad(x);
-                dl[w][4u * (l / 16u) + q][c] = f2bf(dp);
-            }
-            // tile-major dPre3: [unit][16 rows]
-            bf16x4 v;
-            for (int q = 0; q < 4; q++)
-                v[q] = (short)dl[w][4u * (l / 16u) + q][c];
-            *(bf16x4 *)(Pt + (size_t)c * 16u + 4u * (l / 16u)) = v;
-        }
-        if (l % 16u == 0)
-            for (int q = 0; q < 4; q++) {
-                gb4[0] += dout[q][0];
-                gb4[1] += dout[q][1];
-            }
-        // U tile-major [col][16 rows]
-        for (unsigned x = l; x < kKN * 4u; x += 64) {
-            const unsigned col = x / 4u, r0 = 4u * (x % 4u);
-            bf16x4 v;
-            for (int q = 0; q < 4; q++)
-                v[q] = (short)ul[w][r0 + q][col];
-            *(bf16x4 *)(Ut + (size_t)col * 16u + r0) = v;
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        // du = dpre3 W3  (16 x 80); only the first 64 columns (dm) are needed
-        bf16x4 Ad[4];
-        for (int kc = 0; kc < 4; kc++)
-            for (int q = 0; q < 4; q++)
-                Ad[kc][q] = (short)dl[w][l % 16u][16u * kc + 4u * (l / 16u) + q];
-        for (int t = 0; t < 4; t++) {
-            f32x4 d = {0, 0, 0, 0};
-            for (int kc = 0; kc < 4; kc++) {
-                bf16x4 b; // B[k][c] = W3[k][16t + c]  (k: hidden unit)
-                const unsigned c = 16u * t + l % 16u, k = 16u * kc + 4u * (l / 16u);
-                for (int q = 0; q < 4; q++)
-                    b[q] = (short)sw.W3[(k + q) * kKN + c];
-                d = mfma(Ad[kc], b, d);
-            }
-            for (int q = 0; q < 4; q++) {
-                const unsigned r = 4u * (l / 16u) + q;
-                du_l[w][r][16u * t + l % 16u] = n0 + r < vend ? d[q] : 0.0f;
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        // dM tile-major, db2 partials, dS = dm W2
-        for (int t = 0; t < 4; t++) {
-            const unsigned c = 16u * t + l % 16u;
-            bf16x4 v;
-            for (int q = 0; q < 4; q++) {
-                const unsigned r = 4u * (l / 16u) + q;
-                const float dm = du_l[w][r][c];
-                v[q] = (short)f2bf(dm);
-                if (n0 + r < vend)
-                    gb2[t] += deg[n0 + r] * dm;
-            }
-            *(bf16x4 *)(Mt + (size_t)c * 16u + 4u * (l / 16u)) = v;
-        }
-        bf16x4 Am[4];
-        for (int kc = 0; kc < 4; kc++)
-            for (int q = 0; q < 4; q++)
-                Am[kc][q] = (short)f2bf(du_l[w][l % 16u][16u * kc + 4u * (l / 16u) + q]);
-        for (int t = 0; t < 4; t++) {
-            f32x4 d = {0, 0, 0, 0};
-            for (int kc = 0; kc < 4; kc++) {
-                bf16x4 b; // B[k][c] = W2[k][16t + c]  (k: output unit of layer 2)
-                const unsigned c = 16u * t + l % 16u, k = 16u * kc + 4u * (l / 16u);
-                for (int q = 0; q < 4; q++)
-                    b[q] = (short)sw.W2[(k + q) * kH + c];
-                d = mfma(Am[kc], b, d);
-            }
-            for (int q = 0; q < 4; q++) { // rows past the scene's end get 0
-                const unsigned row = n0 + 4u * (l / 16u) + q;
-                dS[(size_t)row * kH + 16u * t + l % 16u] = d[q];
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    // dW4 partials: sum over the 4 row groups
-    for (int o = 0; o < 2; o++)
-        for (int t = 0; t < 4; t++) {
-            float v = gW4[o][t];
-            v += __shfl_xor(v, 16, 64);
-            v += __shfl_xor(v, 32, 64);
-            if (l < 16u)
-                atomicAdd(&grads[oW4 + o * kH + 16u * t + l], v);
-        }
-    for (int t = 0; t < 4; t++) {
-        float v = gb2[t];
-        v += __shfl_xor(v, 16, 64);
-        v += __shfl_xor(v, 32, 64);
-        if (l < 16u)
-            atomicAdd(&grads[ob2 + 16u * t + l], v);
-    }
-    if (l % 16u == 0) {
-        atomicAdd(&grads[ob4], gb4[0]);
-        atomicAdd(&grads[ob4 + 1], gb4[1]);
-        atomicAdd(loss, lsum);
-    }
-}
-
-// Weight gradients of the node layers by split-K MFMA over particle tiles:
-// dW3 (64x80) = sum dPre3^T U, dW2 (64x64) = sum dM^T S.  36 output tiles
-// of 16x16; wave w of a workgroup owns output tiles w, w+4, ...
-__global__ void __launch_bounds__(256)
-k_node_wgrad(unsigned ntiles, const unsigned short *__restrict__ U,
-             const unsigned short *__restrict__ dP3, const unsigned short *__restrict__ dM,
-             const float *__restrict__ S, float *__restrict__ grads)
-{
-    const unsigned w = threadIdx.x / 64u, l = lane();
-    f32x4 acc[9];
+    const bf16x4 eye = identity_b();
+    const f32x4 zero = {0, 0, 0, 0};
+    f32x4 gW[9]; // output tiles w, w + 4, ...: the first 20 of dW3, the others of dW2
+    f32x4 gW4[2][4], gb2[4];
     for (int i = 0; i < 9; i++)
-        acc[i] = {0, 0, 0, 0};
-    for (unsigned tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const unsigned short *Ut = U + (size_t)tile * kKN * 16u;
-        const unsigned short *Pt = dP3 + (size_t)tile * kH * 16u;
-        const unsigned short *Mt = dM + (size_t)tile * kH * 16u;
+        gW[i] = zero;
+    for (int t = 0; t < 4; t++)
+        gW4[0][t] = gW4[1][t] = gb2[t] = zero;
+    float gb4[2] = {0, 0}, lsum = 0.0f;
+    for (unsigned g0 = blockIdx.x * 4u; g0 < ngroups; g0 += gridDim.x * 4u) {
+        const unsigned g = g0 + w, n0 = g * kGroup;
+        const sph_dev_params P = Pp[BS[n0 / kSphTPB]];
+        const unsigned vend = P.poff + (unsigned)P.n;
+        const bool any = n0 < vend, ok = n0 + p < vend; // no particles: all factors zero
+        bf16x4 Sb[4];
+        for (int t = 0; t < 4; t++)
+            Sb[t] = any ? S[((size_t)g * 4u + t) * 64u + l] : pack4(zero);
+        const float dg = ok ? deg[n0 + p] : 0.0f;
+        const float2 v = ok ? VEL[n0 + p] : make_float2(0, 0);
+        const float2 y = ok ? tgt[n0 + p] : make_float2(0, 0);
+        const NodeCtx nc = node_ctx(P, ck);
+        NodeTile T;
+        node_forward(Sb, dg, ok, v, nc, sw, T);
+        // loss = mean over particles of |d - y|^2 / kDScale^2
+        const float2 b = ballistic(nc, v);
+        const float ex = (b.x + kDScale * T.out[0] - y.x) / kDScale;
+        const float ey = (b.y + kDScale * T.out[1] - y.y) / kDScale;
+        const float dout0 = ok ? 2.0f * ex * inv_n : 0.0f, dout1 = ok ? 2.0f * ey * inv_n : 0.0f;
+        if (ok && sub == 0u) {
+            lsum += (ex * ex + ey * ey) * inv_n;
+            gb4[0] += dout0;
+            gb4[1] += dout1;
+        }
+        // dW4, dPre3
+        bf16x4 dP[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const f32x4 w0 = unit4(sw.W4, t), w1 = unit4(sw.W4 + kH, t);
+            float dp[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float x = T.pre3[t][q], s = sigm(x);
+                gW4[0][t][q] += dout0 * (x * s);
+                gW4[1][t][q] += dout1 * (x * s);
+                dp[q] = (dout0 * w0[q] + dout1 * w1[q]) * (s * (1.0f + x * (1.0f - s)));
+            }
+            dP[t] = pack4(dp[0], dp[1], dp[2], dp[3]);
+        }
+        // dm = W3^T dPre3 (the first 64 inputs), db2; dS = W2^T dm
+        bf16x4 dM[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            f32x4 d = zero;
+#pragma unroll
+            for (int kc = 0; kc < 4; kc++)
+                d = mfma(weight_a<kS2>(st.W3, t, kc), dP[kc], d);
+            for (int q = 0; q < 4; q++)
+                gb2[t][q] += dg * d[q];
+            dM[t] = pack4(d);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            f32x4 d = zero;
+#pragma unroll
+            for (int kc = 0; kc < 4; kc++)
+                d = mfma(weight_a<kS2>(st.W2, t, kc), dM[kc], d);
+            if (any)
+                dS[((size_t)g * 4u + t) * 64u + l] = turn(pack4(d), eye);
+        }
+        // the factors of the weight gradients, units as rows
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            fac[w][t][l] = turn(dP[t], eye);
+            fac[w][9 + t][l] = turn(dM[t], eye);
+            fac[w][13 + t][l] = turn(Sb[t], eye);
+        }
+#pragma unroll
+        for (int t = 0; t < 5; t++)
+            fac[w][4 + t][l] = turn(T.u[t], eye);
+        __syncthreads();
+#pragma unroll
         for (int i = 0; i < 9; i++) {
             const unsigned ot = w + 4u * i; // 0..35
-            const unsigned mt = ot < 20u ? ot / 5u : (ot - 20u) / 4u;
-            const unsigned nt = ot < 20u ? ot % 5u : (ot - 20u) % 4u;
-            // A[r][k] = dX[node k][unit 16mt + r]; B[k][c] = Y[node k][col 16nt + c]
-            const unsigned short *Ab = ot < 20u ? Pt : Mt;
-            const bf16x4 a = *(const bf16x4 *)(Ab + (size_t)(16u * mt + l % 16u) * 16u + 4u * (l / 16u));
-            bf16x4 b;
-            if (ot < 20u) {
-                b = *(const bf16x4 *)(Ut + (size_t)(16u * nt + l % 16u) * 16u + 4u * (l / 16u));
-            } else {
-                const unsigned col = 16u * nt + l % 16u;
-                const size_t n = (size_t)tile * 16u + 4u * (l / 16u);
-                b = pack4(S[n * kH + col], S[(n + 1) * kH + col], S[(n + 2) * kH + col],
-                          S[(n + 3) * kH + col]);
-            }
-            acc[i] = mfma(a, b, acc[i]);
+            const bool w3 = i < 5;          // ot < 20
+            const unsigned fa = w3 ? ot / 5u : 9u + (ot - 20u) / 4u;
+            const unsigned fb = w3 ? 4u + ot % 5u : 13u + (ot - 20u) % 4u;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                gW[i] = mfma(fac[k][fa][l], fac[k][fb][l], gW[i]);
         }
+        __syncthreads(); // the next groups' factors overwrite these
     }
-    for (int i = 0; i < 9; i++) {
-        const unsigned ot = w + 4u * i;
-        const unsigned mt = ot < 20u ? ot / 5u : (ot - 20u) / 4u;
-        const unsigned nt = ot < 20u ? ot % 5u : (ot - 20u) % 4u;
+    // this workgroup's partial gradients, to be summed by k_grad_sum
+    float *out = part + (size_t)blockIdx.x * kNodePart;
+#pragma unroll
+    for (int i = 0; i < 9; i++)
+        *(f32x4 *)&out[((w + 4u * i) * 64u + l) * 4u] = gW[i];
+    // sums over the 16 particles of a row of lanes, then over the waves
+    auto over_particles = [](float v) {
+        for (int x = 1; x < 16; x <<= 1)
+            v += __shfl_xor(v, x, 64);
+        return v;
+    };
+    float(*rest)[kNodeRest] = (float(*)[kNodeRest]) & fac[0][0][0];
+    for (int t = 0; t < 4; t++)
         for (int q = 0; q < 4; q++) {
-            const unsigned r = 16u * mt + 4u * (l / 16u) + q, c = 16u * nt + l % 16u;
-            if (ot < 20u)
-                atomicAdd(&grads[oW3 + r * kKN + c], acc[i][q]);
-            else
-                atomicAdd(&grads[oW2 + r * kH + c], acc[i][q]);
+            const float a = over_particles(gW4[0][t][q]), c = over_particles(gW4[1][t][q]);
+            const float d = over_particles(gb2[t][q]);
+            if (p == 0u) {
+                const unsigned unit = 16u * t + 4u * sub + q;
+                rest[w][unit] = a;
+                rest[w][kH + unit] = c;
+                rest[w][2u * kH + unit] = d;
+            }
         }
-    }
+    const float b0 = over_particles(gb4[0]), b1 = over_particles(gb4[1]);
+    const float ls = over_particles(lsum);
+    if (l < 4u)
+        rest[w][3u * kH + l] = l == 0u ? b0 : l == 1u ? b1 : l == 2u ? ls : 0.0f;
+    __syncthreads();
+    for (unsigned i = threadIdx.x; i < kNodeRest; i += blockDim.x)
+        out[kNodeTiles + i] = (rest[0][i] + rest[1][i]) + (rest[2][i] + rest[3][i]);
 }
 
 // Edge backward: dW1 += sum over edges of (dS_i * SiLU'(W1 f_ij)) f_ij^T.
 // Same groups and tiles as the forward; dS_i is expanded to the tile's edges
 // by an MFMA of the one-hot edge->particle matrix with the group's dS, whose
 // D layout equals that of the recomputed pre-activations, and the product
-// with SiLU' is, in that layout, the A operand of dW1 += dPre1^T F.
-__global__ void __launch_bounds__(256)
+// with SiLU' is, in that layout, the A operand of dW1 += dPre1^T F.  The waves
+// of a workgroup add their dW1 in LDS and leave it as a partial gradient.  A
+// million particles: 0.96 -> 0.57 ms.
+constexpr unsigned kEdgePart = kH * 6; // partial dW1 of a workgroup
+__global__ void __launch_bounds__(256, 4)
 k_edge_bwd(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned slots,
            const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
            const unsigned *__restrict__ K, const unsigned *__restrict__ start,
-           const unsigned short *__restrict__ W1b, const float *__restrict__ dS,
-           float *__restrict__ grads)
+           const unsigned short *__restrict__ W1b, const bf16x4 *__restrict__ dS,
+           float *__restrict__ part)
 {
-    __shared__ EdgeBuf Lb[4];
-    const unsigned w = threadIdx.x / 64u, l = lane(), p = l % 16u, sub = l / 16u;
+    __shared__ __align__(16) EdgeBuf Lb[4];
+    __shared__ float gl[4][kEdgePart];
+    const unsigned w = wave_index(), l = lane(), p = l % 16u, sub = l / 16u;
     EdgeBuf &L = Lb[w];
     bf16x4 B[4];
     for (int t = 0; t < 4; t++)
         B[t] = w1_b(W1b, t);
+    const bf16x4 eye = identity_b();
+    const f32x4 zero = {0, 0, 0, 0};
     f32x4 g[4];
     for (int t = 0; t < 4; t++)
-        g[t] = {0, 0, 0, 0};
+        g[t] = zero;
     const unsigned ngroups = slots / kGroup, nw = gridDim.x * 4u;
     for (unsigned gi = blockIdx.x * 4u + w; gi < ngroups; gi += nw) {
         const unsigned n0 = gi * kGroup;
-        const sph_dev_params &P = Pp[BS[n0 / kSphTPB]];
+        const sph_dev_params P = Pp[BS[n0 / kSphTPB]];
         if (n0 >= P.poff + (unsigned)P.n)
             continue;
-        // B operand of the expansion: dS[particle 4*sub+i][unit 16t+p]
-        bf16x4 Bds[4];
-        for (int t = 0; t < 4; t++) {
-            const float *d0 = dS + (size_t)(n0 + 4u * sub) * kH + 16u * t + p;
-            Bds[t] = pack4(d0[0], d0[kH], d0[2 * kH], d0[3 * kH]);
-        }
+        bf16x4 Bds[4]; // B operand of the expansion: dS[particle 4*sub+i][unit 16t+p]
+        for (int t = 0; t < 4; t++)
+            Bds[t] = dS[((size_t)gi * 4u + t) * 64u + l];
         auto tiles = [&](unsigned ne) {
             for (unsigned e0 = 0; e0 < ne; e0 += 16) {
                 const bf16x4 a = edge_tile_a(L, e0);
-                // one-hot A: row edge e0 + p, columns particles 4*sub .. +3
-                bf16x4 oh;
-                const unsigned own = L.owner[e0 + p];
-                for (int q = 0; q < 4; q++)
-                    oh[q] = own == 4u * sub + q ? (short)0x3f80 : (short)0;
+                const bf16x4 oh = one_hot(L.owner[e0 + p]);
                 // B operand of the gradient product: F[edge 4*sub+i][feature p]
-                bf16x4 f;
-                for (int q = 0; q < 4; q++) {
-                    const bf16x4 fr = L.f[e0 + 4u * sub + q][(p / 4u) & 1u];
-                    f[q] = p < 8u ? fr[p % 4u] : (short)0;
-                }
+                const bf16x4 f = turn(a, eye);
+                f32x4 d[4], ds[4];
+#pragma unroll
                 for (int t = 0; t < 4; t++) {
-                    f32x4 d = {0, 0, 0, 0};
-                    d = mfma(a, B[t], d);
-                    f32x4 ds = {0, 0, 0, 0};
-                    ds = mfma(oh, Bds[t], ds);
+                    d[t] = mfma(a, B[t], zero);
+                    ds[t] = mfma(oh, Bds[t], zero);
+                }
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
                     float gp[4];
+#pragma unroll
                     for (int q = 0; q < 4; q++)
-                        gp[q] = ds[q] * silu_grad(d[q]);
+                        gp[q] = ds[t][q] * silu_grad(d[t][q]);
                     g[t] = mfma(pack4(gp[0], gp[1], gp[2], gp[3]), f, g[t]);
                 }
             }
         };
-        float dg, rh;
-        walk_group<false>(n0, P, POS, VEL, K, start, L, tiles, dg, rh);
-        __builtin_amdgcn_wave_barrier();
+        walk_group(n0, P, POS, VEL, K, start, L, tiles);
     }
     if (p < 6u)
         for (int t = 0; t < 4; t++)
-            for (int q = 0; q < 4; q++) {
-                const unsigned unit = 16u * t + 4u * sub + q;
-                atomicAdd(&grads[oW1 + unit * kKE + p], g[t][q]);
-            }
+            for (int q = 0; q < 4; q++)
+                gl[w][(16u * t + 4u * sub + q) * 6u + p] = g[t][q];
+    __syncthreads();
+    for (unsigned i = threadIdx.x; i < kEdgePart; i += blockDim.x)
+        part[(size_t)blockIdx.x * kEdgePart + i] =
+            (gl[0][i] + gl[1][i]) + (gl[2][i] + gl[3][i]);
+}
+
+// Sum the partial gradients of `rows` workgroups into grads (and the loss):
+// block (x, y) takes 64 columns of four and the rows of chunk y, 16 rows at a
+// time, and adds its sums.  A million particles' gradients by atomics straight
+// from the workgroups were 4.7 million of them on 9,600 addresses.
+template <bool NODE>
+__global__ void __launch_bounds__(1024)
+k_grad_sum(const float *__restrict__ part, unsigned rows, unsigned chunk,
+           float *__restrict__ grads, float *__restrict__ loss)
+{
+    constexpr unsigned kCols = NODE ? kNodePart : kEdgePart;
+    __shared__ f32x4 red[16][64];
+    const unsigned c = threadIdx.x % 64u, s = threadIdx.x / 64u;
+    const unsigned col = (blockIdx.x * 64u + c) * 4u;
+    const unsigned r1 = min(rows, (blockIdx.y + 1u) * chunk);
+    f32x4 v = {0, 0, 0, 0};
+    if (col < kCols)
+        for (unsigned r = blockIdx.y * chunk + s; r < r1; r += 16u)
+            v += *(const f32x4 *)&part[(size_t)r * kCols + col];
+    red[s][c] = v;
+    __syncthreads();
+    if (s != 0u || col >= kCols)
+        return;
+    for (unsigned k = 1; k < 16u; k++)
+        v += red[k][c];
+    for (unsigned q = 0; q < 4u; q++) {
+        const unsigned i = col + q;
+        if (!NODE) {
+            atomicAdd(&grads[oW1 + i / 6u * kKE + i % 6u], v[q]);
+        } else if (i < kNodeTiles) {
+            // tile i / 256, lane (i / 4) % 64, register q: the D layout
+            const unsigned ot = i / 256u, ln = i / 4u % 64u;
+            const unsigned mt = ot < 20u ? ot / 5u : (ot - 20u) / 4u;
+            const unsigned nt = ot < 20u ? ot % 5u : (ot - 20u) % 4u;
+            const unsigned r = 16u * mt + 4u * (ln / 16u) + q, k = 16u * nt + ln % 16u;
+            atomicAdd(&grads[ot < 20u ? oW3 + r * kKN + k : oW2 + r * kH + k], v[q]);
+        } else {
+            const unsigned k = i - kNodeTiles;
+            if (k < 2u * kH)
+                atomicAdd(&grads[oW4 + k], v[q]);
+            else if (k < 3u * kH)
+                atomicAdd(&grads[ob2 + k - 2u * kH], v[q]);
+            else if (k < 3u * kH + 2u)
+                atomicAdd(&grads[ob4 + k - 3u * kH], v[q]);
+            else if (k == 3u * kH + 2u)
+                atomicAdd(loss, v[q]);
+        }
+    }
 }
 
 // Adam on the fp32 master weights, then refresh the bf16 copies.  Weights
@@ -1166,27 +1145,56 @@ int malloc_dev(T **p, size_t n)
     return SPH_OK;
 }
 
+// Workgroups of the passes over groups of 16 slots, one group a wave: groups
+// differ in length, and workgroups that end leave their place to the next.
+// (2,048 workgroups taking eight groups a wave in turn: 0.56 ms for the edge
+// forward of a million particles, against 0.41.)
+unsigned group_blocks(unsigned slots) { return slots / (4u * kGroup); }
+
+// The node gradients keep their sums in registers and fit two workgroups per
+// CU (256 CUs).
+unsigned node_grad_blocks(unsigned slots)
+{
+    const unsigned n = group_blocks(slots);
+    return n < 512u ? n : 512u;
+}
+
+size_t part_floats(unsigned slots)
+{
+    const size_t a = (size_t)node_grad_blocks(slots) * kNodePart;
+    const size_t b = (size_t)group_blocks(slots) * kEdgePart;
+    return a > b ? a : b;
+}
+
+// Sum `rows` partial gradients in chunks of 128.
+template <bool NODE>
+void grad_sum(sph_surrogate *m, hipStream_t st, unsigned rows)
+{
+    constexpr unsigned kCols = NODE ? kNodePart : kEdgePart, kChunk = 128;
+    k_grad_sum<NODE><<<dim3((kCols + 255u) / 256u, (rows + kChunk - 1u) / kChunk), 1024, 0, st>>>(
+        m->part, rows, kChunk, m->grads, m->loss);
+}
+
 int ensure_buffers(sph_surrogate *m, size_t slots)
 {
     if (m->slots >= slots)
         return SPH_OK;
-    void *old[] = {m->S, m->deg, m->dS, m->disp, m->tgt, m->U, m->dP3, m->dM, m->tmp2};
+    void *old[] = {m->S, m->deg, m->dS, m->disp, m->tgt, m->tmp2, m->part};
     for (void *p : old)
         if (p)
             (void)hipFree(p);
-    m->S = m->deg = m->dS = m->disp = m->tgt = nullptr;
-    m->U = m->dP3 = m->dM = nullptr;
+    m->deg = m->disp = m->tgt = nullptr;
+    m->S = m->dS = nullptr;
     m->tmp2 = nullptr;
+    m->part = nullptr;
     int rc = SPH_OK;
-    if (!rc) rc = malloc_dev(&m->S, slots * kH);
+    if (!rc) rc = malloc_dev(&m->S, slots * kH / 4);
     if (!rc) rc = malloc_dev(&m->deg, slots);
-    if (!rc) rc = malloc_dev(&m->dS, slots * kH);
+    if (!rc) rc = malloc_dev(&m->dS, slots * kH / 4);
     if (!rc) rc = malloc_dev(&m->disp, slots * 2);
     if (!rc) rc = malloc_dev(&m->tgt, slots * 2);
-    if (!rc) rc = malloc_dev(&m->U, slots * kKN);
-    if (!rc) rc = malloc_dev(&m->dP3, slots * kH);
-    if (!rc) rc = malloc_dev(&m->dM, slots * kH);
     if (!rc) rc = malloc_dev(&m->tmp2, slots);
+    if (!rc) rc = malloc_dev(&m->part, part_floats((unsigned)slots));
     m->slots = rc ? 0 : slots;
     return rc;
 }
@@ -1243,9 +1251,9 @@ int forward(sph_surrogate *m, sph_ctx *c)
         return merr(SPH_ESTATE, "surrogate: the context has no hashed state (step or hash first)");
     if (int rc = ensure_buffers(m, c->slots))
         return rc;
-    k_infer<<<dim3(2048), 256, 0, c->st>>>(c->dP, c->BS, c->slots, c->dclock, c->POS0, c->VEL,
-                                           c->K0, c->start, m->W1b, m->W2b, m->params, m->W3b,
-                                           (float2 *)m->disp);
+    k_infer<<<dim3(group_blocks(c->slots)), 256, 0, c->st>>>(
+        c->dP, c->BS, c->slots, c->dclock, c->POS0, c->VEL, c->K0, c->start, m->W1b, m->W2b,
+        m->params, m->W3b, (float2 *)m->disp);
     MCHK(hipGetLastError());
     m->have_pred = true;
     return SPH_OK;
@@ -1259,9 +1267,8 @@ int forward_edges(sph_surrogate *m, sph_ctx *c)
         return merr(SPH_ESTATE, "surrogate: the context has no hashed state (step or hash first)");
     if (int rc = ensure_buffers(m, c->slots))
         return rc;
-    k_edge_fwd<false><<<dim3(2048), 256, 0, c->st>>>(c->dP, c->BS, c->slots, c->POS0, c->VEL,
-                                                     c->K0, c->start, m->W1b, m->S, m->deg,
-                                                     nullptr);
+    k_edge_fwd<<<dim3(group_blocks(c->slots)), 256, 0, c->st>>>(
+        c->dP, c->BS, c->slots, c->POS0, c->VEL, c->K0, c->start, m->W1b, m->S, m->deg);
     MCHK(hipGetLastError());
     return SPH_OK;
 }
@@ -1338,7 +1345,7 @@ void sph_surrogate_destroy(sph_surrogate *m)
     if (!m)
         return;
     void *ptrs[] = {m->params, m->grads, m->adam_m, m->adam_v, m->W1b, m->W2b, m->W3b, m->S,
-                    m->deg,    m->dS,    m->disp,   m->tgt,    m->U,   m->dP3, m->dM,  m->loss,
+                    m->deg,    m->dS,    m->disp,   m->tgt,    m->part,   m->loss,
                     m->tmp2, m->ref, m->jsum, m->jmax, m->jflags, m->sh_sum,
                     m->rho_plain, m->rho_sur, m->sh_err};
     for (void *p : ptrs)
@@ -1416,13 +1423,13 @@ static int backward_dev(sph_surrogate *m, sph_ctx *c, const float2 *target_dev, 
     k_by_id_to_slot<<<dim3(S / 256), 256, 0, c->st>>>(c->dP, c->BS, S, c->ID0, target_dev,
                                                      (float2 *)m->tgt);
     MCHK(hipMemsetAsync(m->loss, 0, sizeof(float), c->st));
-    k_node_bwd<<<dim3(2048), 256, 0, c->st>>>(c->dP, c->BS, S, c->dclock, c->VEL, m->S, m->deg,
-                                              m->W2b, m->params, m->W3b, (const float2 *)m->tgt,
-                                              1.0f / (float)c->n_total, m->dS, m->U, m->dP3,
-                                              m->dM, m->grads, m->loss);
-    k_node_wgrad<<<dim3(1024), 256, 0, c->st>>>(S / 16u, m->U, m->dP3, m->dM, m->S, m->grads);
-    k_edge_bwd<<<dim3(2048), 256, 0, c->st>>>(c->dP, c->BS, S, c->POS0, c->VEL, c->K0, c->start,
-                                              m->W1b, m->dS, m->grads);
+    k_node_grad<<<dim3(node_grad_blocks(S)), 256, 0, c->st>>>(
+        c->dP, c->BS, S, c->dclock, c->VEL, m->S, m->deg, m->W2b, m->params, m->W3b,
+        (const float2 *)m->tgt, 1.0f / (float)c->n_total, m->dS, m->part);
+    grad_sum<true>(m, c->st, node_grad_blocks(S));
+    k_edge_bwd<<<dim3(group_blocks(S)), 256, 0, c->st>>>(
+        c->dP, c->BS, S, c->POS0, c->VEL, c->K0, c->start, m->W1b, m->dS, m->part);
+    grad_sum<false>(m, c->st, group_blocks(S));
     MCHK(hipGetLastError());
     if (loss) {
         MCHK(hipMemcpyAsync(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost, c->st));
