@@ -253,9 +253,11 @@ int canonicalize(sph_ctx *c)
     sph_launch_pos_of_id(c->st, c->slots, c->dP, c->BS, c->ID0, c->pos_of_id);
     sph_reorder_fields<2> f{{c->PREV, c->RHO}, {c->T2a, c->T2b}};
     sph_launch_permute_by_id(c->st, c->slots, c->dP, c->BS, c->ID1, c->pos_of_id, f);
-    size_t b = sizeof(float2) * (size_t)c->slots;
-    HIPCHK(hipMemcpyAsync(c->PREV, c->T2a, b, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->RHO, c->T2b, b, hipMemcpyDeviceToDevice, c->st));
+    const size_t b = sizeof(float2) * (size_t)c->slots;
+    sph_copy_set cs;
+    cs.add(c->PREV, c->T2a, b);
+    cs.add(c->RHO, c->T2b, b);
+    sph_launch_copy(c->st, cs);
     HIPCHK(hipGetLastError());
     c->aux_order = 0;
     return SPH_OK;
@@ -857,11 +859,12 @@ int sph_phase_hash(sph_ctx *c, int compute_density)
     sph_launch_reorder4(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K1, f,
                         c->ID1, c->plans, c->dC);
     const size_t b = sizeof(float2) * (size_t)S;
+    sph_copy_set cs;
     for (int k = 0; k < 4; k++)
-        HIPCHK(hipMemcpyAsync((void *)f.src[k], f.dst[k], b, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->ID0, c->ID1, sizeof(int) * (size_t)S, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->K0, c->K1, sizeof(unsigned) * (size_t)S, hipMemcpyDeviceToDevice,
-                          c->st));
+        cs.add((void *)f.src[k], f.dst[k], b);
+    cs.add(c->ID0, c->ID1, b / 2);
+    cs.add(c->K0, c->K1, b / 2);
+    sph_launch_copy(c->st, cs);
     if (compute_density)
         sph_launch_density(c->st, S, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->K0, c->start,
                            c->RHO, c->MASK, c->dC, c->lanes);
@@ -916,23 +919,25 @@ int sph_snapshot_save(sph_ctx *c)
 #define A(p, count)                                                                              \
     if (!rc)                                                                                     \
     rc = dalloc(&c->p, count)
-        A(SPOS, N); A(SVEL, N); A(SPREV, N); A(SRHO, N); A(SID, N); A(SK, N); A(Sstart, M);
+        A(SPOS, N); A(SVEL, N); A(SPREV, N); A(SRHO, N); A(SID, N); A(SK, N); A(Sstart, M + 3);
         A(Sclock, 1); A(dflags, c->sc.size());
 #undef A
         if (rc)
             return rc;
     }
     const size_t b2 = sizeof(float2) * N, b1 = sizeof(unsigned) * N;
-    HIPCHK(hipMemcpyAsync(c->SPOS, c->POS0, b2, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->SVEL, c->VEL, b2, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->SPREV, c->PREV, b2, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->SRHO, c->RHO, b2, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->SID, c->ID0, b1, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->SK, c->K0, b1, hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->Sstart, c->start, sizeof(unsigned) * M, hipMemcpyDeviceToDevice,
-                          c->st));
-    HIPCHK(hipMemcpyAsync(c->Sclock, c->dclock, sizeof(unsigned long long),
-                          hipMemcpyDeviceToDevice, c->st));
+    sph_copy_set cs;
+    cs.add(c->SPOS, c->POS0, b2);
+    cs.add(c->SVEL, c->VEL, b2);
+    cs.add(c->SPREV, c->PREV, b2);
+    cs.add(c->SRHO, c->RHO, b2);
+    cs.add(c->SID, c->ID0, b1);
+    cs.add(c->SK, c->K0, b1);
+    cs.add(c->Sstart, c->start, sizeof(unsigned) * M);
+    cs.word_src = c->dclock;
+    cs.word_dst = c->Sclock;
+    sph_launch_copy(c->st, cs);
+    HIPCHK(hipGetLastError());
     c->snap_valid = true;
     c->snap_lists = c->lists_valid;
     return SPH_OK;

