@@ -258,13 +258,13 @@ int sph_set_scene_frozen(sph_ctx *ctx, const int *flags);
 int sph_set_bucket_cap(sph_ctx *ctx, int cap);
 
 /* Launch shape, with no counterpart in the reference: lanes per particle of
- * the fused step's gathers.  0 (the default) chooses by size - 4 when the
- * context has at most two 256-slot tiles per CU of the device (a scene of
- * up to 131,072 particles on 256 CUs), where a launch's time is set by its
- * slowest workgroups, else 1; 1 and 4 force a shape.  Results are bit
- * for bit the same either way: four lanes split a particle's candidate tests
- * and pair terms and apply the terms in the same order.  Any other value is
- * SPH_EINVAL. */
+ * the fused step's gathers.  0 (the default) chooses by size - 16 when the
+ * context has at most half a 256-slot tile per CU of the device (a scene of
+ * up to 32,768 particles on 256 CUs), 4 up to two (131,072), where a launch's
+ * time is set by its slowest workgroups, else 1; 1 and 4 force a shape.
+ * Results are bit for bit the same either way: the lanes split a particle's
+ * candidate tests and pair terms and apply the terms in the same order.  Any
+ * other value is SPH_EINVAL. */
 int sph_set_gather_lanes(sph_ctx *ctx, int lanes);
 /* Sloshing clock offset of one scene: its forcing is evaluated at
  * t = (steps since the last upload or load + steps) * dt, so a scene loaded

@@ -312,7 +312,7 @@ class Solver:
 
     def set_gather_lanes(self, lanes: int = 0):
         """Lanes per particle of the fused step's gathers: 0 chooses by size
-        (4 for small contexts), 1 or 4 force a shape; results are the same."""
+        (16 or 4 for small contexts), 1 or 4 force a shape; results are the same."""
         _check(lib().sph_set_gather_lanes(self._h, int(lanes)), "sph_set_gather_lanes")
 
     def set_scene_tunables(self, scene: int, t: Tunables):

@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 #include "../../include/sph_abi.h"
 
 // Step parameters of one scene as the kernels read them, derived on the
@@ -303,13 +305,12 @@ struct sph_visc_consts {
     float h_recip, dt, sigma, beta;
 };
 
-__device__ __forceinline__ float2 sph_visc_half(float px, float py, float pvx, float pvy, float qx,
-                                                float qy, float qvx, float qvy,
+// QmP: the pair's position difference, r2 its square (or, where the result is
+// not used, any common one).
+__device__ __forceinline__ float2 sph_visc_half(float QmP_x, float QmP_y, float r2, float pvx,
+                                                float pvy, float qvx, float qvy,
                                                 const sph_visc_consts &V, const sph_dev_params &P)
 {
-    const float QmP_x = qx - px;
-    const float QmP_y = qy - py;
-    const float r2 = QmP_x * QmP_x + QmP_y * QmP_y;
     const float along = (pvx - qvx) * QmP_x + (pvy - qvy) * QmP_y;
     const sph_root q = sph_root_common(r2);
     const float u = __builtin_fmaxf(along * q.rinv, 0.0f);
@@ -732,6 +733,105 @@ __device__ __forceinline__ uint2 sph_walk_rows(unsigned self, const sph_rows &R,
     }
     drain();
     return make_uint2(full, half);
+}
+
+// Sixteen lanes per particle (a DPP row of the wave holds one particle), for
+// contexts so small that a launch's time is its longest workgroup's: the
+// candidate rows are taken as one list, sixteen candidates a round, one a
+// lane, straight from memory (a round's records are loaded one round ahead;
+// no tile, no plan, no barrier), and every lane's term - zero where its
+// candidate is none or not within h - is then applied by all sixteen in list
+// order.  That is the canonical order, and a zero term leaves the sums
+// unchanged, so the sums are those of one lane per particle bit for bit.
+//
+// load(k): the record of sorted position k; pair(rec, cand, own, nudged): the
+// candidate's term and whether it was accepted (cand: it is a candidate);
+// apply(a, b) and nudge as in sph_split_body.  Returns this lane's share of the
+// (accepted, in the half list) counts.
+template <int N>
+__device__ __forceinline__ float sph_row_lane(float x)
+{
+    return __uint_as_float(sph_dpp<0x150 + N>(__float_as_uint(x))); // row_newbcast
+}
+
+template <bool NUDGE, class Apply, class Nudge, int... N>
+__device__ __forceinline__ void sph_apply_row(const sph_pair_term &t, bool nudged,
+                                              const Apply &apply, const Nudge &nudge,
+                                              std::integer_sequence<int, N...>)
+{
+    if constexpr (NUDGE)
+        ((nudge(sph_dpp<0x150 + N>(nudged ? 1u : 0u) != 0u),
+          apply(sph_pair_term{sph_row_lane<N>(t.a), sph_row_lane<N>(t.b)})),
+         ...);
+    else
+        (apply(sph_pair_term{sph_row_lane<N>(t.a), sph_row_lane<N>(t.b)}), ...);
+}
+
+template <bool CAP, class Load, class Pair, class Apply, class Nudge>
+__device__ __forceinline__ uint2 sph_walk_wide(unsigned self, bool live, const sph_rows &R,
+                                               unsigned cap, Load &&load, Pair &&pair,
+                                               Apply &&apply, Nudge &&nudge)
+{
+    using Seq = std::make_integer_sequence<int, 16>;
+    // the rows' bounds in values of their own: selects between members of R
+    // can be folded into a load from a selected address (scratch memory)
+    const unsigned p0 = R.b0[0], p1 = R.b0[1], p2 = R.b0[2];
+    const unsigned l0 = R.b1[0], l1 = R.b1[1], l2 = R.b1[2];
+    const unsigned u0 = R.b2[0], u1 = R.b2[1], u2 = R.b2[2];
+    const unsigned n0 = R.b3[0] - p0, n01 = n0 + (R.b3[1] - p1);
+    unsigned total = live ? n01 + (R.b3[2] - p2) : 0u;
+    if (CAP && self - l1 >= cap) // left out of its cell's bucket: walks nothing
+        total = 0;
+    auto position = [=](unsigned t) {
+        unsigned k = p0 + t;
+        k = t >= n0 ? p1 + (t - n0) : k;
+        k = t >= n01 ? p2 + (t - n01) : k;
+        return t < total ? k : self;
+    };
+    unsigned full = 0, half = 0;
+    unsigned t = __lane_id() & 15u, k = position(t);
+    auto rec = load(k);
+    while (__ballot(t < total) != 0ull) {
+        const unsigned kn = position(t + 16u);
+        const auto next = load(kn);
+        // the half list's owner threshold and, under the cap, the rank in the
+        // candidate's cell
+        const bool r1 = t >= n0, r2 = t >= n01;
+        unsigned thr = r1 ? self + 1u : u0;
+        thr = r2 ? l2 : thr;
+        bool cand = k != self;
+        if (CAP) {
+            unsigned c0 = r1 ? p1 : p0, c1 = r1 ? l1 : l0, c2 = r1 ? u1 : u0;
+            c0 = r2 ? p2 : c0;
+            c1 = r2 ? l2 : c1;
+            c2 = r2 ? u2 : c2;
+            c0 = k >= c1 ? c1 : c0;
+            c0 = k >= c2 ? c2 : c0;
+            cand = cand && k - c0 < cap;
+        }
+        bool accepted = false, nudged = false;
+        const sph_pair_term tm = pair(rec, cand, [&] { return k >= thr; }, accepted, nudged);
+        full += accepted ? 1u : 0u;
+        half += accepted && k >= thr ? 1u : 0u;
+        if (__builtin_expect(__ballot(nudged) == 0ull, 1))
+            sph_apply_row<false>(tm, false, apply, nudge, Seq{});
+        else
+            sph_apply_row<true>(tm, nudged, apply, nudge, Seq{});
+        t += 16u;
+        k = kn;
+        rec = next;
+    }
+    return make_uint2(full, half);
+}
+
+// A count over the sixteen lanes of a particle (all of them get it).
+__device__ __forceinline__ unsigned sph_row_sum(unsigned v)
+{
+    v += sph_dpp<0xB1>(v);  // quad_perm 1, 0, 3, 2
+    v += sph_dpp<0x4E>(v);  // quad_perm 2, 3, 0, 1
+    v += sph_dpp<0x141>(v); // row_half_mirror
+    v += sph_dpp<0x140>(v); // row_mirror
+    return v;
 }
 
 // All three candidate rows in one call.

@@ -20,13 +20,13 @@ struct sph_tile_plans {
 // Workgroup size of every particle kernel; scenes are padded to multiples.
 constexpr unsigned kSphTPB = 256;
 
-// Lanes per particle (1 or 4) of the gathers of a context with `slots`
+// Lanes per particle (1, 4 or 16) of the gathers of a context with `slots`
 // padded slots, on the current device.
 int sph_gather_lanes(unsigned slots);
 
 // cap: the reference's bucket cap is on (sph_dev_params::bucket_cap != 0).
-// lanes: lanes per particle of the gathers, 1 or 4 (sph_gather_lanes); 4
-// applies to the fused step's variants (grav, visc and pred; fused relax).
+// lanes: lanes per particle of the gathers, 1, 4 or 16 (sph_gather_lanes);
+// more than one applies to the fused step's variants (grav, visc and pred; fused relax).
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
                              bool cap, const sph_dev_params *P, const int *BS,
                              const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,

@@ -57,7 +57,8 @@ constexpr int kTPB = 256;
 // takes 11.89 ms for 64 steps and their download against 11.59.
 // The four-lanes-per-particle variants (contexts of at most two tiles per
 // CU, so at most eight of their 64-particle workgroups per CU) set no bound:
-// their 74-98 VGPRs still allow 4-6 waves per SIMD, without scratch.
+// their 66-87 VGPRs still allow 5-7 waves per SIMD, without scratch; nor do
+// the sixteen-lane ones (35-64 VGPRs).
 constexpr int kGatherMinBlocks = 6;
 #ifndef SPH_TILE_CAP
 #define SPH_TILE_CAP 1280
@@ -486,7 +487,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
                   float2 *__restrict__ held_vel)
 {
 
-    __shared__ float4 tile[VISC ? kTileCap + kSphWalkPad : 1];
+    __shared__ float4 tile[VISC && LP != 16 ? kTileCap + kSphWalkPad : 1];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
     const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
@@ -496,7 +497,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     // is live)
     const float2 a0 = POS[s], av0 = VEL[s];
     const unsigned ks = VISC ? K[s] : 0u;
-    const sph_tile_plan T = VISC ? plans[blk] : sph_tile_plan{};
+    const sph_tile_plan T = VISC ? plans[LP == 16 ? s0 / kTPB : blk] : sph_tile_plan{};
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -548,7 +549,8 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
         const sph_visc_consts V{sph_vgpr(P.h_recip), sph_vgpr(P.dt), sph_vgpr(P.sigma),
                                 sph_vgpr(P.beta)};
         auto half_impulse = [&](float4 b) {
-            return sph_visc_half(a.x, a.y, avx, avy, b.x, b.y, b.z, b.w, V, P);
+            const float dx = b.x - a.x, ddy = b.y - a.y;
+            return sph_visc_half(dx, ddy, dx * dx + ddy * ddy, avx, avy, b.z, b.w, V, P);
         };
         sph_masks_none mk;
         uint2 fh;
@@ -560,6 +562,22 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
             };
             fh = walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body,
                                            mk);
+        } else if constexpr (LP == 16) {
+            auto pair = [&](float4 b, bool cand, auto &&, bool &accepted, bool &) {
+                const float dx = b.x - a.x, ddy = b.y - a.y;
+                const float r2 = dx * dx + ddy * ddy;
+                accepted = cand && !(r2 > P.h2);
+                const float2 t = sph_visc_half(dx, ddy, accepted ? r2 : 0.5f * P.h2, avx, avy,
+                                               b.z, b.w, V, P);
+                return sph_pair_term{accepted ? t.x : 0.0f, accepted ? t.y : 0.0f};
+            };
+            auto apply = [&](const sph_pair_term &t) {
+                nvx = nvx - t.a;
+                nvy = nvy - t.b;
+            };
+            fh = sph_walk_wide<CAP>(s, live, R, P.bucket_cap, load, pair, apply, [](bool) {});
+            fh.x = sph_row_sum(fh.x);
+            fh.y = sph_row_sum(fh.y);
         } else {
             auto term = [&](unsigned, float4 b, auto &&, bool &) {
                 const float2 t = half_impulse(b);
@@ -621,6 +639,21 @@ k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict
 {
     visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
                                                 out_slot, cnt, C, clock, held_vel);
+}
+
+// Sixteen lanes per particle.
+template <bool CAP>
+__global__ void __launch_bounds__(kTPB, 1)
+k_visc_predict_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+                   const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
+                   const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+                   float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
+                   unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
+                   sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
+                   float2 *__restrict__ held_vel)
+{
+    visc_predict_tile<true, true, true, CAP, 16>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
+                                               out_slot, cnt, C, clock, held_vel);
 }
 
 // src/fluid.c:398-413 as a separate pass (phase API).
@@ -957,7 +990,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // positions only: twice the candidates of the other gathers' float4
     // tiles in the same LDS bytes, so denser rows stay in LDS at no cost in
     // occupancy (registers allow 7 workgroups per CU either way)
-    __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
+    __shared__ float2 tile[LP == 16 ? 1 : 2 * kTileCap + kSphWalkPad];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
     const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
@@ -966,7 +999,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // parameters (every slot of the grid is inside the arrays)
     const float2 a = POS[s];
     const unsigned ks = K[s];
-    const sph_tile_plan T = plans[blk];
+    const sph_tile_plan T = plans[LP == 16 ? s0 / kTPB : blk];
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -986,9 +1019,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const float h_recip = sph_vgpr(P.h_recip);
     // the pair's (1 - r/h)^2 and ^3, or zero outside h (rho + 0 == rho, as
     // rho >= +0)
-    auto pair = [&](float2 b) {
-        const float dx = a.x - b.x, ddy = a.y - b.y;
-        const float r2 = dx * dx + ddy * ddy;
+    auto weights = [&](float r2) {
         const float OmR = 1.0f - sph_sqrt_common(r2) * h_recip;
         const float OmR2 = OmR * OmR;
         float2 t = make_float2(OmR2, OmR2 * OmR);
@@ -1000,6 +1031,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         }
         return t;
     };
+    auto pair = [&](float2 b) { return weights(test(b)); };
     sph_masks_record mk;
     uint2 fh;
     if constexpr (LP == 1) {
@@ -1010,6 +1042,20 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         };
         fh = walk_group<CAP, 2 * kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body,
                                            mk);
+    } else if constexpr (LP == 16) {
+        auto wide = [&](float2 b, bool cand, auto &&, bool &accepted, bool &) {
+            const float r2 = test(b);
+            accepted = cand && !(r2 > P.h2);
+            const float2 t = weights(accepted ? r2 : 0.5f * P.h2);
+            return sph_pair_term{accepted ? t.x : 0.0f, accepted ? t.y : 0.0f};
+        };
+        auto apply = [&](const sph_pair_term &t) {
+            rho = rho + t.a;
+            rhon = rhon + t.b;
+        };
+        fh = sph_walk_wide<CAP>(s, live, R, P.bucket_cap, load, wide, apply, [](bool) {});
+        fh.x = sph_row_sum(fh.x);
+        fh.y = sph_row_sum(fh.y);
     } else {
         auto term = [&](unsigned, float2 b, auto &&, bool &) {
             const float2 t = pair(b);
@@ -1026,7 +1072,8 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     }
     if (live && lead) {
         RHO[s] = make_float2(rho, rhon);
-        masks[s] = mk.m; // for the relaxation of the same step
+        if (LP != 16)
+            masks[s] = mk.m; // for the relaxation of the same step
     }
     const unsigned full = fh.x, half = lead ? fh.y : 0u;
     report_neighbors(full, half, C);
@@ -1053,6 +1100,17 @@ k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS
     density_tile<CAP, 4>(Pp, BS, plans, POS, K, start, RHO, masks, C);
 }
 
+// Sixteen lanes per particle.
+template <bool CAP>
+__global__ void __launch_bounds__(kTPB, 1)
+k_density_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+              const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+              const unsigned *__restrict__ start, float2 *__restrict__ RHO,
+              uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
+{
+    density_tile<CAP, 16>(Pp, BS, plans, POS, K, start, RHO, masks, C);
+}
+
 // Double-density relaxation (src/fluid.c:541-611) in gather form.
 // FUSED adds the velocity update (src/fluid.c:642-653): boundary, then
 // v = (x - x_prev)/dt clamped, and the histogram of the next sort; without
@@ -1069,7 +1127,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
            unsigned long long *__restrict__ clock)
 {
 
-    __shared__ float4 tile[kTileCap + kSphWalkPad];
+    __shared__ float4 tile[LP == 16 ? 1 : kTileCap + kSphWalkPad];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
     const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
@@ -1077,7 +1135,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // the lane's own key and the tile's plan, before the scene
     // parameters (every slot of the grid is inside the arrays)
     const unsigned ks = K[s];
-    const sph_tile_plan T = plans[blk];
+    const sph_tile_plan T = plans[LP == 16 ? s0 / kTPB : blk];
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -1125,9 +1183,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const double dt2 = (double)(P.dt * P.dt);
     // the pair's displacement (zero when not pushed: n - 0 == n); on_nudge
     // hears whether an uncommon pair takes the 1e-6 nudge, before it
-    auto pair = [&](float4 b, auto &&own, auto &&on_nudge) {
-        const float dx = a.x - b.x, ddy = a.y - b.y;
-        const float r2 = dx * dx + ddy * ddy;
+    auto push = [&](float4 b, float dx, float ddy, float r2, auto &&own, auto &&on_nudge) {
         // b - a = -(a - b) exactly in IEEE arithmetic
         const sph_root q = sph_root_common(r2);
         const float D = sph_relax_D(dt2, aP + b.z, aPn + b.w, 1.0f - q.r * h_recip, k_spring, h,
@@ -1137,13 +1193,17 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             const float rr = sph_sqrt(r2);
             const float r_recip = sph_rcp(rr); // 1.0f / rr
             const float ratio = rr * h_recip;
-            const bool push = ratio < 1.0f && rr > 0.0f;
+            const bool moves = ratio < 1.0f && rr > 0.0f;
             const float E = sph_relax_D(dt2, aP + b.z, aPn + b.w, 1.0f - ratio, k_spring, h, rr);
-            t.a = push ? E * -dx * r_recip : 0.0f;
-            t.b = push ? E * -ddy * r_recip : 0.0f;
+            t.a = moves ? E * -dx * r_recip : 0.0f;
+            t.b = moves ? E * -ddy * r_recip : 0.0f;
             on_nudge(rr <= 0.000001f && own());
         }
         return t;
+    };
+    auto pair = [&](float4 b, auto &&own, auto &&on_nudge) {
+        const float dx = a.x - b.x, ddy = a.y - b.y;
+        return push(b, dx, ddy, dx * dx + ddy * ddy, own, on_nudge);
     };
     auto nudge = [&](bool yes) {
         nx = yes ? nx + 0.000001f : nx;
@@ -1162,6 +1222,17 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             sph_masks_none mk;
             walk_group<CAP, kTileCap>(T, tile, load, live, s, R, key, j, P, start, test, body, mk);
         }
+    } else if constexpr (LP == 16) {
+        auto wide = [&](float4 b, bool cand, auto &&own, bool &accepted, bool &nudged) {
+            const float dx = a.x - b.x, ddy = a.y - b.y;
+            const float r2 = dx * dx + ddy * ddy;
+            accepted = cand && !(r2 > P.h2);
+            const sph_pair_term t = push(b, dx, ddy, accepted ? r2 : 0.5f * P.h2, own,
+                                         [&](bool yes) { nudged = yes; });
+            nudged = nudged && accepted;
+            return sph_pair_term{accepted ? t.a : 0.0f, accepted ? t.b : 0.0f};
+        };
+        sph_walk_wide<CAP>(s, live, R, P.bucket_cap, load, wide, apply, nudge);
     } else {
         auto term = [&](unsigned, float4 b, auto &&own, bool &nudged) {
             return pair(b, own, [&](bool yes) { nudged = yes; });
@@ -1222,6 +1293,22 @@ k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 {
     relax_tile<true, CAP, 4>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
                              cnt, masks, C, clock);
+}
+
+// Sixteen lanes per particle.
+template <bool CAP>
+__global__ void __launch_bounds__(kTPB, 1)
+k_relax_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+            const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+            const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
+            const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+            float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
+            unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
+            const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
+            unsigned long long *__restrict__ clock)
+{
+    relax_tile<true, CAP, 16>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
+                            cnt, masks, C, clock);
 }
 
 // Reference coordinate packing (src/fluid.c:356-363), written by id.
@@ -1528,19 +1615,23 @@ k_load_state(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     ID[s] = (int)id;
 }
 
-// Four lanes per particle when the context has at most two 256-slot tiles
-// per CU (a single scene of up to 131,072 particles on 256 CUs).  There the
-// gather launches are short of work, and a launch's time is set by its
-// slowest workgroups: the dense bottom rows of a settling column, whose walks
-// four lanes cut to about a quarter.  Measured on dam breaks of 4k-1M
-// particles (graph steps 21-220 / 501-600, one lane against four): 4k 164 /
-// 87 us; 65k 164 / 91; 131k 96 against 77 and 239 against 135; 262k 102
-// against 112 and 247 against 175; 524k 121 against 183; 1M 170 against 323.
-// Past the crossover the quad's repeated per-particle work and four times
-// the tiles (staging, plans) cost more than the shorter walks gain.
-// SPH_SMALL_SCENE_LANES=1 turns the four-lane path off.
+// Several lanes per particle in small contexts.  There the gather launches are
+// short of work, and a launch's time is set by its slowest workgroups: the
+// dense bottom rows of a settling column, whose walks the lanes share.  Sixteen
+// when there is at most half a 256-slot tile per CU (32,768 particles on 256
+// CUs), four up to two (131,072), one beyond, where the lanes' repeated
+// per-particle work costs more than the shorter walks gain.  Measured on dam
+// breaks, us a step over steps 21-84 / 251-314 (one lane, four, sixteen):
+//   1.5k   56 / 90     39 / 57     31 / 39
+//   4k     54 / 133    40 / 77     30 / 48
+//   16k    57 / 139    43 / 80     39 / 58
+//   33k    56 / 133    43 / 79     48 / 64
+//   66k    56 / 134    48 / 81     63 / 83
+//   131k   60 / 135    68 / 85     96 / 118
+//   262k   67 / 141    97 / 119   154 / 185
+// SPH_SMALL_SCENE_LANES=1 turns the several-lane paths off.
 #ifndef SPH_SMALL_SCENE_LANES
-#define SPH_SMALL_SCENE_LANES 4
+#define SPH_SMALL_SCENE_LANES 16
 #endif
 int sph_gather_lanes(unsigned slots)
 {
@@ -1550,9 +1641,11 @@ int sph_gather_lanes(unsigned slots)
         (void)hipGetLastError();
         return 1;
     }
-    const unsigned long long tiles = slots / kTPB;
-    return SPH_SMALL_SCENE_LANES == 4 && cus > 0 && tiles <= 2ull * (unsigned long long)cus ? 4
-                                                                                             : 1;
+    if (cus <= 0)
+        return 1;
+    const unsigned long long tiles = slots / kTPB, n = (unsigned long long)cus;
+    const int lanes = 2ull * tiles <= n ? 16 : tiles <= 2ull * n ? 4 : 1;
+    return lanes <= SPH_SMALL_SCENE_LANES ? lanes : SPH_SMALL_SCENE_LANES;
 }
 
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
@@ -1568,6 +1661,9 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
 #define VP4(CAP)                                                                                 \
     launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS,    \
            VEL, K, start, opos, okey, oslot, cnt, C, clock, held_vel)
+#define VP16(CAP)                                                                                \
+    launch(k_visc_predict_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, plans.t256, POS, VEL, K, \
+           start, opos, okey, oslot, cnt, C, clock, held_vel)
 #define VPC(G, V, R)                                                                             \
     do {                                                                                         \
         if (cap)                                                                                 \
@@ -1577,7 +1673,12 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
     } while (0)
     // without viscosity the walk does not run: no capped variant; four lanes
     // per particle for the fused step's variant only
-    if (grav && visc && pred && lanes == 4) {
+    if (grav && visc && pred && lanes == 16) {
+        if (cap)
+            VP16(true);
+        else
+            VP16(false);
+    } else if (grav && visc && pred && lanes == 4) {
         if (cap)
             VP4(true);
         else
@@ -1594,6 +1695,7 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
         VP(false, false, true, false);
     else
         VPC(true, true, false);
+#undef VP16
 #undef VP4
 #undef VPC
 #undef VP
@@ -1698,7 +1800,13 @@ void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_
                         const unsigned *start, float2 *RHO, uint4 *masks, sph_dev_counters *C,
                         int lanes)
 {
-    if (lanes == 4 && cap)
+    if (lanes == 16 && cap)
+        launch(k_density_row<true>, GRID(16 * slots), kTPB, st, P, BS, plans.t256, POS, K, start,
+               RHO, masks, C);
+    else if (lanes == 16)
+        launch(k_density_row<false>, GRID(16 * slots), kTPB, st, P, BS, plans.t256, POS, K, start,
+               RHO, masks, C);
+    else if (lanes == 4 && cap)
         launch(k_density_quad<true>, GRID(4 * slots), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
                C);
     else if (lanes == 4)
@@ -1723,8 +1831,15 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
 #define RL4(CAP)                                                                                 \
     launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, PREV, RHO, K, start,  \
            opos, ovel, okey, oslot, cnt, masks, C, clock)
-    // four lanes per particle for the fused step's variant only
-    if (fused && lanes == 4 && cap)
+#define RL16(CAP)                                                                                \
+    launch(k_relax_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, \
+           start, opos, ovel, okey, oslot, cnt, masks, C, clock)
+    // several lanes per particle for the fused step's variant only
+    if (fused && lanes == 16 && cap)
+        RL16(true);
+    else if (fused && lanes == 16)
+        RL16(false);
+    else if (fused && lanes == 4 && cap)
         RL4(true);
     else if (fused && lanes == 4)
         RL4(false);
@@ -1736,6 +1851,7 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
         RL(false, true);
     else
         RL(false, false);
+#undef RL16
 #undef RL4
 #undef RL
 }
