@@ -175,7 +175,26 @@ void enqueue_sort_tail(sph_ctx *c, const int *id_src, unsigned *key_dst)
     }
 }
 
-// The fused step: 11 launches, no host synchronisation.
+// One of the fused step's two sorts (first: of the predicted state): the
+// particles f.src, ids id_src, by the keys and slots their producer left.
+void enqueue_sort(sph_ctx *c, bool small, bool first, const int *id_src, int *id_dst,
+                  unsigned *key_dst, const sph_reorder_fields<2> &f)
+{
+    if (small) {
+        Tick t(c, KRO);
+        sph_launch_sort_small(c->st, c->slots, c->dP, c->BS, c->ukey, first ? c->cnt : c->cnt2,
+                              first ? c->cnt2 : c->cnt, c->cells + 1, c->start,
+                              sph_buckets{c->lists, id_src}, f, id_dst, key_dst, c->dC);
+        return;
+    }
+    enqueue_sort_tail(c, id_src, key_dst);
+    Tick t(c, KRO);
+    sph_launch_reorder2(c->st, c->slots, c->dP, c->BS, c->start, c->perm_src, c->perm_id, key_dst,
+                        f, id_dst, c->plans, c->dC);
+}
+
+// The fused step: 11 launches (5 with one-launch sorts), no host
+// synchronisation.
 //   visc_predict: gravity + viscosity + predict + boundary + key/slot
 //   scan, scan, scatter, reorder   -> sorted predicted state (POS1, PREV)
 //   density                        -> RHO
@@ -185,19 +204,18 @@ void enqueue_fused_step(sph_ctx *c, bool visc)
 {
     const unsigned S = c->slots;
     const bool cap = c->bucket_cap != 0;
+    // the first step after an upload has no lists to walk, and its prediction
+    // (one lane per particle) leaves slots
+    const bool small = c->small_sort && visc;
+    int *lists = small ? c->lists : nullptr;
     {
         Tick t(c, KV);
-        sph_launch_visc_predict(c->st, S, true, visc, true, cap, c->dPA, c->BS, c->plans, c->POS0, c->VEL,
-                                c->K0, c->start, c->UPOS, c->ukey, c->uslot, c->cnt, c->dC,
-                                c->dclock, c->UVEL, c->lanes);
+        sph_launch_visc_predict(c->st, S, true, visc, true, cap, c->dPA, c->BS, c->plans, c->POS0,
+                                c->VEL, c->K0, c->start, c->UPOS, c->ukey, c->uslot, c->cnt, c->dC,
+                                c->dclock, c->UVEL, c->lanes, sph_buckets{lists, c->ID0});
     }
-    enqueue_sort_tail(c, c->ID0, c->K1);
-    {
-        Tick t(c, KRO);
-        sph_reorder_fields<2> f{{c->UPOS, c->POS0}, {c->POS1, c->PREV}};
-        sph_launch_reorder2(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K1,
-                            f, c->ID1, c->plans, c->dC);
-    }
+    enqueue_sort(c, small, true, c->ID0, c->ID1, c->K1,
+                 sph_reorder_fields<2>{{c->UPOS, c->POS0}, {c->POS1, c->PREV}});
     {
         Tick t(c, KDE);
         sph_launch_density(c->st, S, cap, c->dP, c->BS, c->plans, c->POS1, c->K1, c->start, c->RHO,
@@ -205,17 +223,32 @@ void enqueue_fused_step(sph_ctx *c, bool visc)
     }
     {
         Tick t(c, KRE);
-        sph_launch_relax(c->st, S, true, cap, c->dP, c->BS, c->plans, c->POS1, c->PREV, c->RHO, c->K1,
-                         c->start, c->UPOS, c->UVEL, c->ukey, c->uslot, c->cnt, c->MASK, c->dC,
-                         c->dclock, c->lanes);
+        sph_launch_relax(c->st, S, true, cap, c->dP, c->BS, c->plans, c->POS1, c->PREV, c->RHO,
+                         c->K1, c->start, c->UPOS, c->UVEL, c->ukey, c->uslot,
+                         small ? c->cnt2 : c->cnt, c->MASK, c->dC, c->dclock, c->lanes,
+                         sph_buckets{lists, c->ID1});
     }
-    enqueue_sort_tail(c, c->ID1, c->K0);
-    {
-        Tick t(c, KRO);
-        sph_reorder_fields<2> f{{c->UPOS, c->UVEL}, {c->POS0, c->VEL}};
-        sph_launch_reorder2(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K0,
-                            f, c->ID0, c->plans, c->dC);
-    }
+    enqueue_sort(c, small, false, c->ID1, c->ID0, c->K0,
+                 sph_reorder_fields<2>{{c->UPOS, c->UVEL}, {c->POS0, c->VEL}});
+}
+
+// The current hash's tile plans, for a gather that needs them after steps
+// whose sorts made none.
+void ensure_current_plans(sph_ctx *c)
+{
+    if (!c->plans_ok && c->lists_valid && c->n_total)
+        sph_launch_plan(c->st, c->slots, c->dP, c->BS, c->start, c->K0, c->plans);
+    c->plans_ok = true;
+}
+
+// Before fused steps: sixteen-lane gathers need no plans, and their one-launch
+// sorts leave none.
+void ensure_step_plans(sph_ctx *c)
+{
+    if (c->lanes != 16)
+        ensure_current_plans(c);
+    if (c->small_sort)
+        c->plans_ok = false;
 }
 
 int build_graph(sph_ctx *c, int steps, hipGraphExec_t *out)
@@ -280,12 +313,21 @@ int dalloc(T **p, size_t count)
     return SPH_OK;
 }
 
-// The four-lane gathers' plans exist in the contexts that use them.
-int ensure_plans(sph_ctx *c)
+// What the context's lanes per particle need: the four-lane gathers their
+// plans, sixteen-lane ones in a small grid the one-launch sort's lists.
+int ensure_lane_buffers(sph_ctx *c)
 {
-    if (c->lanes != 4 || c->plans.t64)
-        return SPH_OK;
-    return dalloc(&c->plans.t64, (size_t)c->slots / 64);
+    const unsigned m = c->cells + 1;
+    int rc = SPH_OK;
+    if (c->lanes == 4 && !c->plans.t64)
+        rc = dalloc(&c->plans.t64, (size_t)c->slots / 64);
+    const bool small = sph_sort_small_fits(m, c->lanes);
+    if (!rc && small && !c->cnt2)
+        rc = dalloc(&c->cnt2, sph_scan_padded(m));
+    if (!rc && small && !c->lists)
+        rc = dalloc(&c->lists, (size_t)m * kBucketRow);
+    c->small_sort = !rc && small;
+    return rc;
 }
 
 int check_scene_desc(const sph_scene_desc &d, int idx)
@@ -380,7 +422,7 @@ int sph_create_batch(sph_ctx **out, const sph_scene_desc *scenes, int nscenes)
 #undef A
     if (!rc) {
         c->start = c->start_mem + 4; // a spare entry before, 16-byte aligned for the scans
-        rc = ensure_plans(c);
+        rc = ensure_lane_buffers(c);
     }
     if (!rc) {
         hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
@@ -440,7 +482,8 @@ void sph_destroy(sph_ctx *c)
                     c->cnt,  c->start_mem, c->bsum,    c->coords,  c->dP,        c->BS,
                     c->dC,   c->dclock, c->SPOS,    c->SVEL,    c->SPREV,     c->SRHO,
                     c->SID,  c->SK,    c->Sstart,  c->Sclock,  c->dflags, c->MASK,
-                    c->dPA,  c->XY,    c->ACC,     c->AOS,     c->plans.t256, c->plans.t64};
+                    c->dPA,  c->XY,    c->ACC,     c->AOS,     c->plans.t256, c->plans.t64,
+                    c->cnt2, c->lists};
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);
@@ -673,13 +716,8 @@ int sph_set_gather_lanes(sph_ctx *c, int lanes)
     if (want != c->lanes)
         free_graphs(c); // the captured steps launch the other kernel variants
     c->lanes = want;
-    if (int rc = ensure_plans(c))
-        return rc;
-    if (c->lists_valid && c->n_total) { // the current hash's plans for these lanes
-        sph_launch_plan(c->st, c->slots, c->dP, c->BS, c->start, c->K0, c->plans);
-        HIPCHK(hipGetLastError());
-    }
-    return SPH_OK;
+    c->plans_ok = false; // the current hash's, for these lanes, when a gather needs them
+    return ensure_lane_buffers(c);
 }
 
 int sph_step_eager(sph_ctx *c, int nsteps)
@@ -692,9 +730,12 @@ int sph_step_eager(sph_ctx *c, int nsteps)
         return SPH_OK;
     if (int rc = refresh_first_half_params(c))
         return rc;
+    if (c->lists_valid)
+        ensure_step_plans(c);
     for (int i = 0; i < nsteps; i++) {
         enqueue_fused_step(c, c->lists_valid);
         c->lists_valid = true;
+        c->plans_ok = !c->small_sort;
         c->aux_order = 1;
         c->steps++;
         c->hashes += 2;
@@ -723,6 +764,7 @@ int sph_step(sph_ctx *c, int nsteps)
         return rc;
     if (int rc = ensure_graphs(c))
         return rc;
+    ensure_step_plans(c);
     while (nsteps >= kGraphSteps) {
         HIPCHK(hipGraphLaunch(c->gK, c->st));
         nsteps -= kGraphSteps;
@@ -788,6 +830,7 @@ int sph_step_tunables2(sph_ctx *c, const tunable_parameters *first,
     } else {
         rc = ensure_graphs(c);
         if (!rc) {
+            ensure_step_plans(c);
             hipError_t e = hipGraphLaunch(c->g1, c->st);
             if (e != hipSuccess)
                 rc = set_err(SPH_EHIP, "hipGraphLaunch failed: %s", hipGetErrorString(e));
@@ -822,9 +865,10 @@ int sph_phase_viscosity(sph_ctx *c)
         return rc;
     if (!c->lists_valid || c->n_total == 0)
         return SPH_OK; // empty lists (src/fluid.c:202)
+    ensure_current_plans(c);
     sph_launch_visc_predict(c->st, c->slots, false, true, false, c->bucket_cap != 0, c->dP, c->BS,
                             c->plans, c->POS0, c->VEL, c->K0, c->start, c->UVEL, nullptr, nullptr, c->cnt,
-                            c->dC, c->dclock, nullptr, c->lanes);
+                            c->dC, c->dclock, nullptr, c->lanes, sph_buckets{});
     HIPCHK(hipMemcpyAsync(c->VEL, c->UVEL, sizeof(float2) * (size_t)c->slots,
                           hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());
@@ -858,6 +902,7 @@ int sph_phase_hash(sph_ctx *c, int compute_density)
                             {c->POS1, c->UVEL, c->T2a, c->T2b}};
     sph_launch_reorder4(c->st, S, c->dP, c->BS, c->start, c->perm_src, c->perm_id, c->K1, f,
                         c->ID1, c->plans, c->dC);
+    c->plans_ok = true;
     const size_t b = sizeof(float2) * (size_t)S;
     sph_copy_set cs;
     for (int k = 0; k < 4; k++)
@@ -884,9 +929,10 @@ int sph_phase_relax(sph_ctx *c)
         return SPH_OK;
     if (!c->lists_valid)
         return set_err(SPH_ESTATE, "sph_phase_relax: no hash since upload");
+    ensure_current_plans(c);
     sph_launch_relax(c->st, c->slots, false, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->PREV,
                      c->RHO, c->K0, c->start, c->UPOS, nullptr, nullptr, nullptr, nullptr,
-                     nullptr, c->dC, c->dclock, c->lanes);
+                     nullptr, c->dC, c->dclock, c->lanes, sph_buckets{});
     HIPCHK(hipMemcpyAsync(c->POS0, c->UPOS, sizeof(float2) * (size_t)c->slots,
                           hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());
@@ -966,7 +1012,7 @@ int sph_snapshot_restore(sph_ctx *c, const int *scene_flags)
                        {c->POS0, c->VEL, c->PREV, c->RHO},
                        c->SID, c->ID0, c->SK, c->Sstart, c->K0, c->start};
     sph_launch_restore(c->st, c->slots, c->dP, c->BS, c->dflags, a);
-    sph_launch_plan(c->st, c->slots, c->dP, c->BS, c->start, c->K0, c->plans);
+    c->plans_ok = false;
     HIPCHK(hipMemcpyAsync(c->dclock, c->Sclock, sizeof(unsigned long long),
                           hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());
@@ -1215,6 +1261,7 @@ int sph_time_kernels(sph_ctx *c, int nsteps, int max_kinds, const char **names, 
         if (rc)
             return rc;
     }
+    ensure_step_plans(c);
     // One start/stop event pair per launch, created up front; the launches
     // record them around the kernels themselves (hipExtLaunchKernelGGL), and
     // all nsteps steps are enqueued before the one synchronisation.
@@ -1301,3 +1348,4 @@ int sph_selftest_rcp(unsigned lo_bits, unsigned hi_bits, unsigned long long *mis
 } // extern "C"
 
 int sph_internal_canonicalize(sph_ctx *c) { return canonicalize(c); }
+void sph_internal_plans(sph_ctx *c) { ensure_current_plans(c); }

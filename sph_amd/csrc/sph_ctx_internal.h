@@ -56,6 +56,13 @@ struct sph_ctx {
              *start = nullptr, *bsum = nullptr;
     unsigned *start_mem = nullptr; // start's allocation (start has a spare entry before it)
     sph_tile_plans plans;          // of the hash that K0 or K1 and start describe
+    bool plans_ok = false;         // ... made since that hash (a small sort makes none)
+    // one-launch sorts of a small context: the second count array (cnt is zero
+    // between steps, cnt2 is cleared by each step's first sort) and the cells'
+    // member lists
+    bool small_sort = false;
+    unsigned *cnt2 = nullptr;
+    int *lists = nullptr;
     short *coords = nullptr;
     uint4 *MASK = nullptr; // per slot: the density pass's first accepted-candidate masks
     float2 *ACC = nullptr;  // (a_x, a_y) by caller index: carried, never changed (src/fluid.c)
@@ -77,5 +84,7 @@ struct sph_ctx {
     size_t tidx = 0;
 };
 
-// Bring PREV/RHO into the canonical (ID0) order; defined in sph_ctx.hip.
+// Bring PREV/RHO into the canonical (ID0) order, and make the current hash's
+// tile plans if its sort made none; defined in sph_ctx.hip.
 int sph_internal_canonicalize(sph_ctx *c);
+void sph_internal_plans(sph_ctx *c);

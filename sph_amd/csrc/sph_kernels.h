@@ -17,6 +17,16 @@ struct sph_tile_plans {
     sph_tile_plan *t256 = nullptr, *t64 = nullptr;
 };
 
+// The per-cell member lists of a small context's sort (sph_launch_sort_small):
+// row `cell` of kBucketRow ints holds the ids of the particles that claimed
+// its first kBucketRow slots.  rows null: no lists; ids: the producing
+// kernel's particles' ids.
+constexpr unsigned kBucketRow = 128;
+struct sph_buckets {
+    int *rows = nullptr;
+    const int *ids = nullptr;
+};
+
 // Workgroup size of every particle kernel; scenes are padded to multiples.
 constexpr unsigned kSphTPB = 256;
 
@@ -32,7 +42,7 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
                              const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,
                              float2 *opos, unsigned *okey, unsigned *oslot, unsigned *cnt,
                              sph_dev_counters *C, const unsigned long long *clock,
-                             float2 *held_vel, int lanes);
+                             float2 *held_vel, int lanes, const sph_buckets &lists);
 void sph_launch_gravity(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                         float2 *VEL, float2 *RHO);
 void sph_launch_predict(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
@@ -64,6 +74,15 @@ void sph_launch_reorder4(hipStream_t st, unsigned slots, const sph_dev_params *P
                          const unsigned *start, const int *perm_src, const int *perm_id,
                          const unsigned *skey, sph_reorder_fields<4> f, int *id_dst,
                          const sph_tile_plans &plans, sph_dev_counters *C);
+// The whole sort of a small context (sph_sort_small_fits), whose producing
+// kernel left its members' ids in `lists`: starts, sorted keys, ids and fields
+// in one launch, and cnt_next cleared.
+bool sph_sort_small_fits(unsigned m, int lanes);
+void sph_launch_sort_small(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
+                           const unsigned *key, const unsigned *cnt, unsigned *cnt_next,
+                           unsigned m, unsigned *start, const sph_buckets &lists,
+                           sph_reorder_fields<2> f, int *id_dst, unsigned *key_dst,
+                           sph_dev_counters *C);
 // The tile plans alone, of sorted keys that no reorder has just placed.
 void sph_launch_plan(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                      const unsigned *start, const unsigned *skey, const sph_tile_plans &plans);
@@ -76,7 +95,7 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
                       const float2 *POS, const float2 *PREV, const float2 *RHO, const unsigned *K,
                       const unsigned *start, float2 *opos, float2 *ovel, unsigned *okey,
                       unsigned *oslot, unsigned *cnt, const uint4 *masks, sph_dev_counters *C,
-                      unsigned long long *clock, int lanes);
+                      unsigned long long *clock, int lanes, const sph_buckets &lists);
 void sph_launch_pack_coords(hipStream_t st, unsigned slots, const sph_dev_params *P,
                             const int *BS, const float2 *POS, const int *ID, short *out);
 void sph_launch_neighbor_lists(hipStream_t st, unsigned slots, const sph_dev_params *P,

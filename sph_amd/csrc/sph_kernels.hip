@@ -22,7 +22,8 @@
 // for the next sort); a scatter drops (id, source) pairs into the cell
 // ranges; the reorder kernel ranks each particle by id inside its cell and
 // gathers its fields there - the canonical (cell, id) order of
-// src/hash.c:153-163.
+// src/hash.c:153-163.  In a small context one kernel does all that follows the
+// claims (k_sort_small).
 //
 // Several independent scenes can share one launch: each scene owns a
 // 256-aligned range of slots of the sorted arrays and a range of global
@@ -250,6 +251,19 @@ __device__ __forceinline__ unsigned wave_slot(unsigned *cnt, unsigned key)
     return __shfl(base, leader, 64) + rank;
 }
 
+// Claim a slot of cell `key` for the next sort: the slot itself, or the
+// particle's id in the cell's member list (ids beyond the row are found by the
+// sort).
+__device__ __forceinline__ void claim_slot(unsigned s, unsigned key, int id, unsigned *cnt,
+                                           unsigned *out_slot, const sph_buckets &lists)
+{
+    const unsigned slot = wave_slot(cnt, key);
+    if (!lists.rows)
+        out_slot[s] = slot;
+    else if (slot < kBucketRow)
+        lists.rows[(size_t)key * kBucketRow + slot] = id;
+}
+
 // LDS storage of a tile of CAPACITY records (plus the walk's padding): as
 // the records are, or - float4 records, SPH_SPLIT_TILES - as two planes of
 // float2, (x, y) and (z, w), in the same bytes, so that the candidate tests
@@ -406,11 +420,13 @@ __device__ __forceinline__ GlobalSrc<Rec, Load> global_src(Load l)
 }
 
 // The cell row of the lane's particle (a pad lane's: row 0, its stand-in
-// cell's), from the plan unless the tile spans more than two.
+// cell's), from the plan unless there is none (NO_PLAN) or the tile spans more
+// than two.
+template <bool NO_PLAN>
 __device__ __forceinline__ unsigned cell_row(const sph_tile_plan &T, bool live, unsigned s,
                                              unsigned key, const sph_dev_params &P)
 {
-    if (T.wide)
+    if (NO_PLAN || T.wide)
         return (key - P.cell_base) / P.sx;
     return live ? T.jA + (s >= T.split ? 1u : 0u) : 0u;
 }
@@ -484,7 +500,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
                   float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                   unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                   sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
-                  float2 *__restrict__ held_vel)
+                  float2 *__restrict__ held_vel, const sph_buckets &lists = {})
 {
 
     __shared__ float4 tile[VISC && LP != 16 ? kTileCap + kSphWalkPad : 1];
@@ -497,7 +513,8 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     // is live)
     const float2 a0 = POS[s], av0 = VEL[s];
     const unsigned ks = VISC ? K[s] : 0u;
-    const sph_tile_plan T = VISC ? plans[LP == 16 ? s0 / kTPB : blk] : sph_tile_plan{};
+    const int id = lists.rows ? lists.ids[s] : 0;
+    const sph_tile_plan T = VISC && LP != 16 ? plans[blk] : sph_tile_plan{};
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -516,7 +533,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
             held_vel[s] = VEL[s];
             const unsigned key = sph_cell_key(a.x, a.y, P, &C->key_out_of_range);
             out_key[s] = key;
-            out_slot[s] = wave_slot(cnt, key);
+            claim_slot(s, key, id, cnt, out_slot, lists);
         }
         return;
     }
@@ -528,7 +545,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     const float2 a = a0, av = av0;
     const bool live = s < s1;
     const unsigned key = VISC && live ? ks : P.cell_base; // pad lanes: any valid cell
-    const unsigned j = VISC ? cell_row(T, live, s, key, P) : 0u;
+    const unsigned j = VISC ? cell_row<LP == 16>(T, live, s, key, P) : 0u;
     const sph_rows R = VISC ? sph_row_bounds(key, j, P, start) : sph_rows{};
     const float avx = slosh ? av.x + sdt : av.x;
     const float avy = GRAV ? av.y + gdt : av.y;
@@ -603,7 +620,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
             out_pos[s] = make_float2(x, y);
             const unsigned nk = sph_cell_key(x, y, P, &C->key_out_of_range);
             out_key[s] = nk;
-            out_slot[s] = wave_slot(cnt, nk);
+            claim_slot(s, nk, id, cnt, out_slot, lists);
         } else {
             out_pos[s] = make_float2(nvx, nvy);
         }
@@ -645,15 +662,15 @@ k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
 k_visc_predict_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-                   const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
+                   const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
                    const unsigned *__restrict__ K, const unsigned *__restrict__ start,
                    float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                    unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
-                   float2 *__restrict__ held_vel)
+                   float2 *__restrict__ held_vel, sph_buckets lists)
 {
-    visc_predict_tile<true, true, true, CAP, 16>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
-                                               out_slot, cnt, C, clock, held_vel);
+    visc_predict_tile<true, true, true, CAP, 16>(Pp, BS, nullptr, POS, VEL, K, start, out_pos, out_key,
+                                               out_slot, cnt, C, clock, held_vel, lists);
 }
 
 // src/fluid.c:398-413 as a separate pass (phase API).
@@ -967,6 +984,159 @@ k_reorder(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         raise_max(&C->max_cell_count, m);
 }
 
+// The whole sort of a small context in one launch.  Every workgroup makes all
+// cell starts for itself, in LDS, from the counts (at most kSmallCounts; they
+// come from L2), and then places its own 256 source particles: the rank in the
+// cell from the cell's member list, the fields straight to their sorted
+// position.  The starts in memory are written, and the other counts cleared,
+// by all workgroups together.  Two count arrays take turns (the counts read
+// here are cleared by the next sort), because no workgroup may clear what
+// another still reads.  The members of a cell that its list's row does not
+// hold are searched for among the scene's keys, by the whole workgroup, one
+// such cell after the other.
+//
+// us a step with this sort, against scan + scatter + reorder, steps 21-84 /
+// 251-314: 1.5k 24 / 31 against 31 / 39, 4k 24 / 39 against 30 / 48, 16k 32 /
+// 51 against 39 / 58, 25k 38 / 55 against 44 / 62.
+// TPB threads, of which the first 256 own a particle each; thread t sums the
+// counts [SEG t, SEG t + SEG) of the LDS copy (four spare words a segment keep
+// the threads' 16-byte reads on different banks).
+constexpr unsigned kSmallCounts = 32768;
+
+template <int SEG, int TPB>
+__global__ void __launch_bounds__(TPB)
+k_sort_small(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+             const unsigned *__restrict__ key, const uint4 *__restrict__ cnt,
+             uint4 *__restrict__ cnt_next, unsigned mp, uint4 *__restrict__ start,
+             sph_buckets lists, sph_reorder_fields<2> f, int *__restrict__ id_dst,
+             unsigned *__restrict__ key_dst, sph_dev_counters *__restrict__ C)
+{
+    constexpr unsigned kStride = SEG + 4;
+    __shared__ __align__(16) unsigned sc[TPB * kStride];
+    __shared__ unsigned wsum[TPB / kWave];
+    auto at = [](unsigned c) { return c / SEG * kStride + c % SEG; };
+    const unsigned blk = blockIdx.x, t = threadIdx.x;
+    const bool owner = TPB == kTPB || t < (unsigned)kTPB;
+    const unsigned i = blk * kTPB + (owner ? t : 0u);
+    // the own particle, on its way while the starts are made
+    const unsigned k0 = key[i];
+    const int myid = lists.ids[i];
+    const float2 v0 = f.src[0][i], v1 = f.src[1][i];
+    const sph_dev_params &P = Pp[BS[blk]];
+    const unsigned end = P.poff + (unsigned)P.n;
+    const bool live = owner && i < end;
+    const unsigned c = live ? k0 : 0u;
+    // the start of the cell's list, as well
+    constexpr unsigned kFirst = 16;
+    int4 row[kFirst / 4];
+    const int4 *list = reinterpret_cast<const int4 *>(lists.rows + (size_t)c * kBucketRow);
+#pragma unroll
+    for (unsigned u = 0; u < kFirst / 4; u++)
+        row[u] = list[u];
+    // counts into LDS, then exclusive sums in place
+    for (unsigned u = t; u < mp / 4u; u += TPB)
+        *(uint4 *)&sc[at(4u * u)] = cnt[u];
+    __syncthreads();
+    const unsigned segs = mp / SEG; // mp: a multiple of 2,048, at most TPB segments
+    unsigned *seg = &sc[t * kStride];
+    unsigned tot = 0;
+    if (t < segs)
+        for (unsigned u = 0; u < SEG; u += 4)
+            tot += sum4(*(const uint4 *)&seg[u]);
+    unsigned inc = tot;
+    const unsigned lane = t & (kWave - 1u);
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const unsigned y = (unsigned)__shfl_up((int)inc, o, kWave);
+        inc += lane >= (unsigned)o ? y : 0u;
+    }
+    if (lane == kWave - 1u)
+        wsum[t / kWave] = inc;
+    __syncthreads();
+    unsigned run = inc - tot;
+    for (unsigned w = 0; w < t / kWave; w++)
+        run += wsum[w];
+    if (t < segs)
+        for (unsigned u = 0; u < SEG; u += 4) {
+            const uint4 n = *(const uint4 *)&seg[u];
+            *(uint4 *)&seg[u] = make_uint4(run, run + n.x, run + n.x + n.y, run + n.x + n.y + n.z);
+            run += sum4(n);
+        }
+    __syncthreads();
+    // every workgroup's share of the starts and of the cleared counts
+    for (unsigned u = blk * TPB + t; u < mp / 4u; u += gridDim.x * TPB) {
+        start[u] = *(const uint4 *)&sc[at(4u * u)];
+        cnt_next[u] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    const unsigned b = sc[at(c)], n = sc[at(c + 1u)] - b; // c + 1 <= cells < mp
+    unsigned rank = 0;
+    if (live && n <= kBucketRow) {
+        auto count4 = [&](int4 q, unsigned m) {
+            rank += (m < n && q.x < myid ? 1u : 0u) + (m + 1u < n && q.y < myid ? 1u : 0u) +
+                    (m + 2u < n && q.z < myid ? 1u : 0u) + (m + 3u < n && q.w < myid ? 1u : 0u);
+        };
+#pragma unroll
+        for (unsigned u = 0; u < kFirst / 4; u++)
+            count4(row[u], 4u * u);
+        for (unsigned m = kFirst; m < n; m += 16u) {
+            int4 q[4];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++)
+                q[u] = list[min(m / 4u + u, kBucketRow / 4u - 1u)];
+#pragma unroll
+            for (unsigned u = 0; u < 4; u++)
+                count4(q[u], m + 4u * u);
+        }
+    }
+    bool over = live && n > kBucketRow;
+    if (__syncthreads_or(over)) {
+        __shared__ unsigned pick, nfound;
+        __shared__ int found[TPB];
+        for (;;) {
+            if (t == 0) {
+                pick = ~0u;
+                nfound = 0;
+            }
+            __syncthreads();
+            if (over)
+                atomicMin(&pick, c);
+            __syncthreads();
+            const unsigned cell = pick;
+            if (cell == ~0u)
+                break; // every thread at once
+            const bool mine = over && c == cell;
+            for (unsigned m0 = P.poff; m0 < end; m0 += TPB) {
+                if (m0 + t < end && key[m0 + t] == cell)
+                    found[atomicAdd(&nfound, 1u)] = lists.ids[m0 + t];
+                __syncthreads();
+                const unsigned nf = nfound;
+                if (mine)
+                    for (unsigned u = 0; u < nf; u++)
+                        rank += found[u] < myid ? 1u : 0u;
+                __syncthreads();
+                if (t == 0)
+                    nfound = 0;
+                __syncthreads();
+            }
+            over = over && !mine;
+        }
+    }
+    unsigned occupancy = 0;
+    if (live) {
+        const unsigned d = b + rank;
+        f.dst[0][d] = v0;
+        f.dst[1][d] = v1;
+        id_dst[d] = myid;
+        key_dst[d] = c;
+        if (rank == SPH_REF_MAX_BUCKET)
+            atomicAdd(&C->bucket_overflow, 1ull);
+        occupancy = rank + 1;
+    }
+    const unsigned m = wave_max_u32(occupancy);
+    if (lane0())
+        raise_max(&C->max_cell_count, m);
+}
+
 // The tile plans alone (sph_launch_plan).
 __global__ void __launch_bounds__(kTPB)
 k_plan(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsigned tiles,
@@ -999,7 +1169,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // parameters (every slot of the grid is inside the arrays)
     const float2 a = POS[s];
     const unsigned ks = K[s];
-    const sph_tile_plan T = plans[LP == 16 ? s0 / kTPB : blk];
+    const sph_tile_plan T = LP != 16 ? plans[blk] : sph_tile_plan{};
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -1008,7 +1178,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // the candidate rows, before the barriers
     const bool live = s < s1;
     const unsigned key = live ? ks : P.cell_base; // pad lanes: any valid cell
-    const unsigned j = cell_row(T, live, s, key, P);
+    const unsigned j = cell_row<LP == 16>(T, live, s, key, P);
     const sph_rows R = sph_row_bounds(key, j, P, start);
     float rho = 0.0f, rhon = 0.0f;
     auto load = [&](unsigned g) { return POS[g]; };
@@ -1104,11 +1274,11 @@ k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
 k_density_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-              const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+              const float2 *__restrict__ POS, const unsigned *__restrict__ K,
               const unsigned *__restrict__ start, float2 *__restrict__ RHO,
               uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
-    density_tile<CAP, 16>(Pp, BS, plans, POS, K, start, RHO, masks, C);
+    density_tile<CAP, 16>(Pp, BS, nullptr, POS, K, start, RHO, masks, C);
 }
 
 // Double-density relaxation (src/fluid.c:541-611) in gather form.
@@ -1124,7 +1294,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
            float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
            unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
            const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
-           unsigned long long *__restrict__ clock)
+           unsigned long long *__restrict__ clock, const sph_buckets &lists = {})
 {
 
     __shared__ float4 tile[LP == 16 ? 1 : kTileCap + kSphWalkPad];
@@ -1135,7 +1305,8 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     // the lane's own key and the tile's plan, before the scene
     // parameters (every slot of the grid is inside the arrays)
     const unsigned ks = K[s];
-    const sph_tile_plan T = plans[LP == 16 ? s0 / kTPB : blk];
+    const int id = lists.rows ? lists.ids[s] : 0;
+    const sph_tile_plan T = LP != 16 ? plans[blk] : sph_tile_plan{};
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
@@ -1154,7 +1325,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             out_pos[s] = a;
             const unsigned nk = sph_cell_key(a.x, a.y, P, &C->key_out_of_range);
             out_key[s] = nk;
-            out_slot[s] = wave_slot(cnt, nk);
+            claim_slot(s, nk, id, cnt, out_slot, lists);
         }
         return;
     }
@@ -1164,7 +1335,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const float2 ar = RHO[s];
     const bool live = s < s1;
     const unsigned key = live ? ks : P.cell_base; // pad lanes: any valid cell
-    const unsigned j = cell_row(T, live, s, key, P);
+    const unsigned j = cell_row<LP == 16>(T, live, s, key, P);
     const sph_rows R = sph_row_bounds(key, j, P, start);
     // a neighbour's record carries its pressure and near-pressure
     // (src/fluid.c:563-564), evaluated once per record rather than per pair
@@ -1259,7 +1430,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             atomicAdd(&C->nonfinite, 1ull);
         const unsigned nk = sph_cell_key(nx, ny, P, &C->key_out_of_range);
         out_key[s] = nk;
-        out_slot[s] = wave_slot(cnt, nk);
+        claim_slot(s, nk, id, cnt, out_slot, lists);
     }
     out_pos[s] = make_float2(nx, ny);
 }
@@ -1299,16 +1470,16 @@ k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
 k_relax_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-            const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+            const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
             const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
             const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
             float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
             unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
             const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
-            unsigned long long *__restrict__ clock)
+            unsigned long long *__restrict__ clock, sph_buckets lists)
 {
-    relax_tile<true, CAP, 16>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
-                            cnt, masks, C, clock);
+    relax_tile<true, CAP, 16>(Pp, BS, nullptr, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
+                            cnt, masks, C, clock, lists);
 }
 
 // Reference coordinate packing (src/fluid.c:356-363), written by id.
@@ -1622,13 +1793,14 @@ k_load_state(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 // CUs), four up to two (131,072), one beyond, where the lanes' repeated
 // per-particle work costs more than the shorter walks gain.  Measured on dam
 // breaks, us a step over steps 21-84 / 251-314 (one lane, four, sixteen):
-//   1.5k   56 / 90     39 / 57     31 / 39
-//   4k     54 / 133    40 / 77     30 / 48
-//   16k    57 / 139    43 / 80     39 / 58
-//   33k    56 / 133    43 / 79     48 / 64
+//   1.5k   56 / 90     39 / 57     24 / 31
+//   4k     54 / 133    40 / 77     24 / 39
+//   16k    57 / 139    43 / 80     32 / 51
+//   33k    56 / 133    43 / 79     44 / 60
 //   66k    56 / 134    48 / 81     63 / 83
 //   131k   60 / 135    68 / 85     96 / 118
 //   262k   67 / 141    97 / 119   154 / 185
+// (sixteen lanes with k_sort_small up to 33k; 39 / 58 at 16k without).
 // SPH_SMALL_SCENE_LANES=1 turns the several-lane paths off.
 #ifndef SPH_SMALL_SCENE_LANES
 #define SPH_SMALL_SCENE_LANES 16
@@ -1653,7 +1825,7 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
                              const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,
                              float2 *opos, unsigned *okey, unsigned *oslot, unsigned *cnt,
                              sph_dev_counters *C, const unsigned long long *clock,
-                             float2 *held_vel, int lanes)
+                             float2 *held_vel, int lanes, const sph_buckets &lists)
 {
 #define VP(G, V, R, CAP)                                                                         \
     launch(k_visc_predict<G, V, R, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, VEL, K, start, opos, \
@@ -1662,8 +1834,8 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
     launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS,    \
            VEL, K, start, opos, okey, oslot, cnt, C, clock, held_vel)
 #define VP16(CAP)                                                                                \
-    launch(k_visc_predict_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, plans.t256, POS, VEL, K, \
-           start, opos, okey, oslot, cnt, C, clock, held_vel)
+    launch(k_visc_predict_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, POS, VEL, K, start, opos,   \
+           okey, oslot, cnt, C, clock, held_vel, lists)
 #define VPC(G, V, R)                                                                             \
     do {                                                                                         \
         if (cap)                                                                                 \
@@ -1788,6 +1960,35 @@ void sph_launch_reorder4(hipStream_t st, unsigned slots, const sph_dev_params *P
            skey, f, id_dst, planners, plans, C);
 }
 
+bool sph_sort_small_fits(unsigned m, int lanes)
+{
+    return lanes == 16 && sph_scan_padded(m) <= kSmallCounts;
+}
+
+void sph_launch_sort_small(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
+                           const unsigned *key, const unsigned *cnt, unsigned *cnt_next,
+                           unsigned m, unsigned *start, const sph_buckets &lists,
+                           sph_reorder_fields<2> f, int *id_dst, unsigned *key_dst,
+                           sph_dev_counters *C)
+{
+    const unsigned mp = (unsigned)sph_scan_padded(m);
+#define SORT(SEG, TPB)                                                                           \
+    launch(k_sort_small<SEG, TPB>, GRID(slots), TPB, st, P, BS, key,                             \
+           reinterpret_cast<const uint4 *>(cnt), reinterpret_cast<uint4 *>(cnt_next), mp,        \
+           reinterpret_cast<uint4 *>(start), lists, f, id_dst, key_dst, C)
+    if (mp <= 2048u)
+        SORT(8, 256);
+    else if (mp <= 4096u)
+        SORT(16, 256);
+    else if (mp <= 8192u)
+        SORT(16, 512);
+    else if (mp <= 16384u)
+        SORT(16, 1024);
+    else
+        SORT(32, 1024);
+#undef SORT
+}
+
 void sph_launch_plan(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                      const unsigned *start, const unsigned *skey, const sph_tile_plans &plans)
 {
@@ -1801,11 +2002,11 @@ void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_
                         int lanes)
 {
     if (lanes == 16 && cap)
-        launch(k_density_row<true>, GRID(16 * slots), kTPB, st, P, BS, plans.t256, POS, K, start,
-               RHO, masks, C);
+        launch(k_density_row<true>, GRID(16 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
+               C);
     else if (lanes == 16)
-        launch(k_density_row<false>, GRID(16 * slots), kTPB, st, P, BS, plans.t256, POS, K, start,
-               RHO, masks, C);
+        launch(k_density_row<false>, GRID(16 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
+               C);
     else if (lanes == 4 && cap)
         launch(k_density_quad<true>, GRID(4 * slots), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
                C);
@@ -1823,7 +2024,7 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
                       const float2 *POS, const float2 *PREV, const float2 *RHO, const unsigned *K,
                       const unsigned *start, float2 *opos, float2 *ovel, unsigned *okey,
                       unsigned *oslot, unsigned *cnt, const uint4 *masks, sph_dev_counters *C,
-                      unsigned long long *clock, int lanes)
+                      unsigned long long *clock, int lanes, const sph_buckets &lists)
 {
 #define RL(F, CAP)                                                                               \
     launch(k_relax<F, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, start, opos, ovel,   \
@@ -1832,8 +2033,8 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
     launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, PREV, RHO, K, start,  \
            opos, ovel, okey, oslot, cnt, masks, C, clock)
 #define RL16(CAP)                                                                                \
-    launch(k_relax_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, \
-           start, opos, ovel, okey, oslot, cnt, masks, C, clock)
+    launch(k_relax_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, POS, PREV, RHO, K, start, opos, \
+           ovel, okey, oslot, cnt, masks, C, clock, lists)
     // several lanes per particle for the fused step's variant only
     if (fused && lanes == 16 && cap)
         RL16(true);

@@ -1260,6 +1260,8 @@ int density_now(sph_ctx *c)
         return rc;
     if (!c->lists_valid)
         return merr(SPH_ESTATE, "surrogate: state not hashed");
+    if (c->lanes != 16)
+        sph_internal_plans(c);
     sph_launch_density(c->st, c->slots, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->K0,
                        c->start, c->RHO, c->MASK, c->dC, c->lanes);
     MCHK(hipGetLastError());
