@@ -356,17 +356,17 @@ class Solver:
         self.tunables = second
 
     def download_positions(self) -> np.ndarray:
-        out = np.zeros((self.n, 2), np.float32)
+        out = np.empty((self.n, 2), np.float32)
         _check(lib().sph_download_positions(self._h, out.ctypes.data), "sph_download_positions")
         return out
 
     def download(self) -> np.ndarray:
-        out = np.zeros(self.n, PARTICLE)
+        out = np.empty(self.n, PARTICLE)
         _check(lib().sph_download(self._h, out.ctypes.data), "sph_download")
         return out
 
     def pack_coords(self) -> np.ndarray:
-        out = np.zeros((self.n, 2), np.int16)
+        out = np.empty((self.n, 2), np.int16)
         _check(lib().sph_pack_coords_i16(self._h, out.ctypes.data), "sph_pack_coords_i16")
         return out
 
@@ -473,7 +473,7 @@ class Surrogate:
         _check_m(lib().sph_surrogate_zero_grads(self._h), "zero_grads")
 
     def predict(self, solver: Solver) -> np.ndarray:
-        out = np.zeros((solver.n, 2), np.float32)
+        out = np.empty((solver.n, 2), np.float32)
         _check_m(lib().sph_surrogate_predict(self._h, solver._h, out.ctypes.data), "predict")
         return out
 

@@ -65,6 +65,12 @@ struct sph_ctx {
     int *lists = nullptr;
     short *coords = nullptr;
     uint4 *MASK = nullptr; // per slot: the density pass's first accepted-candidate masks
+    // pinned memory through which large results reach the caller's (two halves
+    // of ring_half bytes; null in contexts whose results are small), its
+    // pieces' flags and the last value that marked them
+    char *ring = nullptr;
+    unsigned *ring_flags = nullptr, ring_mark = 0;
+    size_t ring_half = 0;
     float2 *ACC = nullptr;  // (a_x, a_y) by caller index: carried, never changed (src/fluid.c)
     float *AOS = nullptr;   // fluid_particle records by caller index (allocated on first download)
     bool lists_valid = false; // a hash ran since upload: K0/start describe POS0
@@ -83,6 +89,11 @@ struct sph_ctx {
     std::vector<int> *tkind = nullptr;
     size_t tidx = 0;
 };
+
+// Copy `bytes` of device memory (16-byte aligned, a multiple of 4) to the
+// caller's pageable memory after all work of the context's stream, and wait;
+// defined in sph_ctx.hip.
+int sph_internal_fetch(sph_ctx *c, void *out, const void *src, size_t bytes);
 
 // Bring PREV/RHO into the canonical (ID0) order, and make the current hash's
 // tile plans if its sort made none; defined in sph_ctx.hip.

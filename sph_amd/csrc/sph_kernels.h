@@ -86,6 +86,11 @@ void sph_launch_sort_small(hipStream_t st, unsigned slots, const sph_dev_params 
 // The tile plans alone, of sorted keys that no reorder has just placed.
 void sph_launch_plan(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                      const unsigned *start, const unsigned *skey, const sph_tile_plans &plans);
+// Copy src to pinned host memory, and set the flag of every kHostPiece bytes to
+// `mark` once they are there.
+constexpr size_t kHostPiece = 32u << 10;
+void sph_launch_to_host(hipStream_t st, const void *src, void *dst, size_t bytes,
+                        unsigned *flags, unsigned mark);
 void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_params *P,
                         const int *BS, const sph_tile_plans &plans, const float2 *POS, const unsigned *K,
                         const unsigned *start, float2 *RHO, uint4 *masks, sph_dev_counters *C,

@@ -1482,6 +1482,35 @@ k_relax_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
                             cnt, masks, C, clock, lists);
 }
 
+// One piece of a result to pinned host memory and, when the host can read it,
+// the piece's flag: the host copies a piece on while the next ones cross the
+// link, which bounds this kernel (19 us a MB).
+__global__ void __launch_bounds__(kTPB)
+k_to_host(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t bytes,
+          unsigned *__restrict__ flags, unsigned mark)
+{
+    constexpr unsigned kWords = kHostPiece / sizeof(uint4), kEach = kWords / kTPB;
+    const size_t w0 = (size_t)blockIdx.x * kWords, words = bytes / sizeof(uint4);
+    const unsigned t = threadIdx.x;
+    uint4 v[kEach];
+#pragma unroll
+    for (unsigned u = 0; u < kEach; u++)
+        if (w0 + u * kTPB + t < words)
+            v[u] = src[w0 + u * kTPB + t];
+#pragma unroll
+    for (unsigned u = 0; u < kEach; u++)
+        if (w0 + u * kTPB + t < words)
+            dst[w0 + u * kTPB + t] = v[u];
+    const unsigned rest = (unsigned)(bytes % sizeof(uint4)) / 4u;
+    if (blockIdx.x == gridDim.x - 1 && t < rest)
+        reinterpret_cast<unsigned *>(dst + words)[t] =
+            reinterpret_cast<const unsigned *>(src + words)[t];
+    __threadfence_system();
+    __syncthreads();
+    if (t == 0)
+        __hip_atomic_store(&flags[blockIdx.x], mark, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Reference coordinate packing (src/fluid.c:356-363), written by id.
 __global__ void __launch_bounds__(kTPB)
 k_pack_coords(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
@@ -2055,6 +2084,13 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
 #undef RL16
 #undef RL4
 #undef RL
+}
+
+void sph_launch_to_host(hipStream_t st, const void *src, void *dst, size_t bytes,
+                        unsigned *flags, unsigned mark)
+{
+    launch(k_to_host, dim3((unsigned)((bytes + kHostPiece - 1) / kHostPiece)), kTPB, st,
+           (const uint4 *)src, (uint4 *)dst, bytes, flags, mark);
 }
 
 void sph_launch_pack_coords(hipStream_t st, unsigned slots, const sph_dev_params *P,

@@ -1426,9 +1426,9 @@ int sph_surrogate_predict(sph_surrogate *m, sph_ctx *c, float *disp_by_id)
     if (disp_by_id && c->n_total) {
         k_slot_to_by_id<<<dim3(c->slots / 256), 256, 0, c->st>>>(
             c->dP, c->BS, c->slots, c->ID0, (const float2 *)m->disp, m->tmp2);
-        MCHK(hipMemcpyAsync(disp_by_id, m->tmp2, sizeof(float2) * (size_t)c->n_total,
-                            hipMemcpyDeviceToHost, c->st));
-        MCHK(hipStreamSynchronize(c->st));
+        if (int rc = sph_internal_fetch(c, disp_by_id, m->tmp2,
+                                        sizeof(float2) * (size_t)c->n_total))
+            return merr(rc, "%s", sph_last_error());
     }
     return SPH_OK;
 }
