@@ -176,7 +176,7 @@ void enqueue_sort_tail(sph_ctx *c, const int *id_src, unsigned *key_dst)
     {
         Tick t(c, KSC);
         sph_launch_scatter(c->st, c->slots, c->dP, c->BS, c->ukey, c->uslot, c->start, id_src,
-                           c->perm_src, c->perm_id, key_dst);
+                           c->perm_src, c->perm_id, key_dst, c->plans);
     }
 }
 
@@ -241,6 +241,8 @@ void enqueue_fused_step(sph_ctx *c, bool visc)
 // whose sorts made none.
 void ensure_current_plans(sph_ctx *c)
 {
+    if (!c->plans_ok && c->lists_valid && c->n_total && c->plans.crowded_n)
+        (void)hipMemsetAsync(c->plans.crowded_n, 0, sizeof(unsigned), c->st);
     if (!c->plans_ok && c->lists_valid && c->n_total)
         sph_launch_plan(c->st, c->slots, c->dP, c->BS, c->start, c->K0, c->plans);
     c->plans_ok = true;
@@ -319,13 +321,25 @@ int dalloc(T **p, size_t count)
 }
 
 // What the context's lanes per particle need: the four-lane gathers their
-// plans, sixteen-lane ones in a small grid the one-launch sort's lists.
+// plans, a middle context its list of crowded tiles, sixteen-lane gathers in a
+// small grid the one-launch sort's lists.
 int ensure_lane_buffers(sph_ctx *c)
 {
     const unsigned m = c->cells + 1;
     int rc = SPH_OK;
-    if (c->lanes == 4 && !c->plans.t64)
-        rc = dalloc(&c->plans.t64, (size_t)c->slots / 64);
+    sph_tile_plans &plans = c->plans;
+    const bool listed = c->lanes_ruled && sph_lists_crowded(c->slots, c->lanes);
+    plans.crowded_max = listed ? c->slots / kSphTPB / 8 * 2 : 0; // even: whole rounds of XCDs
+    if ((c->lanes == 4 || listed) && !plans.t64)
+        rc = dalloc(&plans.t64, (size_t)c->slots / 64);
+    if (!rc && listed && !plans.crowded_n)
+        rc = dalloc(&plans.crowded_n, 1);
+    if (!rc && listed && !plans.crowded)
+        rc = dalloc(&plans.crowded, (size_t)c->slots / kSphTPB);
+    if (!listed && plans.crowded) {
+        (void)hipFree(plans.crowded);
+        plans.crowded = nullptr;
+    }
     const bool small = sph_sort_small_fits(m, c->lanes);
     if (!rc && small && !c->cnt2)
         rc = dalloc(&c->cnt2, sph_scan_padded(m));
@@ -658,6 +672,7 @@ void sph_destroy(sph_ctx *c)
                     c->dC,   c->dclock, c->SPOS,    c->SVEL,    c->SPREV,     c->SRHO,
                     c->SID,  c->SK,    c->Sstart,  c->Sclock,  c->dflags, c->MASK,
                     c->dPA,  c->XY,    c->ACC,     c->AOS,     c->plans.t256, c->plans.t64,
+                    c->plans.crowded, c->plans.crowded_n,
                     c->cnt2, c->lists};
     for (void *p : ptrs)
         if (p)
@@ -888,9 +903,10 @@ int sph_set_gather_lanes(sph_ctx *c, int lanes)
         return set_err(SPH_EINVAL, "sph_set_gather_lanes: lanes %d is not 0, 1 or 4", lanes);
     const int want = lanes ? lanes : sph_gather_lanes(c->slots);
     HIPCHK(hipStreamSynchronize(c->st));
-    if (want != c->lanes)
+    if (want != c->lanes || c->lanes_ruled != (lanes == 0))
         free_graphs(c); // the captured steps launch the other kernel variants
     c->lanes = want;
+    c->lanes_ruled = lanes == 0;
     c->plans_ok = false; // the current hash's, for these lanes, when a gather needs them
     return ensure_lane_buffers(c);
 }

@@ -15,6 +15,9 @@ struct sph_reorder_fields {
 // (the four-lane gathers' tiles; null unless the context uses those).
 struct sph_tile_plans {
     sph_tile_plan *t256 = nullptr, *t64 = nullptr;
+    // The crowded ones among the tiles of 256, which four lanes per particle
+    // walk (null: no list): *crowded_n of them, the first crowded_max listed.
+    unsigned *crowded = nullptr, *crowded_n = nullptr, crowded_max = 0;
 };
 
 // The per-cell member lists of a small context's sort (sph_launch_sort_small):
@@ -33,6 +36,8 @@ constexpr unsigned kSphTPB = 256;
 // Lanes per particle (1, 4 or 16) of the gathers of a context with `slots`
 // padded slots, on the current device.
 int sph_gather_lanes(unsigned slots);
+// Whether a context with these lanes lists its crowded tiles.
+bool sph_lists_crowded(unsigned slots, int lanes);
 
 // cap: the reference's bucket cap is on (sph_dev_params::bucket_cap != 0).
 // lanes: lanes per particle of the gathers, 1, 4 or 16 (sph_gather_lanes);
@@ -64,7 +69,8 @@ void sph_launch_scan_apply(hipStream_t st, unsigned *cnt, unsigned m, const unsi
                            unsigned *start);
 void sph_launch_scatter(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                         const unsigned *key, const unsigned *slot, const unsigned *start,
-                        const int *id_src, int *perm_src, int *perm_id, unsigned *key_dst);
+                        const int *id_src, int *perm_src, int *perm_id, unsigned *key_dst,
+                        const sph_tile_plans &plans);
 // skey: the sorted keys the scatter wrote (its key_dst)
 void sph_launch_reorder2(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                          const unsigned *start, const int *perm_src, const int *perm_id,

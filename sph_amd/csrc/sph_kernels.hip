@@ -137,6 +137,20 @@ __device__ __forceinline__ void add_pad(const sph_dev_params &P, unsigned s0, un
 // Tiles: the candidate ranges of one workgroup of sorted particles.  The plan
 // (sph_tile_plan) is uniform over the workgroup, so all of this stays in
 // scalar registers.
+// Middle contexts (sph_lists_crowded) have few workgroups, and their launches
+// last as long as the slowest: in a settling column a twentieth of the tiles
+// has 220 - 300 candidates a particle where the mean is 50.  There the planner
+// lists the tiles of at least kCrowdedAt candidates a particle, and workgroups
+// that start first walk their quarters with four lanes per particle.  us a step
+// of 250k particles, steps 21-84 / 41-104 / 101-164 / 251-314 / 451-514: 70 / 76
+// / 96 / 141 / 194 without, 69 / 70 / 75 / 99 / 139 with (from 80 candidates on 70
+// / 71 / 76 / 99 / 140, from 100 72 / 74 / 77 / 100 / 139).  Sixteen lanes: 2 - 4%
+// slower.  The quarters after a workgroup's own tile instead of in workgroups of
+// their own: 128 where it is 99 now.
+constexpr unsigned kCrowdedAt = 64;
+// These kernels hold both walks, in 84 - 101 VGPRs without scratch.
+constexpr int kMixedMinBlocks = 5;
+constexpr unsigned kCrowded = 2; // in a plan's `wide`: the tile is listed
 struct Tile {
     int off[6];       // LDS index = sorted position + off[segment]
     unsigned tb[6];   // LDS index of the segment's first record
@@ -159,8 +173,8 @@ __device__ __forceinline__ Tile make_tile(const sph_tile_plan &p, unsigned cap)
         T.off[q] = (int)T.total - (int)p.g0[q];
         T.total += p.len[q];
     }
-    T.ok = !p.wide && T.total <= cap;
-    T.rows_ok = !p.wide && T.len[0] + T.len[3] <= cap && T.len[1] + T.len[4] <= cap &&
+    T.ok = !(p.wide & 1u) && T.total <= cap;
+    T.rows_ok = !(p.wide & 1u) && T.len[0] + T.len[3] <= cap && T.len[1] + T.len[4] <= cap &&
                 T.len[2] + T.len[5] <= cap;
     return T;
 }
@@ -191,6 +205,30 @@ __device__ __forceinline__ void make_plan(unsigned p, unsigned tiles,
     const unsigned kf = skey[f] - P.cell_base, kl = skey[min(f + size, end) - 1u] - P.cell_base;
     const unsigned jA = kf / sx, jB = kl / sx;
     const bool wide = jB > jA + 1;
+    // the most candidates of the first, the middle and the last particle of the
+    // whole tile: lane q < 6 counts row q % 3 of the first (q < 3)
+    // or the last, and of the middle
+    unsigned most = 0;
+    if (plans.crowded) {
+        const unsigned f0 = f / kTPB * kTPB, l0 = min(f0 + kTPB, end) - 1u;
+        auto row_of = [&](unsigned s) {
+            const unsigned k = skey[s] - P.cell_base, x = k % sx;
+            const long r = (long)(k / sx) + (long)(q % 3u) - 1;
+            if (q >= 6u || r < 0 || r >= (long)sy)
+                return 0u;
+            const unsigned row = P.cell_base + (unsigned)r * sx;
+            return start[row + (x + 1u < sx ? x + 2u : sx)] - start[row + (x > 0 ? x - 1u : 0u)];
+        };
+        const unsigned e = row_of(q < 3u ? f0 : l0), m = row_of((f0 + l0) / 2u);
+        const int base = (int)(threadIdx.x & 63u & ~7u);
+        auto rows3 = [&](unsigned v, int at) {
+            return (unsigned)(__shfl((int)v, base + at) + __shfl((int)v, base + at + 1) +
+                              __shfl((int)v, base + at + 2));
+        };
+        most = max(max(rows3(e, 0), rows3(e, 3)), rows3(m, 0));
+        if (quarter && most < kCrowdedAt)
+            return; // a quarter that no workgroup takes
+    }
     if (q < 6u) {
         const unsigned rho = q / 3u, j = jA + rho;
         const long r = (long)j + (long)(q % 3u) - 1;
@@ -209,6 +247,13 @@ __device__ __forceinline__ void make_plan(unsigned p, unsigned tiles,
         out->split = jB > jA ? start[P.cell_base + (jA + 1) * sx] : ~0u;
         out->scene = scene;
         out->wide = wide ? 1u : 0u;
+        if (size == kTPB && most >= kCrowdedAt) {
+            const unsigned at = atomicAdd(plans.crowded_n, 1u);
+            if (at < plans.crowded_max) {
+                plans.crowded[at] = n;
+                out->wide |= kCrowded;
+            }
+        }
     }
 }
 
@@ -426,7 +471,7 @@ template <bool NO_PLAN>
 __device__ __forceinline__ unsigned cell_row(const sph_tile_plan &T, bool live, unsigned s,
                                              unsigned key, const sph_dev_params &P)
 {
-    if (NO_PLAN || T.wide)
+    if (NO_PLAN || (T.wide & 1u))
         return (key - P.cell_base) / P.sx;
     return live ? T.jA + (s >= T.split ? 1u : 0u) : 0u;
 }
@@ -492,7 +537,7 @@ __device__ __forceinline__ uint2 walk_group(const sph_tile_plan &plan, Rec *tile
 // PRED: x_prev = x; x += v*dt; boundary; then the new cell key and a slot
 //       in that cell (histogram of the next sort).  Without PRED the
 //       post-viscosity velocity is written to out_pos.
-template <bool GRAV, bool VISC, bool PRED, bool CAP, int LP = 1>
+template <bool GRAV, bool VISC, bool PRED, bool CAP, int LP = 1, bool LISTED = false>
 __device__ __forceinline__ void
 visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
                   const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
@@ -500,12 +545,10 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
                   float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                   unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                   sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
-                  float2 *__restrict__ held_vel, const sph_buckets &lists = {})
+                  float2 *__restrict__ held_vel, float4 *tile, unsigned blk,
+                  const sph_buckets &lists = {})
 {
-
-    __shared__ float4 tile[VISC && LP != 16 ? kTileCap + kSphWalkPad : 1];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
-    const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
     const unsigned s = s0 + threadIdx.x / LP;
     // loads that need no scene parameter go out before the parameters (every
@@ -519,6 +562,8 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
     const float gdt = P.g_neg * P.dt;
+    if (LISTED && (T.wide & kCrowded))
+        return; // four lanes per particle walk it
     if (PRED)
         add_pad(P, s0, cnt);
     if (s0 >= s1)
@@ -639,23 +684,51 @@ k_visc_predict(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS
                sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                float2 *__restrict__ held_vel)
 {
+    __shared__ float4 tile[VISC ? kTileCap + kSphWalkPad : 1];
     visc_predict_tile<GRAV, VISC, PRED, CAP, 1>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
-                                                out_slot, cnt, C, clock, held_vel);
+                                                out_slot, cnt, C, clock, held_vel, tile,
+                                                xcd_block());
 }
 
-// The fused step's variant with four lanes per particle (sph_gather_lanes).
+// The fused step's variant with one lane per particle, and four in crowded
+// tiles.
+template <bool CAP>
+__global__ void __launch_bounds__(kTPB, kMixedMinBlocks)
+k_visc_predict_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, sph_tile_plans plans,
+    const float2 *__restrict__ POS, const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
+    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+    unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
+    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
+    float2 *__restrict__ held_vel)
+{
+    __shared__ float4 tile[kTileCap + kSphWalkPad];
+    const unsigned listed = plans.crowded_max * 4u;
+    if (blockIdx.x < listed) {
+        const unsigned k = blockIdx.x / 4u;
+        if (k < *plans.crowded_n)
+            visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans.t64, POS, VEL, K, start, out_pos,
+            out_key, out_slot, cnt, C, clock, held_vel, tile,
+                plans.crowded[k] * 4u + blockIdx.x % 4u);
+        return;
+    }
+    visc_predict_tile<true, true, true, CAP, 1, true>(Pp, BS, plans.t256, POS, VEL, K, start, out_pos,
+            out_key, out_slot, cnt, C, clock, held_vel, tile,
+        xcd_block(listed));
+}
+
+// With four lanes per particle (sph_gather_lanes).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
-k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-                    const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
-                    const unsigned *__restrict__ K, const unsigned *__restrict__ start,
-                    float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
-                    unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
-                    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
-                    float2 *__restrict__ held_vel)
+k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, const sph_tile_plan *__restrict__ plans,
+    const float2 *__restrict__ POS, const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
+    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+    unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
+    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
+    float2 *__restrict__ held_vel)
 {
-    visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
-                                                out_slot, cnt, C, clock, held_vel);
+    __shared__ float4 tile[kTileCap + kSphWalkPad];
+    visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans, POS, VEL, K, start, out_pos,
+            out_key, out_slot, cnt, C, clock, held_vel, tile, xcd_block());
 }
 
 // Sixteen lanes per particle.
@@ -670,7 +743,7 @@ k_visc_predict_row(const sph_dev_params *__restrict__ Pp, const int *__restrict_
                    float2 *__restrict__ held_vel, sph_buckets lists)
 {
     visc_predict_tile<true, true, true, CAP, 16>(Pp, BS, nullptr, POS, VEL, K, start, out_pos, out_key,
-                                               out_slot, cnt, C, clock, held_vel, lists);
+                                               out_slot, cnt, C, clock, held_vel, nullptr, xcd_block(), lists);
 }
 
 // src/fluid.c:398-413 as a separate pass (phase API).
@@ -864,9 +937,12 @@ __global__ void __launch_bounds__(kTPB)
 k_scatter(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
           const unsigned *__restrict__ key, const unsigned *__restrict__ slot,
           const unsigned *__restrict__ start, const int *__restrict__ id_src,
-          int *__restrict__ perm_src, int *__restrict__ perm_id, unsigned *__restrict__ key_dst)
+          int *__restrict__ perm_src, int *__restrict__ perm_id, unsigned *__restrict__ key_dst,
+          unsigned *__restrict__ crowded_n)
 {
     const unsigned blk = xcd_block();
+    if (blockIdx.x == 0 && threadIdx.x == 0 && crowded_n)
+        *crowded_n = 0; // for the plans that the reorder makes
     const sph_dev_params &P = Pp[BS[blk]];
     const unsigned i = blk * kTPB + threadIdx.x;
     if (i >= P.poff + (unsigned)P.n)
@@ -1149,20 +1225,14 @@ k_plan(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsign
 // ---------------------------------------------------------------------------
 // Density (src/hash.c:190-194, 225-229 with src/fluid.c:527-539) in gather
 // form: each particle sums (1-r/h)^2 and (1-r/h)^3 over its neighbours.
-template <bool CAP, int LP = 1>
+template <bool CAP, int LP = 1, bool LISTED = false>
 __device__ __forceinline__ void
 density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
              const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
              const unsigned *__restrict__ start, float2 *__restrict__ RHO,
-             uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
+             uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C, float2 *tile, unsigned blk)
 {
-
-    // positions only: twice the candidates of the other gathers' float4
-    // tiles in the same LDS bytes, so denser rows stay in LDS at no cost in
-    // occupancy (registers allow 7 workgroups per CU either way)
-    __shared__ float2 tile[LP == 16 ? 1 : 2 * kTileCap + kSphWalkPad];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
-    const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
     const unsigned s = s0 + threadIdx.x / LP;
     // the lane's own particle and the tile's plan, before the scene
@@ -1173,8 +1243,8 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
-    if (s0 >= s1 || P.frozen)
-        return; // a padding workgroup, or a frozen scene
+    if (s0 >= s1 || P.frozen || (LISTED && (T.wide & kCrowded)))
+        return; // a padding workgroup, a frozen scene, or a tile that four lanes walk
     // the candidate rows, before the barriers
     const bool live = s < s1;
     const unsigned key = live ? ks : P.cell_base; // pad lanes: any valid cell
@@ -1249,6 +1319,9 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     report_neighbors(full, half, C);
 }
 
+// Its tiles hold positions only: twice the candidates of the other gathers'
+// float4 tiles in the same LDS bytes, so denser rows stay in LDS at no cost in
+// occupancy (registers allow 7 workgroups per CU either way).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, kGatherMinBlocks)
 k_density(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
@@ -1256,18 +1329,42 @@ k_density(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
           const unsigned *__restrict__ start, float2 *__restrict__ RHO,
           uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
-    density_tile<CAP, 1>(Pp, BS, plans, POS, K, start, RHO, masks, C);
+    __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
+    density_tile<CAP, 1>(Pp, BS, plans, POS, K, start, RHO, masks, C, tile, xcd_block());
 }
 
-// Four lanes per particle.
+// The fused step's variant with one lane per particle, and four in crowded
+// tiles.
+template <bool CAP>
+__global__ void __launch_bounds__(kTPB, kMixedMinBlocks)
+k_density_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, sph_tile_plans plans,
+    const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+    const unsigned *__restrict__ start, float2 *__restrict__ RHO, uint4 *__restrict__ masks,
+    sph_dev_counters *__restrict__ C)
+{
+    __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
+    const unsigned listed = plans.crowded_max * 4u;
+    if (blockIdx.x < listed) {
+        const unsigned k = blockIdx.x / 4u;
+        if (k < *plans.crowded_n)
+            density_tile<CAP, 4>(Pp, BS, plans.t64, POS, K, start, RHO, masks, C, tile,
+                plans.crowded[k] * 4u + blockIdx.x % 4u);
+        return;
+    }
+    density_tile<CAP, 1, true>(Pp, BS, plans.t256, POS, K, start, RHO, masks, C, tile,
+        xcd_block(listed));
+}
+
+// With four lanes per particle (sph_gather_lanes).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
-k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-               const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
-               const unsigned *__restrict__ start, float2 *__restrict__ RHO,
-               uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
+k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, const sph_tile_plan *__restrict__ plans,
+    const float2 *__restrict__ POS, const unsigned *__restrict__ K,
+    const unsigned *__restrict__ start, float2 *__restrict__ RHO, uint4 *__restrict__ masks,
+    sph_dev_counters *__restrict__ C)
 {
-    density_tile<CAP, 4>(Pp, BS, plans, POS, K, start, RHO, masks, C);
+    __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
+    density_tile<CAP, 4>(Pp, BS, plans, POS, K, start, RHO, masks, C, tile, xcd_block());
 }
 
 // Sixteen lanes per particle.
@@ -1278,14 +1375,14 @@ k_density_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
               const unsigned *__restrict__ start, float2 *__restrict__ RHO,
               uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
-    density_tile<CAP, 16>(Pp, BS, nullptr, POS, K, start, RHO, masks, C);
+    density_tile<CAP, 16>(Pp, BS, nullptr, POS, K, start, RHO, masks, C, nullptr, xcd_block());
 }
 
 // Double-density relaxation (src/fluid.c:541-611) in gather form.
 // FUSED adds the velocity update (src/fluid.c:642-653): boundary, then
 // v = (x - x_prev)/dt clamped, and the histogram of the next sort; without
 // FUSED only the relaxed positions are written.
-template <bool FUSED, bool CAP, int LP = 1>
+template <bool FUSED, bool CAP, int LP = 1, bool LISTED = false>
 __device__ __forceinline__ void
 relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
            const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
@@ -1294,12 +1391,10 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
            float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
            unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
            const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
-           unsigned long long *__restrict__ clock, const sph_buckets &lists = {})
+           unsigned long long *__restrict__ clock, float4 *tile, unsigned blk,
+           const sph_buckets &lists = {})
 {
-
-    __shared__ float4 tile[LP == 16 ? 1 : kTileCap + kSphWalkPad];
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
-    const unsigned blk = xcd_block();
     const unsigned s0 = blk * kPer;
     const unsigned s = s0 + threadIdx.x / LP;
     // the lane's own key and the tile's plan, before the scene
@@ -1310,9 +1405,11 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
+    if (LISTED && (T.wide & kCrowded))
+        return; // four lanes per particle walk it
     if (FUSED) {
         add_pad(P, s0, cnt);
-        if (blockIdx.x == 0 && threadIdx.x == 0)
+        if (s0 == 0 && threadIdx.x == 0)
             atomicAdd(clock, 1ull); // one step of simulated time
     }
     if (s0 >= s1)
@@ -1446,24 +1543,52 @@ k_relax(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
         unsigned long long *__restrict__ clock)
 {
+    __shared__ float4 tile[kTileCap + kSphWalkPad];
     relax_tile<FUSED, CAP, 1>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
-                              cnt, masks, C, clock);
+                              cnt, masks, C, clock, tile, xcd_block());
 }
 
-// The fused variant with four lanes per particle.
+// The fused step's variant with one lane per particle, and four in crowded
+// tiles.
+template <bool CAP>
+__global__ void __launch_bounds__(kTPB, CAP ? kMixedMinBlocks - 1 : kMixedMinBlocks)
+k_relax_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, sph_tile_plans plans,
+    const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+    const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
+    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+    float2 *__restrict__ out_vel, unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
+    unsigned *__restrict__ cnt, const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
+    unsigned long long *__restrict__ clock)
+{
+    __shared__ float4 tile[kTileCap + kSphWalkPad];
+    const unsigned listed = plans.crowded_max * 4u;
+    if (blockIdx.x < listed) {
+        const unsigned k = blockIdx.x / 4u;
+        if (k < *plans.crowded_n)
+            relax_tile<true, CAP, 4>(Pp, BS, plans.t64, POS, PREV, RHO, K, start,
+            out_pos, out_vel, out_key, out_slot, cnt, masks, C, clock, tile,
+                plans.crowded[k] * 4u + blockIdx.x % 4u);
+        return;
+    }
+    relax_tile<true, CAP, 1, true>(Pp, BS, plans.t256, POS, PREV, RHO, K, start,
+            out_pos, out_vel, out_key, out_slot, cnt, masks, C, clock, tile,
+        xcd_block(listed));
+}
+
+// With four lanes per particle (sph_gather_lanes).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
-k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-             const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
-             const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
-             const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
-             float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
-             unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
-             const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
-             unsigned long long *__restrict__ clock)
+k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, const sph_tile_plan *__restrict__ plans,
+    const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
+    const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
+    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+    float2 *__restrict__ out_vel, unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
+    unsigned *__restrict__ cnt, const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
+    unsigned long long *__restrict__ clock)
 {
-    relax_tile<true, CAP, 4>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
-                             cnt, masks, C, clock);
+    __shared__ float4 tile[kTileCap + kSphWalkPad];
+    relax_tile<true, CAP, 4>(Pp, BS, plans, POS, PREV, RHO, K, start,
+            out_pos, out_vel, out_key, out_slot, cnt, masks, C, clock, tile, xcd_block());
 }
 
 // Sixteen lanes per particle.
@@ -1479,12 +1604,12 @@ k_relax_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             unsigned long long *__restrict__ clock, sph_buckets lists)
 {
     relax_tile<true, CAP, 16>(Pp, BS, nullptr, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
-                            cnt, masks, C, clock, lists);
+                            cnt, masks, C, clock, nullptr, xcd_block(), lists);
 }
 
 // One piece of a result to pinned host memory and, when the host can read it,
 // the piece's flag: the host copies a piece on while the next ones cross the
-// link, which bounds this kernel (19 us a MB).
+// link, which bounds this kernel (23 us a MB).
 __global__ void __launch_bounds__(kTPB)
 k_to_host(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t bytes,
           unsigned *__restrict__ flags, unsigned mark)
@@ -1834,19 +1959,35 @@ k_load_state(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 #ifndef SPH_SMALL_SCENE_LANES
 #define SPH_SMALL_SCENE_LANES 16
 #endif
-int sph_gather_lanes(unsigned slots)
+static unsigned device_cus()
 {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
         (void)hipGetLastError();
-        return 1;
+        return 0;
     }
-    if (cus <= 0)
+    return cus > 0 ? (unsigned)cus : 0u;
+}
+
+int sph_gather_lanes(unsigned slots)
+{
+    const unsigned long long tiles = slots / kTPB, n = device_cus();
+    if (!n)
         return 1;
-    const unsigned long long tiles = slots / kTPB, n = (unsigned long long)cus;
     const int lanes = 2ull * tiles <= n ? 16 : tiles <= 2ull * n ? 4 : 1;
     return lanes <= SPH_SMALL_SCENE_LANES ? lanes : SPH_SMALL_SCENE_LANES;
+}
+
+// Up to four tiles per CU (262,144 particles on 256 CUs) all workgroups are
+// resident at once; beyond, the mixed kernels' five a CU, where the one-lane
+// kernels have seven, cost more while the fluid is evenly spread than the lists
+// gain (320k particles: 79 against 74 us a step over steps 21-84, 89 against 100
+// over 101-164), and from 1M on the chip is busy with the sum of the work (1M,
+// steps 501-600: 290 against 247).
+bool sph_lists_crowded(unsigned slots, int lanes)
+{
+    return lanes == 1 && slots / kTPB <= 4u * device_cus();
 }
 
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
@@ -1859,6 +2000,9 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
 #define VP(G, V, R, CAP)                                                                         \
     launch(k_visc_predict<G, V, R, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, VEL, K, start, opos, \
            okey, oslot, cnt, C, clock, held_vel)
+#define VPM(CAP)                                                                                 \
+    launch(k_visc_predict_mixed<CAP>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, VEL, K, start,     \
+           opos, okey, oslot, cnt, C, clock, held_vel)
 #define VP4(CAP)                                                                                 \
     launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS,    \
            VEL, K, start, opos, okey, oslot, cnt, C, clock, held_vel)
@@ -1884,6 +2028,11 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
             VP4(true);
         else
             VP4(false);
+    } else if (grav && visc && pred && plans.crowded) {
+        if (cap)
+            VPM(true);
+        else
+            VPM(false);
     } else if (grav && visc && pred)
         VPC(true, true, true);
     else if (grav && !visc && pred)
@@ -1898,6 +2047,7 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
         VPC(true, true, false);
 #undef VP16
 #undef VP4
+#undef VPM
 #undef VPC
 #undef VP
 }
@@ -1963,10 +2113,11 @@ void sph_launch_scan_single(hipStream_t st, unsigned *cnt, unsigned m, unsigned 
 
 void sph_launch_scatter(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
                         const unsigned *key, const unsigned *slot, const unsigned *start,
-                        const int *id_src, int *perm_src, int *perm_id, unsigned *key_dst)
+                        const int *id_src, int *perm_src, int *perm_id, unsigned *key_dst,
+                        const sph_tile_plans &plans)
 {
     launch(k_scatter, GRID(slots), kTPB, st, P, BS, key, slot, start, id_src, perm_src, perm_id,
-           key_dst);
+           key_dst, plans.crowded_n);
 }
 
 void sph_launch_reorder2(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
@@ -2037,10 +2188,16 @@ void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_
         launch(k_density_row<false>, GRID(16 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
                C);
     else if (lanes == 4 && cap)
-        launch(k_density_quad<true>, GRID(4 * slots), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
+        launch(k_density_quad<true>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
                C);
     else if (lanes == 4)
-        launch(k_density_quad<false>, GRID(4 * slots), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
+        launch(k_density_quad<false>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
+               C);
+    else if (plans.crowded && cap)
+        launch(k_density_mixed<true>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, K, start, RHO, masks,
+               C);
+    else if (plans.crowded)
+        launch(k_density_mixed<false>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, K, start, RHO, masks,
                C);
     else if (cap)
         launch(k_density<true>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO, masks, C);
@@ -2058,6 +2215,9 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
 #define RL(F, CAP)                                                                               \
     launch(k_relax<F, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, start, opos, ovel,   \
            okey, oslot, cnt, masks, C, clock)
+#define RLM(CAP)                                                                                 \
+    launch(k_relax_mixed<CAP>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, PREV, RHO, K, start,      \
+           opos, ovel, okey, oslot, cnt, masks, C, clock)
 #define RL4(CAP)                                                                                 \
     launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, PREV, RHO, K, start,  \
            opos, ovel, okey, oslot, cnt, masks, C, clock)
@@ -2073,6 +2233,10 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
         RL4(true);
     else if (fused && lanes == 4)
         RL4(false);
+    else if (fused && plans.crowded && cap)
+        RLM(true);
+    else if (fused && plans.crowded)
+        RLM(false);
     else if (fused && cap)
         RL(true, true);
     else if (fused)
@@ -2083,6 +2247,7 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
         RL(false, false);
 #undef RL16
 #undef RL4
+#undef RLM
 #undef RL
 }
 
