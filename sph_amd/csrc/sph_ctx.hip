@@ -15,6 +15,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
@@ -354,15 +355,17 @@ int ensure_lane_buffers(sph_ctx *c)
 // a page fault for every page of a fresh array) between two transfers.  Here a
 // kernel writes them to pinned memory, a half of the context's ring at a launch,
 // and this call's threads copy the pieces on as they arrive; the link bounds it
-// (23 us a MB).  While the GPU still computes, the helpers touch the array's
-// pages, which changes nothing in them.
+// (23 us a MB).  While the GPU still computes, the helpers have the array's
+// pages made, which changes nothing in them.
 //
 // us of a download, the runtime's copy and this one: 1 MB 91 / 91 (after four
 // steps 289 / 248), 2 MB 141 / 111, 8 MB 492 / 282; 64 steps of 1M particles and
 // their 54 MB 35.8 / 31.7 ms.  Below kFetchLeast the threads' start costs what
 // it gains.  One helper 293 for the 8 MB, three 262 but 73 / 63 for 0.5 MB; four
-// or seven, and halves of 1, 4 or 8 MB, no faster.
-constexpr size_t kFetchLeast = 1u << 20, kFetchHalf = 2u << 20;
+// or seven, and halves of 2, 4 or 8 MB, no faster.  The pages of pinned memory
+// are mapped for the host at their first use, 0.4 ms a MB, so a context is made
+// with its ring touched: a first prediction of 1M particles takes 1.1 ms, else 1.8.
+constexpr size_t kFetchLeast = 1u << 20, kFetchHalf = 1u << 20;
 constexpr int kFetchThreads = 2;
 
 struct Fetch {
@@ -404,13 +407,15 @@ struct Fetch {
     }
     void help(int n)
     {
-        constexpr size_t kPage = 4096;
+        // (a kernel without this advice refuses it, and the copies fault)
+        constexpr size_t kStep = 256u << 10, kPage = 4096;
         const size_t share = (bytes + kFetchThreads - 1) / kFetchThreads;
-        for (size_t at = n * share; at < std::min(bytes, (n + 1) * share); at += kPage) {
-            if (started.load(std::memory_order_relaxed))
+        const size_t first = (size_t)out + n * share, end = (size_t)out + std::min(bytes, (n + 1) * share);
+        for (size_t at = (first + kPage - 1) / kPage * kPage; at + kPage <= end; at += kStep) {
+            const size_t len = std::min(kStep, (end - at) / kPage * kPage);
+            if (started.load(std::memory_order_relaxed) ||
+                madvise((void *)at, len, MADV_POPULATE_WRITE) != 0)
                 break;
-            volatile char *p = out + at;
-            *p = *p;
         }
         {
             std::unique_lock<std::mutex> lock(mutex);
@@ -515,6 +520,7 @@ void alloc_ring(sph_ctx *c)
         return;
     }
     memset(c->ring_flags, 0, flags);
+    memset(c->ring, 0, 2 * c->ring_half); // maps its pages
 }
 
 int check_scene_desc(const sph_scene_desc &d, int idx)
