@@ -261,7 +261,8 @@ int sph_set_bucket_cap(sph_ctx *ctx, int cap);
  * the fused step's gathers.  0 (the default) chooses by size - 16 when the
  * context has at most half a 256-slot tile per CU of the device (a scene of
  * up to 32,768 particles on 256 CUs), 4 up to two (131,072), where a launch's
- * time is set by its slowest workgroups, else 1; 1 and 4 force a shape.
+ * time is set by its slowest workgroups, else 1, with 4 in crowded tiles up to
+ * four tiles per CU (262,144); 1 and 4 force a shape.
  * Results are bit for bit the same either way: the lanes split a particle's
  * candidate tests and pair terms and apply the terms in the same order.  Any
  * other value is SPH_EINVAL. */
