@@ -562,8 +562,8 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
     const float gdt = P.g_neg * P.dt;
-    if (LISTED && (T.wide & kCrowded))
-        return; // four lanes per particle walk it
+    if (LISTED && s0 < s1 && (T.wide & kCrowded))
+        return; // four lanes per particle walk it (a tile of no particle has no plan)
     if (PRED)
         add_pad(P, s0, cnt);
     if (s0 >= s1)
@@ -1405,8 +1405,8 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const sph_dev_params P = Pp[BS[blk / LP]];
     const unsigned s1 = min(s0 + kPer, P.poff + (unsigned)P.n);
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
-    if (LISTED && (T.wide & kCrowded))
-        return; // four lanes per particle walk it
+    if (LISTED && s0 < s1 && (T.wide & kCrowded))
+        return; // four lanes per particle walk it (a tile of no particle has no plan)
     if (FUSED) {
         add_pad(P, s0, cnt);
         if (s0 == 0 && threadIdx.x == 0)
