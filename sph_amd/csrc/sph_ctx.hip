@@ -315,39 +315,63 @@ template <class T>
 int dalloc(T **p, size_t count)
 {
     hipError_t e = hipMalloc((void **)p, sizeof(T) * (count ? count : 1));
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError(); // reported here, and no launch's error
         return set_err(SPH_ENOMEM, "hipMalloc(%zu x %zu B) failed: %s", count, sizeof(T),
                        hipGetErrorString(e));
+    }
     return SPH_OK;
 }
 
-// What the context's lanes per particle need: the four-lane gathers their
-// plans, a middle context its list of crowded tiles, sixteen-lane gathers in a
-// small grid the one-launch sort's lists.
-int ensure_lane_buffers(sph_ctx *c)
+// Give the context `lanes` lanes per particle (ruled: by the size rule), with
+// the memory that they need: the four-lane gathers their plans, a middle context
+// its list of crowded tiles, sixteen-lane gathers in a small grid the one-launch
+// sort's lists.  Nothing changes unless all of it is there.  No work of the
+// context is in flight, and the caller drops its graphs where the shape changes.
+int take_lanes(sph_ctx *c, int lanes, bool ruled)
 {
     const unsigned m = c->cells + 1;
+    const bool listed = ruled && sph_lists_crowded(c->slots, lanes);
+    const bool quarters = listed || lanes == 4, small = sph_sort_small_fits(m, lanes);
+    sph_tile_plans plans = c->plans;
+    unsigned *cnt2 = c->cnt2;
+    int *lists = c->lists;
     int rc = SPH_OK;
-    sph_tile_plans &plans = c->plans;
-    const bool listed = c->lanes_ruled && sph_lists_crowded(c->slots, c->lanes);
-    plans.crowded_max = listed ? c->slots / kSphTPB / 8 * 2 : 0; // even: whole rounds of XCDs
-    if ((c->lanes == 4 || listed) && !plans.t64)
+    if (quarters && !plans.t64)
         rc = dalloc(&plans.t64, (size_t)c->slots / 64);
     if (!rc && listed && !plans.crowded_n)
         rc = dalloc(&plans.crowded_n, 1);
     if (!rc && listed && !plans.crowded)
         rc = dalloc(&plans.crowded, (size_t)c->slots / kSphTPB);
-    if (!listed && plans.crowded) {
-        (void)hipFree(plans.crowded);
-        plans.crowded = nullptr;
+    if (!rc && small && !cnt2)
+        rc = dalloc(&cnt2, sph_scan_padded(m));
+    if (!rc && small && !lists)
+        rc = dalloc(&lists, (size_t)m * kBucketRow);
+    // (the failed array is null like the ones after it)
+    auto release = [&](auto *p, bool yes) {
+        if (p && yes)
+            (void)hipFree(p);
+    };
+    release(plans.t64, rc ? !c->plans.t64 : !quarters);
+    release(plans.crowded_n, rc ? !c->plans.crowded_n : !listed);
+    release(plans.crowded, rc ? !c->plans.crowded : !listed);
+    if (rc) {
+        release(cnt2, !c->cnt2);
+        return rc;
     }
-    const bool small = sph_sort_small_fits(m, c->lanes);
-    if (!rc && small && !c->cnt2)
-        rc = dalloc(&c->cnt2, sph_scan_padded(m));
-    if (!rc && small && !c->lists)
-        rc = dalloc(&c->lists, (size_t)m * kBucketRow);
-    c->small_sort = !rc && small;
-    return rc;
+    if (!quarters)
+        plans.t64 = nullptr;
+    if (!listed)
+        plans.crowded = plans.crowded_n = nullptr;
+    plans.crowded_max = listed ? c->slots / kSphTPB / 8 * 2 : 0; // even: whole rounds of XCDs
+    c->plans = plans;
+    c->cnt2 = cnt2;
+    c->lists = lists;
+    c->small_sort = small;
+    c->lanes = lanes;
+    c->lanes_ruled = ruled;
+    return SPH_OK;
 }
 
 // Large results for the caller's pageable memory.  The runtime's own copy takes
@@ -597,7 +621,6 @@ int sph_create_batch(sph_ctx **out, const sph_scene_desc *scenes, int nscenes)
     }
     c->cells = (unsigned)cells;
     c->slots = (unsigned)slots;
-    c->lanes = sph_gather_lanes(c->slots);
     int rc = SPH_OK;
     const size_t N = c->slots, M = (size_t)c->cells + 1;
     const size_t MP = sph_scan_padded((unsigned)M); // the scan works on whole tiles
@@ -615,7 +638,7 @@ int sph_create_batch(sph_ctx **out, const sph_scene_desc *scenes, int nscenes)
 #undef A
     if (!rc) {
         c->start = c->start_mem + 4; // a spare entry before, 16-byte aligned for the scans
-        rc = ensure_lane_buffers(c);
+        rc = take_lanes(c, sph_gather_lanes(c->slots), true);
     }
     if (!rc) {
         hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
@@ -909,12 +932,13 @@ int sph_set_gather_lanes(sph_ctx *c, int lanes)
         return set_err(SPH_EINVAL, "sph_set_gather_lanes: lanes %d is not 0, 1 or 4", lanes);
     const int want = lanes ? lanes : sph_gather_lanes(c->slots);
     HIPCHK(hipStreamSynchronize(c->st));
-    if (want != c->lanes || c->lanes_ruled != (lanes == 0))
+    const bool changes = want != c->lanes || c->lanes_ruled != (lanes == 0);
+    if (int rc = take_lanes(c, want, lanes == 0))
+        return rc;
+    if (changes)
         free_graphs(c); // the captured steps launch the other kernel variants
-    c->lanes = want;
-    c->lanes_ruled = lanes == 0;
     c->plans_ok = false; // the current hash's, for these lanes, when a gather needs them
-    return ensure_lane_buffers(c);
+    return SPH_OK;
 }
 
 int sph_step_eager(sph_ctx *c, int nsteps)
