@@ -1181,17 +1181,16 @@ int sph_snapshot_save(sph_ctx *c)
     if (int rc = canonicalize(c))
         return rc;
     const size_t N = c->slots, M = (size_t)c->cells + 1;
-    if (!c->SPOS) {
-        int rc = SPH_OK;
+    // made on first use, one by one: a call that found no memory may come again
+    int rc = SPH_OK;
 #define A(p, count)                                                                              \
-    if (!rc)                                                                                     \
+    if (!rc && !c->p)                                                                            \
     rc = dalloc(&c->p, count)
-        A(SPOS, N); A(SVEL, N); A(SPREV, N); A(SRHO, N); A(SID, N); A(SK, N); A(Sstart, M + 3);
-        A(Sclock, 1); A(dflags, c->sc.size());
+    A(SPOS, N); A(SVEL, N); A(SPREV, N); A(SRHO, N); A(SID, N); A(SK, N); A(Sstart, M + 3);
+    A(Sclock, 1); A(dflags, c->sc.size());
 #undef A
-        if (rc)
-            return rc;
-    }
+    if (rc)
+        return rc;
     const size_t b2 = sizeof(float2) * N, b1 = sizeof(unsigned) * N;
     sph_copy_set cs;
     cs.add(c->SPOS, c->POS0, b2);
