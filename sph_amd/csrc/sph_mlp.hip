@@ -249,8 +249,8 @@ __device__ __forceinline__ float walk_group(unsigned n0, const sph_dev_params &P
 }
 
 // A operand of an edge tile: lane l holds edge e0 + l%16, features 4*(l/16)
-// .. +3.  Features 8..15 stand against zero weights: those lanes read the
-// first eight again.
+// .. +3.  Features 8..15 are zero in the model; those lanes read the first eight
+// again, against weights that w1_b makes zero.
 __device__ __forceinline__ bf16x4 edge_tile_a(const EdgeBuf &L, unsigned e0)
 {
     return L.f[e0 + lane() % 16u][(lane() / 16u) & 1u];
@@ -295,11 +295,19 @@ __device__ __forceinline__ bf16x4 turn(bf16x4 x, bf16x4 eye)
     return pack4(mfma(x, eye, d));
 }
 
-// B operand of W1^T for hidden-unit tile t: B[k][c] = W1[16t + c][k].
+// B operand of W1^T for hidden-unit tile t: B[k][c] = W1[16t + c][k].  The
+// padding columns 8..15 stand against repeated features (edge_tile_a) and take no
+// part whatever a caller set them to: zero, or NaN where times zero is NaN.
 __device__ __forceinline__ bf16x4 w1_b(const unsigned short *W1b, int t)
 {
     const unsigned c = 16u * t + lane() % 16u, k = 4u * (lane() / 16u);
-    return *(const bf16x4 *)(W1b + c * kKE + k);
+    uint2 w = *(const uint2 *)(W1b + c * kKE + k);
+    if (k >= 8u) {
+        auto none = [](unsigned x) { return (x & 0x7f80u) == 0x7f80u ? 0x7fc0u : 0u; };
+        w.x = none(w.x) | none(w.x >> 16) << 16;
+        w.y = none(w.y) | none(w.y >> 16) << 16;
+    }
+    return __builtin_bit_cast(bf16x4, w);
 }
 
 // The edge sums of a group: acc[t] += SiLU(W1 f)^T over the first ne edges,
