@@ -519,6 +519,18 @@ hipError_t fetch_ring(sph_ctx *c, void *out, const void *src, size_t bytes)
     return e != hipSuccess ? e : s;
 }
 
+// Is `out` memory that the runtime knows nothing of?  Pinned memory, which the
+// runtime's copy fills straight from the device (54 MB in 1.01 ms, through the
+// ring 1.52), and device memory, which is not for host copies, go to that copy.
+bool pageable(const void *out)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, out) == hipSuccess)
+        return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError(); // (an unknown pointer is an error to some runtimes)
+    return true;
+}
+
 void free_ring(sph_ctx *c)
 {
     if (c->ring)
@@ -1560,7 +1572,7 @@ int sph_selftest_rcp(unsigned lo_bits, unsigned hi_bits, unsigned long long *mis
 
 int sph_internal_fetch(sph_ctx *c, void *out, const void *src, size_t bytes)
 {
-    if (c->ring && bytes >= kFetchLeast) {
+    if (c->ring && bytes >= kFetchLeast && pageable(out)) {
         HIPCHK(fetch_ring(c, out, src, bytes));
         return SPH_OK;
     }

@@ -92,8 +92,8 @@ struct sph_ctx {
 };
 
 // Copy `bytes` of device memory (16-byte aligned, a multiple of 4) to the
-// caller's pageable memory after all work of the context's stream, and wait;
-// defined in sph_ctx.hip.
+// caller's memory after all work of the context's stream, and wait; defined in
+// sph_ctx.hip.
 int sph_internal_fetch(sph_ctx *c, void *out, const void *src, size_t bytes);
 
 // Bring PREV/RHO into the canonical (ID0) order, and make the current hash's
