@@ -359,7 +359,8 @@ struct sph_surrogate {
     // the macro-step plainly from the same start; 0 = off
     int shadow_every = 0;
     float *sh_sum = nullptr;              // per scene: the plain shadow's density sum
-    float *rho_plain = nullptr, *rho_sur = nullptr; // density by caller index
+    float *rho_plain = nullptr, *rho_sur = nullptr; // density by caller index, of
+    size_t rho_slots = 0;                           // contexts of up to so many slots
     float *sh_err = nullptr;              // per scene: sum (sur - plain)^2, sum plain^2
     double sh_stats[8] = {0};             // see sph_surrogate_shadow_stats
 };
@@ -1170,8 +1171,10 @@ int merr(int code, const char *fmt, ...)
 template <class T>
 int malloc_dev(T **p, size_t n)
 {
-    if (hipMalloc((void **)p, sizeof(T) * (n ? n : 1)) != hipSuccess)
+    if (hipMalloc((void **)p, sizeof(T) * (n ? n : 1)) != hipSuccess) {
+        *p = nullptr;
         return merr(SPH_ENOMEM, "hipMalloc of %zu x %zu B failed", n, sizeof(T));
+    }
     return SPH_OK;
 }
 
@@ -1249,6 +1252,21 @@ int ensure_judge(sph_surrogate *m, const sph_ctx *c)
     if (!rc) rc = malloc_dev(&m->sh_sum, ns);
     if (!rc) rc = malloc_dev(&m->sh_err, 2 * ns);
     m->ns = rc ? 0 : ns;
+    return rc;
+}
+
+// The shadows' densities, for the largest context so far.
+int ensure_shadow(sph_surrogate *m, size_t slots)
+{
+    if (m->rho_slots >= slots)
+        return SPH_OK;
+    for (float *p : {m->rho_plain, m->rho_sur})
+        if (p)
+            (void)hipFree(p);
+    m->rho_plain = m->rho_sur = nullptr;
+    int rc = malloc_dev(&m->rho_plain, slots);
+    if (!rc) rc = malloc_dev(&m->rho_sur, slots);
+    m->rho_slots = rc ? 0 : slots;
     return rc;
 }
 
@@ -1697,12 +1715,8 @@ int sph_surrogate_macro_step(sph_surrogate *m, sph_ctx *c, float tol, int *flags
         return merr(SPH_EHIP, "snapshot failed: %s", sph_last_error());
     const unsigned S = c->slots;
     if (nshadow) { // the shadowed scenes' plain macro-step, then back to the start
-        if (!m->rho_plain) {
-            if (int rc = malloc_dev(&m->rho_plain, S))
-                return rc;
-            if (int rc = malloc_dev(&m->rho_sur, S))
-                return rc;
-        }
+        if (int rc = ensure_shadow(m, S))
+            return rc;
         std::vector<int> frozen((size_t)ns), none((size_t)ns, 0);
         for (int s = 0; s < ns; s++)
             frozen[s] = shadow[s] ? 0 : 1;
