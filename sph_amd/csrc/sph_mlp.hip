@@ -1642,6 +1642,8 @@ int sph_surrogate_apply(sph_surrogate *m, sph_ctx *c)
         return merr(SPH_EINVAL, "null argument");
     if (!m->have_pred)
         return merr(SPH_ESTATE, "sph_surrogate_apply: no prediction");
+    if (m->slots < c->slots)
+        return merr(SPH_ESTATE, "sph_surrogate_apply: the prediction is of a smaller context");
     if (int rc = sph_internal_canonicalize(c))
         return rc;
     const unsigned S = c->slots;

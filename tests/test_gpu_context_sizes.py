@@ -1,7 +1,7 @@
-"""Shadow judging with one network on contexts of different sizes: its density
-buffers must grow with the context.  The larger context's states, flags and
-shadow statistics after a smaller one's macro-steps must equal those after a
-larger one's."""
+"""One network on contexts of different sizes.  Shadow judging's density buffers
+must grow with the context: the larger context's states, flags and shadow
+statistics after a smaller one's macro-steps must equal those after a larger
+one's.  A prediction is not applied to a context larger than it covers."""
 import numpy as np
 import pytest
 
@@ -43,3 +43,19 @@ def test_network_goes_on_to_a_larger_context():
     assert a[1] == b[1] and a[2] == b[2]
     same = a[0] == b[0]
     assert same
+
+
+def test_prediction_of_a_smaller_context_is_refused():
+    m = sa.Surrogate(seed=4)
+    small, large = batch(12, 10, seed=1), batch(90, 80, seed=2)
+    m.predict(small)
+    before = large.download()
+    with pytest.raises(sa.SphError, match="smaller context"):
+        m.apply(large)
+    same = large.download().tobytes() == before.tobytes()
+    assert same
+    m.apply(small)  # the prediction is still there
+    m.predict(large)
+    m.apply(large)
+    small.close()
+    large.close()
