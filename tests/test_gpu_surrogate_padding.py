@@ -1,7 +1,8 @@
 """The padding columns of W1 and W3 take no part in the network, whatever finite
-values a caller set them to: predictions, losses and gradients are the same bit
-for bit (up to 8,192 slots, whose partial gradients are one chunk).  A padding
-weight that is no number makes the prediction none, as zero times it does."""
+values a caller set them to: predictions, losses, gradients and the prediction
+after an optimiser step are the same bit for bit (up to 8,192 slots, whose partial
+gradients are one chunk).  A padding weight that is no number makes the prediction
+none, as zero times it does."""
 import numpy as np
 import pytest
 
@@ -30,7 +31,9 @@ def answers(s, p, target):
     m.zero_grads()
     pred = m.predict(s)
     loss = m.backward(s, target)
-    return pred, np.float32(loss), m.grads()
+    grads = m.grads()
+    m.adam(1e-2)
+    return pred, np.float32(loss), grads, m.predict(s)
 
 
 @pytest.mark.parametrize("columns", [slice(6, 8), slice(8, 14), slice(6, 16)])
@@ -44,7 +47,8 @@ def test_padding_columns_have_no_effect(columns):
     w1 = q[sr.oW1:sr.oW2].reshape(sr.H, sr.KE)
     w1[:, columns] = rng.uniform(-3, 3, w1[:, columns].shape)
     q[sr.oW3:sr.oW4].reshape(sr.H, sr.KN)[:, 69:] = rng.uniform(-3, 3, (sr.H, sr.KN - 69))
-    for what, a, b in zip(("prediction", "loss", "gradients"), answers(s, q, target), want):
+    for what, a, b in zip(("prediction", "loss", "gradients", "next prediction"),
+                          answers(s, q, target), want):
         same = a.tobytes() == b.tobytes()
         assert same, what
     m = sa.Surrogate(seed=1)
