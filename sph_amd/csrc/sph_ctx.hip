@@ -16,6 +16,9 @@
 #include <stdlib.h>
 #include <string.h>
 #include <sys/mman.h>
+#ifndef MADV_POPULATE_WRITE
+#define MADV_POPULATE_WRITE 23 // Linux 5.14; older headers lack the name
+#endif
 
 #include <algorithm>
 #include <atomic>
@@ -434,7 +437,8 @@ struct Fetch {
         // (a kernel without this advice refuses it, and the copies fault)
         constexpr size_t kStep = 256u << 10, kPage = 4096;
         const size_t share = (bytes + kFetchThreads - 1) / kFetchThreads;
-        const size_t first = (size_t)out + n * share, end = (size_t)out + std::min(bytes, (n + 1) * share);
+        const size_t first = (size_t)out + n * share;
+        const size_t end = (size_t)out + std::min(bytes, (n + 1) * share);
         for (size_t at = (first + kPage - 1) / kPage * kPage; at + kPage <= end; at += kStep) {
             const size_t len = std::min(kStep, (end - at) / kPage * kPage);
             if (started.load(std::memory_order_relaxed) ||
@@ -644,7 +648,8 @@ int sph_create_batch(sph_ctx **out, const sph_scene_desc *scenes, int nscenes)
     A(POS1, N + kSphWalkPad); A(UPOS, N); A(UVEL, N); A(T2a, N); A(T2b, N);
     A(ID0, N); A(ID1, N); A(perm_src, N); A(perm_id, N); A(pos_of_id, N);
     A(K0, N); A(K1, N); A(ukey, N); A(uslot, N);
-    A(cnt, MP); A(start_mem, MP + 8); A(plans.t256, N / kSphTPB); A(bsum, sph_scan_blocks((unsigned)M));
+    A(cnt, MP); A(start_mem, MP + 8); A(bsum, sph_scan_blocks((unsigned)M));
+    A(plans.t256, N / kSphTPB);
     A(coords, 2 * N); A(MASK, N); A(dP, (size_t)nscenes); A(dPA, (size_t)nscenes); A(ACC, N);
     A(BS, N / kSphTPB); A(dC, 1); A(dclock, 1);
 #undef A
@@ -709,7 +714,7 @@ void sph_destroy(sph_ctx *c)
     void *ptrs[] = {c->POS0, c->VEL,  c->PREV,     c->RHO,     c->POS1,      c->UPOS,
                     c->UVEL, c->T2a,  c->T2b,      c->ID0,     c->ID1,       c->perm_src,
                     c->perm_id, c->pos_of_id, c->K0, c->K1,    c->ukey,      c->uslot,
-                    c->cnt,  c->start_mem, c->bsum,    c->coords,  c->dP,        c->BS,
+                    c->cnt,  c->start_mem, c->bsum, c->coords,     c->dP,        c->BS,
                     c->dC,   c->dclock, c->SPOS,    c->SVEL,    c->SPREV,     c->SRHO,
                     c->SID,  c->SK,    c->Sstart,  c->Sclock,  c->dflags, c->MASK,
                     c->dPA,  c->XY,    c->ACC,     c->AOS,     c->plans.t256, c->plans.t64,
@@ -1100,8 +1105,8 @@ int sph_phase_viscosity(sph_ctx *c)
         return SPH_OK; // empty lists (src/fluid.c:202)
     ensure_current_plans(c);
     sph_launch_visc_predict(c->st, c->slots, false, true, false, c->bucket_cap != 0, c->dP, c->BS,
-                            c->plans, c->POS0, c->VEL, c->K0, c->start, c->UVEL, nullptr, nullptr, c->cnt,
-                            c->dC, c->dclock, nullptr, c->lanes, sph_buckets{});
+                            c->plans, c->POS0, c->VEL, c->K0, c->start, c->UVEL, nullptr, nullptr,
+                            c->cnt, c->dC, c->dclock, nullptr, c->lanes, sph_buckets{});
     HIPCHK(hipMemcpyAsync(c->VEL, c->UVEL, sizeof(float2) * (size_t)c->slots,
                           hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());
@@ -1144,8 +1149,8 @@ int sph_phase_hash(sph_ctx *c, int compute_density)
     cs.add(c->K0, c->K1, b / 2);
     sph_launch_copy(c->st, cs);
     if (compute_density)
-        sph_launch_density(c->st, S, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->K0, c->start,
-                           c->RHO, c->MASK, c->dC, c->lanes);
+        sph_launch_density(c->st, S, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->K0,
+                           c->start, c->RHO, c->MASK, c->dC, c->lanes);
     HIPCHK(hipGetLastError());
     c->lists_valid = true;
     c->hashes++;
@@ -1163,8 +1168,8 @@ int sph_phase_relax(sph_ctx *c)
     if (!c->lists_valid)
         return set_err(SPH_ESTATE, "sph_phase_relax: no hash since upload");
     ensure_current_plans(c);
-    sph_launch_relax(c->st, c->slots, false, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0, c->PREV,
-                     c->RHO, c->K0, c->start, c->UPOS, nullptr, nullptr, nullptr, nullptr,
+    sph_launch_relax(c->st, c->slots, false, c->bucket_cap != 0, c->dP, c->BS, c->plans, c->POS0,
+                     c->PREV, c->RHO, c->K0, c->start, c->UPOS, nullptr, nullptr, nullptr, nullptr,
                      nullptr, c->dC, c->dclock, c->lanes, sph_buckets{});
     HIPCHK(hipMemcpyAsync(c->POS0, c->UPOS, sizeof(float2) * (size_t)c->slots,
                           hipMemcpyDeviceToDevice, c->st));

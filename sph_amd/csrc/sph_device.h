@@ -39,7 +39,7 @@ struct sph_dev_params {
     int frozen;        // 1: the fused step leaves this scene's state unchanged
     int h_pow2;        // 1: h is a power of two with a normal reciprocal, so that
                        //    x / h == x * h_recip for every x (both round x 2^-k once)
-    unsigned near_h2;  // bits of a float a little below h^2 (sph_common_pair)
+    unsigned near_h2;  // bits of a float a little below h^2 (sph_uncommon_pair)
     unsigned bucket_cap; // 0, or the reference's per-cell bucket cap: a particle
                          // ranked bucket_cap or later by id in its cell is in
                          // no neighbour set of the hash (src/hash.c:153-164)
@@ -385,7 +385,7 @@ __device__ __forceinline__ void sph_walk(unsigned s, unsigned key, const sph_dev
     }
 }
 
-// The plan of a tile of consecutive sorted particles (sph_make_plan), made
+// The plan of a tile of consecutive sorted particles (make_plan), made
 // once per sort by the reorder kernel, for every gather that follows.  The
 // candidate rows of the tile's (at most two) cell rows are six segments of
 // the sorted arrays: segment 3 rho + dy + 1 holds, for the particles in cell
@@ -400,8 +400,7 @@ struct alignas(64) sph_tile_plan {
     unsigned g0[6], len[6]; // begin and length of the segments
     unsigned jA;            // cell row of the first particle
     unsigned split;         // sorted position where row jA + 1 begins
-    int scene;
-    unsigned wide;          // 1: more than two cell rows, no segments
+    unsigned wide;          // bit 0: more than two cell rows, no segments
 };
 
 // The candidate rows of a particle in global cell `key`: row dy = -1, 0, 1
@@ -519,7 +518,7 @@ __device__ __forceinline__ sph_pair_term sph_quad_term(const sph_pair_term &t)
 // above h2), branch-free, into a mask
 // of accepted ones, from which the particle's own slot `self` is cleared;
 // non-empty masks wait in a per-lane queue of up to three chunks (mask,
-// source index of bit 0, owner threshold).  Pass 2 drains the queue in the
+// source index of bit 0).  Pass 2 drains the queue in the
 // order the chunks were found, lowest bit first, running body() on each
 // accepted candidate: exactly sph_walk's visiting order, so sums are
 // bit-identical.  The whole wave drains together, at the end and whenever
@@ -532,10 +531,11 @@ __device__ __forceinline__ sph_pair_term sph_quad_term(const sph_pair_term &t)
 // in self's half list when the candidate lies in a forward cell (0,+1),
 // (+1,-1), (+1,0), (+1,+1) or shares self's cell at a later sorted position
 // (cells are sorted by id), i.e. when its sorted position is at least b1 in
-// row +1, self + 1 in row 0 and b2 in row -1.  body(idx, own, rec) receives
-// that test for the candidate when OWN is set (false otherwise); idx is the
-// candidate's index in the source.  mk supplies or keeps the masks of the
-// lane's first chunks (sph_masks_*).  Returns (accepted, in the half list).
+// row +1, self + 1 in row 0 and b2 in row -1.  body(idx, rec, own) may ask that
+// of a pair by own(), which takes the rows' bounds anew from rows() (only
+// coincident pairs ask); idx is the candidate's index in the source.  mk supplies
+// or keeps the masks of the lane's first chunks (sph_masks_*).  Returns
+// (accepted, in the half list).
 //
 // CAP applies the reference's bucket cap `cap`: a candidate ranked cap or
 // later in its cell (its sorted position minus the cell's start) is masked

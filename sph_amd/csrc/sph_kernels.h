@@ -44,8 +44,9 @@ bool sph_lists_crowded(unsigned slots, int lanes);
 // more than one applies to the fused step's variants (grav, visc and pred; fused relax).
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
                              bool cap, const sph_dev_params *P, const int *BS,
-                             const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,
-                             float2 *opos, unsigned *okey, unsigned *oslot, unsigned *cnt,
+                             const sph_tile_plans &plans, const float2 *POS, const float2 *VEL,
+                             const unsigned *K, const unsigned *start, float2 *opos,
+                             unsigned *okey, unsigned *oslot, unsigned *cnt,
                              sph_dev_counters *C, const unsigned long long *clock,
                              float2 *held_vel, int lanes, const sph_buckets &lists);
 void sph_launch_gravity(hipStream_t st, unsigned slots, const sph_dev_params *P, const int *BS,
@@ -98,9 +99,9 @@ constexpr size_t kHostPiece = 32u << 10;
 void sph_launch_to_host(hipStream_t st, const void *src, void *dst, size_t bytes,
                         unsigned *flags, unsigned mark);
 void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_params *P,
-                        const int *BS, const sph_tile_plans &plans, const float2 *POS, const unsigned *K,
-                        const unsigned *start, float2 *RHO, uint4 *masks, sph_dev_counters *C,
-                        int lanes);
+                        const int *BS, const sph_tile_plans &plans, const float2 *POS,
+                        const unsigned *K, const unsigned *start, float2 *RHO, uint4 *masks,
+                        sph_dev_counters *C, int lanes);
 void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
                       const sph_dev_params *P, const int *BS, const sph_tile_plans &plans,
                       const float2 *POS, const float2 *PREV, const float2 *RHO, const unsigned *K,

@@ -245,7 +245,6 @@ __device__ __forceinline__ void make_plan(unsigned p, unsigned tiles,
     } else if (q == 6u) {
         out->jA = jA;
         out->split = jB > jA ? start[P.cell_base + (jA + 1) * sx] : ~0u;
-        out->scene = scene;
         out->wide = wide ? 1u : 0u;
         if (size == kTPB && most >= kCrowdedAt) {
             const unsigned at = atomicAdd(plans.crowded_n, 1u);
@@ -541,8 +540,9 @@ template <bool GRAV, bool VISC, bool PRED, bool CAP, int LP = 1, bool LISTED = f
 __device__ __forceinline__ void
 visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
                   const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
-                  const float2 *__restrict__ VEL, const unsigned *__restrict__ K, const unsigned *__restrict__ start,
-                  float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
+                  const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
+                  const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+                  unsigned *__restrict__ out_key,
                   unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                   sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                   float2 *__restrict__ held_vel, float4 *tile, unsigned blk,
@@ -585,8 +585,7 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
     // sloshing: horizontal box acceleration, applied like gravity
     const bool slosh = GRAV && P.slosh_amp != 0.0f;
     const float sdt = slosh ? sph_slosh_accel(P, *clock) * P.dt : 0.0f;
-    // the lane's own particle and candidate rows, loaded before the planning
-    // barriers
+    // the lane's own particle and candidate rows, loaded before the staging
     const float2 a = a0, av = av0;
     const bool live = s < s1;
     const unsigned key = VISC && live ? ks : P.cell_base; // pad lanes: any valid cell
@@ -650,9 +649,10 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
                 nvy = nvy - t.b;
             };
             auto never = [](bool) {};
-            sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply, never};
-            fh = walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb,
-                                               mk);
+            sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply,
+                                                                                never};
+            fh = walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test,
+                                               sb, mk);
         }
         full = fh.x;
         half = lead ? fh.y : 0u; // a particle's half list counted once
@@ -677,16 +677,17 @@ visc_predict_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__
 template <bool GRAV, bool VISC, bool PRED, bool CAP>
 __global__ void __launch_bounds__(kTPB, kGatherMinBlocks)
 k_visc_predict(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-               const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
-               const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+               const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+               const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
+               const unsigned *__restrict__ start,
                float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
                unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
                sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                float2 *__restrict__ held_vel)
 {
     __shared__ float4 tile[VISC ? kTileCap + kSphWalkPad : 1];
-    visc_predict_tile<GRAV, VISC, PRED, CAP, 1>(Pp, BS, plans, POS, VEL, K, start, out_pos, out_key,
-                                                out_slot, cnt, C, clock, held_vel, tile,
+    visc_predict_tile<GRAV, VISC, PRED, CAP, 1>(Pp, BS, plans, POS, VEL, K, start, out_pos,
+                                                out_key, out_slot, cnt, C, clock, held_vel, tile,
                                                 xcd_block());
 }
 
@@ -694,41 +695,45 @@ k_visc_predict(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS
 // tiles.
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, kMixedMinBlocks)
-k_visc_predict_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, sph_tile_plans plans,
-    const float2 *__restrict__ POS, const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
-    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
-    unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
-    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
-    float2 *__restrict__ held_vel)
+k_visc_predict_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+                     sph_tile_plans plans,
+                     const float2 *__restrict__ POS, const float2 *__restrict__ VEL,
+                     const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+                     float2 *__restrict__ out_pos, unsigned *__restrict__ out_key,
+                     unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
+                     sph_dev_counters *__restrict__ C,
+                     const unsigned long long *__restrict__ clock, float2 *__restrict__ held_vel)
 {
     __shared__ float4 tile[kTileCap + kSphWalkPad];
     const unsigned listed = plans.crowded_max * 4u;
     if (blockIdx.x < listed) {
         const unsigned k = blockIdx.x / 4u;
         if (k < *plans.crowded_n)
-            visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans.t64, POS, VEL, K, start, out_pos,
-            out_key, out_slot, cnt, C, clock, held_vel, tile,
-                plans.crowded[k] * 4u + blockIdx.x % 4u);
+            visc_predict_tile<true, true, true, CAP, 4>(
+                Pp, BS, plans.t64, POS, VEL, K, start, out_pos, out_key, out_slot, cnt, C, clock,
+                held_vel, tile, plans.crowded[k] * 4u + blockIdx.x % 4u);
         return;
     }
-    visc_predict_tile<true, true, true, CAP, 1, true>(Pp, BS, plans.t256, POS, VEL, K, start, out_pos,
-            out_key, out_slot, cnt, C, clock, held_vel, tile,
-        xcd_block(listed));
+    visc_predict_tile<true, true, true, CAP, 1, true>(Pp, BS, plans.t256, POS, VEL, K, start,
+                                                      out_pos, out_key, out_slot, cnt, C, clock,
+                                                      held_vel, tile, xcd_block(listed));
 }
 
 // With four lanes per particle (sph_gather_lanes).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
-k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, const sph_tile_plan *__restrict__ plans,
-    const float2 *__restrict__ POS, const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
-    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
-    unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
-    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
-    float2 *__restrict__ held_vel)
+k_visc_predict_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+                    const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+                    const float2 *__restrict__ VEL, const unsigned *__restrict__ K,
+                    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+                    unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
+                    unsigned *__restrict__ cnt, sph_dev_counters *__restrict__ C,
+                    const unsigned long long *__restrict__ clock, float2 *__restrict__ held_vel)
 {
     __shared__ float4 tile[kTileCap + kSphWalkPad];
     visc_predict_tile<true, true, true, CAP, 4>(Pp, BS, plans, POS, VEL, K, start, out_pos,
-            out_key, out_slot, cnt, C, clock, held_vel, tile, xcd_block());
+                                                out_key, out_slot, cnt, C, clock, held_vel, tile,
+                                                xcd_block());
 }
 
 // Sixteen lanes per particle.
@@ -742,8 +747,9 @@ k_visc_predict_row(const sph_dev_params *__restrict__ Pp, const int *__restrict_
                    sph_dev_counters *__restrict__ C, const unsigned long long *__restrict__ clock,
                    float2 *__restrict__ held_vel, sph_buckets lists)
 {
-    visc_predict_tile<true, true, true, CAP, 16>(Pp, BS, nullptr, POS, VEL, K, start, out_pos, out_key,
-                                               out_slot, cnt, C, clock, held_vel, nullptr, xcd_block(), lists);
+    visc_predict_tile<true, true, true, CAP, 16>(Pp, BS, nullptr, POS, VEL, K, start, out_pos,
+                                                 out_key, out_slot, cnt, C, clock, held_vel,
+                                                 nullptr, xcd_block(), lists);
 }
 
 // src/fluid.c:398-413 as a separate pass (phase API).
@@ -1228,9 +1234,10 @@ k_plan(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, unsign
 template <bool CAP, int LP = 1, bool LISTED = false>
 __device__ __forceinline__ void
 density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-             const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
-             const unsigned *__restrict__ start, float2 *__restrict__ RHO,
-             uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C, float2 *tile, unsigned blk)
+             const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+             const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+             float2 *__restrict__ RHO, uint4 *__restrict__ masks,
+             sph_dev_counters *__restrict__ C, float2 *tile, unsigned blk)
 {
     constexpr unsigned kPer = kTPB / LP; // particles per workgroup
     const unsigned s0 = blk * kPer;
@@ -1245,7 +1252,7 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
     const bool lead = threadIdx.x % LP == 0; // the lane that stores the particle's results
     if (s0 >= s1 || P.frozen || (LISTED && (T.wide & kCrowded)))
         return; // a padding workgroup, a frozen scene, or a tile that four lanes walk
-    // the candidate rows, before the barriers
+    // the candidate rows, before the staging
     const bool live = s < s1;
     const unsigned key = live ? ks : P.cell_base; // pad lanes: any valid cell
     const unsigned j = cell_row<LP == 16>(T, live, s, key, P);
@@ -1307,8 +1314,8 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         };
         auto never = [](bool) {};
         sph_split_body<decltype(term), decltype(apply), decltype(never)> sb{term, apply, never};
-        fh = walk_group<CAP, 2 * kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb,
-                                               mk);
+        fh = walk_group<CAP, 2 * kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test,
+                                               sb, mk);
     }
     if (live && lead) {
         RHO[s] = make_float2(rho, rhon);
@@ -1325,9 +1332,9 @@ density_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, kGatherMinBlocks)
 k_density(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-          const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const unsigned *__restrict__ K,
-          const unsigned *__restrict__ start, float2 *__restrict__ RHO,
-          uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
+          const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+          const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+          float2 *__restrict__ RHO, uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C)
 {
     __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
     density_tile<CAP, 1>(Pp, BS, plans, POS, K, start, RHO, masks, C, tile, xcd_block());
@@ -1337,10 +1344,11 @@ k_density(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 // tiles.
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, kMixedMinBlocks)
-k_density_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, sph_tile_plans plans,
-    const float2 *__restrict__ POS, const unsigned *__restrict__ K,
-    const unsigned *__restrict__ start, float2 *__restrict__ RHO, uint4 *__restrict__ masks,
-    sph_dev_counters *__restrict__ C)
+k_density_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+                sph_tile_plans plans, const float2 *__restrict__ POS,
+                const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+                float2 *__restrict__ RHO, uint4 *__restrict__ masks,
+                sph_dev_counters *__restrict__ C)
 {
     __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
     const unsigned listed = plans.crowded_max * 4u;
@@ -1348,20 +1356,21 @@ k_density_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ B
         const unsigned k = blockIdx.x / 4u;
         if (k < *plans.crowded_n)
             density_tile<CAP, 4>(Pp, BS, plans.t64, POS, K, start, RHO, masks, C, tile,
-                plans.crowded[k] * 4u + blockIdx.x % 4u);
+                                 plans.crowded[k] * 4u + blockIdx.x % 4u);
         return;
     }
     density_tile<CAP, 1, true>(Pp, BS, plans.t256, POS, K, start, RHO, masks, C, tile,
-        xcd_block(listed));
+                               xcd_block(listed));
 }
 
 // With four lanes per particle (sph_gather_lanes).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
-k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, const sph_tile_plan *__restrict__ plans,
-    const float2 *__restrict__ POS, const unsigned *__restrict__ K,
-    const unsigned *__restrict__ start, float2 *__restrict__ RHO, uint4 *__restrict__ masks,
-    sph_dev_counters *__restrict__ C)
+k_density_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+               const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+               const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+               float2 *__restrict__ RHO, uint4 *__restrict__ masks,
+               sph_dev_counters *__restrict__ C)
 {
     __shared__ float2 tile[2 * kTileCap + kSphWalkPad];
     density_tile<CAP, 4>(Pp, BS, plans, POS, K, start, RHO, masks, C, tile, xcd_block());
@@ -1385,9 +1394,10 @@ k_density_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool FUSED, bool CAP, int LP = 1, bool LISTED = false>
 __device__ __forceinline__ void
 relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-           const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
-           const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
-           const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+           const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+           const float2 *__restrict__ PREV, const float2 *__restrict__ RHO,
+           const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+           float2 *__restrict__ out_pos,
            float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
            unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
            const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
@@ -1426,8 +1436,7 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         }
         return;
     }
-    // the lane's own particle and candidate rows, loaded before the planning
-    // barriers
+    // the lane's own particle and candidate rows, loaded before the staging
     const float2 a = POS[s];
     const float2 ar = RHO[s];
     const bool live = s < s1;
@@ -1508,10 +1517,12 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
         sph_split_body<decltype(term), decltype(apply), decltype(nudge)> sb{term, apply, nudge};
         if (FUSED) {
             sph_masks_replay mk{live ? masks[s] : make_uint4(0u, 0u, 0u, 0u)};
-            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb, mk);
+            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb,
+                                          mk);
         } else {
             sph_masks_none mk;
-            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb, mk);
+            walk_group<CAP, kTileCap, LP>(T, tile, load, live, s, R, key, j, P, start, test, sb,
+                                          mk);
         }
     }
     if (!live || !lead)
@@ -1535,60 +1546,63 @@ relax_tile(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
 template <bool FUSED, bool CAP>
 __global__ void __launch_bounds__(kTPB, CAP ? kGatherMinBlocks - 1 : kGatherMinBlocks)
 k_relax(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
-        const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
-        const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
-        const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
+        const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+        const float2 *__restrict__ PREV, const float2 *__restrict__ RHO,
+        const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+        float2 *__restrict__ out_pos,
         float2 *__restrict__ out_vel, unsigned *__restrict__ out_key,
         unsigned *__restrict__ out_slot, unsigned *__restrict__ cnt,
         const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
         unsigned long long *__restrict__ clock)
 {
     __shared__ float4 tile[kTileCap + kSphWalkPad];
-    relax_tile<FUSED, CAP, 1>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
-                              cnt, masks, C, clock, tile, xcd_block());
+    relax_tile<FUSED, CAP, 1>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key,
+                              out_slot, cnt, masks, C, clock, tile, xcd_block());
 }
 
 // The fused step's variant with one lane per particle, and four in crowded
 // tiles.
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, CAP ? kMixedMinBlocks - 1 : kMixedMinBlocks)
-k_relax_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, sph_tile_plans plans,
-    const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
-    const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
-    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
-    float2 *__restrict__ out_vel, unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
-    unsigned *__restrict__ cnt, const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
-    unsigned long long *__restrict__ clock)
+k_relax_mixed(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+              sph_tile_plans plans, const float2 *__restrict__ POS,
+              const float2 *__restrict__ PREV, const float2 *__restrict__ RHO,
+              const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+              float2 *__restrict__ out_pos, float2 *__restrict__ out_vel,
+              unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
+              unsigned *__restrict__ cnt, const uint4 *__restrict__ masks,
+              sph_dev_counters *__restrict__ C, unsigned long long *__restrict__ clock)
 {
     __shared__ float4 tile[kTileCap + kSphWalkPad];
     const unsigned listed = plans.crowded_max * 4u;
     if (blockIdx.x < listed) {
         const unsigned k = blockIdx.x / 4u;
         if (k < *plans.crowded_n)
-            relax_tile<true, CAP, 4>(Pp, BS, plans.t64, POS, PREV, RHO, K, start,
-            out_pos, out_vel, out_key, out_slot, cnt, masks, C, clock, tile,
-                plans.crowded[k] * 4u + blockIdx.x % 4u);
+            relax_tile<true, CAP, 4>(Pp, BS, plans.t64, POS, PREV, RHO, K, start, out_pos,
+                                     out_vel, out_key, out_slot, cnt, masks, C, clock, tile,
+                                     plans.crowded[k] * 4u + blockIdx.x % 4u);
         return;
     }
-    relax_tile<true, CAP, 1, true>(Pp, BS, plans.t256, POS, PREV, RHO, K, start,
-            out_pos, out_vel, out_key, out_slot, cnt, masks, C, clock, tile,
-        xcd_block(listed));
+    relax_tile<true, CAP, 1, true>(Pp, BS, plans.t256, POS, PREV, RHO, K, start, out_pos, out_vel,
+                                   out_key, out_slot, cnt, masks, C, clock, tile,
+                                   xcd_block(listed));
 }
 
 // With four lanes per particle (sph_gather_lanes).
 template <bool CAP>
 __global__ void __launch_bounds__(kTPB, 1)
-k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS, const sph_tile_plan *__restrict__ plans,
-    const float2 *__restrict__ POS, const float2 *__restrict__ PREV,
-    const float2 *__restrict__ RHO, const unsigned *__restrict__ K,
-    const unsigned *__restrict__ start, float2 *__restrict__ out_pos,
-    float2 *__restrict__ out_vel, unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
-    unsigned *__restrict__ cnt, const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
-    unsigned long long *__restrict__ clock)
+k_relax_quad(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
+             const sph_tile_plan *__restrict__ plans, const float2 *__restrict__ POS,
+             const float2 *__restrict__ PREV, const float2 *__restrict__ RHO,
+             const unsigned *__restrict__ K, const unsigned *__restrict__ start,
+             float2 *__restrict__ out_pos, float2 *__restrict__ out_vel,
+             unsigned *__restrict__ out_key, unsigned *__restrict__ out_slot,
+             unsigned *__restrict__ cnt, const uint4 *__restrict__ masks,
+             sph_dev_counters *__restrict__ C, unsigned long long *__restrict__ clock)
 {
     __shared__ float4 tile[kTileCap + kSphWalkPad];
-    relax_tile<true, CAP, 4>(Pp, BS, plans, POS, PREV, RHO, K, start,
-            out_pos, out_vel, out_key, out_slot, cnt, masks, C, clock, tile, xcd_block());
+    relax_tile<true, CAP, 4>(Pp, BS, plans, POS, PREV, RHO, K, start, out_pos, out_vel, out_key,
+                             out_slot, cnt, masks, C, clock, tile, xcd_block());
 }
 
 // Sixteen lanes per particle.
@@ -1603,8 +1617,8 @@ k_relax_row(const sph_dev_params *__restrict__ Pp, const int *__restrict__ BS,
             const uint4 *__restrict__ masks, sph_dev_counters *__restrict__ C,
             unsigned long long *__restrict__ clock, sph_buckets lists)
 {
-    relax_tile<true, CAP, 16>(Pp, BS, nullptr, POS, PREV, RHO, K, start, out_pos, out_vel, out_key, out_slot,
-                            cnt, masks, C, clock, nullptr, xcd_block(), lists);
+    relax_tile<true, CAP, 16>(Pp, BS, nullptr, POS, PREV, RHO, K, start, out_pos, out_vel, out_key,
+                              out_slot, cnt, masks, C, clock, nullptr, xcd_block(), lists);
 }
 
 // One piece of a result to pinned host memory and, when the host can read it,
@@ -1990,25 +2004,32 @@ bool sph_lists_crowded(unsigned slots, int lanes)
     return lanes == 1 && slots / kTPB <= 4u * device_cus();
 }
 
+// The mixed kernels' workgroups: a quarter of a listed tile each, then the tiles.
+static dim3 mixed_grid(unsigned slots, const sph_tile_plans &plans)
+{
+    return dim3(slots / kTPB + 4u * plans.crowded_max);
+}
+
 void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool visc, bool pred,
                              bool cap, const sph_dev_params *P, const int *BS,
-                             const sph_tile_plans &plans, const float2 *POS, const float2 *VEL, const unsigned *K, const unsigned *start,
-                             float2 *opos, unsigned *okey, unsigned *oslot, unsigned *cnt,
+                             const sph_tile_plans &plans, const float2 *POS, const float2 *VEL,
+                             const unsigned *K, const unsigned *start, float2 *opos,
+                             unsigned *okey, unsigned *oslot, unsigned *cnt,
                              sph_dev_counters *C, const unsigned long long *clock,
                              float2 *held_vel, int lanes, const sph_buckets &lists)
 {
 #define VP(G, V, R, CAP)                                                                         \
-    launch(k_visc_predict<G, V, R, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, VEL, K, start, opos, \
-           okey, oslot, cnt, C, clock, held_vel)
+    launch(k_visc_predict<G, V, R, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, VEL, K,  \
+           start, opos, okey, oslot, cnt, C, clock, held_vel)
 #define VPM(CAP)                                                                                 \
-    launch(k_visc_predict_mixed<CAP>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, VEL, K, start,     \
-           opos, okey, oslot, cnt, C, clock, held_vel)
-#define VP4(CAP)                                                                                 \
-    launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS,    \
+    launch(k_visc_predict_mixed<CAP>, mixed_grid(slots, plans), kTPB, st, P, BS, plans, POS,     \
            VEL, K, start, opos, okey, oslot, cnt, C, clock, held_vel)
+#define VP4(CAP)                                                                                 \
+    launch(k_visc_predict_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, VEL, K, \
+           start, opos, okey, oslot, cnt, C, clock, held_vel)
 #define VP16(CAP)                                                                                \
-    launch(k_visc_predict_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, POS, VEL, K, start, opos,   \
-           okey, oslot, cnt, C, clock, held_vel, lists)
+    launch(k_visc_predict_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, POS, VEL, K, start,     \
+           opos, okey, oslot, cnt, C, clock, held_vel, lists)
 #define VPC(G, V, R)                                                                             \
     do {                                                                                         \
         if (cap)                                                                                 \
@@ -2016,7 +2037,7 @@ void sph_launch_visc_predict(hipStream_t st, unsigned slots, bool grav, bool vis
         else                                                                                     \
             VP(G, V, R, false);                                                                  \
     } while (0)
-    // without viscosity the walk does not run: no capped variant; four lanes
+    // without viscosity the walk does not run: no capped variant; several lanes
     // per particle for the fused step's variant only
     if (grav && visc && pred && lanes == 16) {
         if (cap)
@@ -2177,9 +2198,9 @@ void sph_launch_plan(hipStream_t st, unsigned slots, const sph_dev_params *P, co
 }
 
 void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_params *P,
-                        const int *BS, const sph_tile_plans &plans, const float2 *POS, const unsigned *K,
-                        const unsigned *start, float2 *RHO, uint4 *masks, sph_dev_counters *C,
-                        int lanes)
+                        const int *BS, const sph_tile_plans &plans, const float2 *POS,
+                        const unsigned *K, const unsigned *start, float2 *RHO, uint4 *masks,
+                        sph_dev_counters *C, int lanes)
 {
     if (lanes == 16 && cap)
         launch(k_density_row<true>, GRID(16 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
@@ -2188,21 +2209,23 @@ void sph_launch_density(hipStream_t st, unsigned slots, bool cap, const sph_dev_
         launch(k_density_row<false>, GRID(16 * slots), kTPB, st, P, BS, POS, K, start, RHO, masks,
                C);
     else if (lanes == 4 && cap)
-        launch(k_density_quad<true>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
-               C);
+        launch(k_density_quad<true>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, K, start,
+               RHO, masks, C);
     else if (lanes == 4)
-        launch(k_density_quad<false>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, K, start, RHO, masks,
-               C);
+        launch(k_density_quad<false>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, K,
+               start, RHO, masks, C);
     else if (plans.crowded && cap)
-        launch(k_density_mixed<true>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, K, start, RHO, masks,
-               C);
+        launch(k_density_mixed<true>, mixed_grid(slots, plans), kTPB, st, P, BS, plans, POS, K,
+               start, RHO, masks, C);
     else if (plans.crowded)
-        launch(k_density_mixed<false>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, K, start, RHO, masks,
-               C);
+        launch(k_density_mixed<false>, mixed_grid(slots, plans), kTPB, st, P, BS, plans, POS, K,
+               start, RHO, masks, C);
     else if (cap)
-        launch(k_density<true>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO, masks, C);
+        launch(k_density<true>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO,
+               masks, C);
     else
-        launch(k_density<false>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO, masks, C);
+        launch(k_density<false>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, K, start, RHO,
+               masks, C);
 }
 
 void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
@@ -2213,17 +2236,17 @@ void sph_launch_relax(hipStream_t st, unsigned slots, bool fused, bool cap,
                       unsigned long long *clock, int lanes, const sph_buckets &lists)
 {
 #define RL(F, CAP)                                                                               \
-    launch(k_relax<F, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, start, opos, ovel,   \
-           okey, oslot, cnt, masks, C, clock)
+    launch(k_relax<F, CAP>, GRID(slots), kTPB, st, P, BS, plans.t256, POS, PREV, RHO, K, start,  \
+           opos, ovel, okey, oslot, cnt, masks, C, clock)
 #define RLM(CAP)                                                                                 \
-    launch(k_relax_mixed<CAP>, dim3((unsigned)(slots / kTPB) + 4u * plans.crowded_max), kTPB, st, P, BS, plans, POS, PREV, RHO, K, start,      \
-           opos, ovel, okey, oslot, cnt, masks, C, clock)
+    launch(k_relax_mixed<CAP>, mixed_grid(slots, plans), kTPB, st, P, BS, plans, POS, PREV, RHO, \
+           K, start, opos, ovel, okey, oslot, cnt, masks, C, clock)
 #define RL4(CAP)                                                                                 \
-    launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, PREV, RHO, K, start,  \
-           opos, ovel, okey, oslot, cnt, masks, C, clock)
+    launch(k_relax_quad<CAP>, GRID(4 * (slots)), kTPB, st, P, BS, plans.t64, POS, PREV, RHO, K,  \
+           start, opos, ovel, okey, oslot, cnt, masks, C, clock)
 #define RL16(CAP)                                                                                \
-    launch(k_relax_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, POS, PREV, RHO, K, start, opos, \
-           ovel, okey, oslot, cnt, masks, C, clock, lists)
+    launch(k_relax_row<CAP>, GRID(16 * (slots)), kTPB, st, P, BS, POS, PREV, RHO, K, start,      \
+           opos, ovel, okey, oslot, cnt, masks, C, clock, lists)
     // several lanes per particle for the fused step's variant only
     if (fused && lanes == 16 && cap)
         RL16(true);

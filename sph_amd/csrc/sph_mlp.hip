@@ -66,8 +66,6 @@ __device__ __forceinline__ unsigned short f2bf(float f)
     return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 
-__device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float((unsigned)b << 16); }
-
 // Logistic function from the hardware exp2 and reciprocal (1 ulp each): the
 // network is trained and run with this definition on both passes.
 __device__ __forceinline__ float sigm(float x)
@@ -883,7 +881,7 @@ __device__ __forceinline__ unsigned short w1_bits(int i, float x)
 }
 
 // Adam on the fp32 master weights, then refresh the bf16 copies.  Weights
-// of the padding columns (W1 beyond 6 inputs, W3 beyond 69) stay zero.
+// of the padding columns (W1 beyond 6 inputs, W3 beyond 69) stay as they are.
 __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
                        float *__restrict__ v, int n, float lr, float b1, float b2, float eps,
                        float c1, float c2, unsigned short *__restrict__ W1b,
@@ -1730,7 +1728,8 @@ int sph_surrogate_macro_step(sph_surrogate *m, sph_ctx *c, float tol, int *flags
             return merr(SPH_EHIP, "shadow step failed: %s", sph_last_error());
         if (int rc = density_now(c))
             return rc;
-        k_scene_density<<<dim3((unsigned)ns), kDensityTPB, 0, c->st>>>(c->dP, c->RHO, m->sh_sum, m->jmax);
+        k_scene_density<<<dim3((unsigned)ns), kDensityTPB, 0, c->st>>>(c->dP, c->RHO, m->sh_sum,
+                                                                       m->jmax);
         k_rho_by_id<<<dim3(S / 256), 256, 0, c->st>>>(c->dP, c->BS, S, c->RHO, c->ID0,
                                                       m->rho_plain);
         MCHK(hipGetLastError());
