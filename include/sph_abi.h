@@ -248,7 +248,8 @@ int sph_set_scene_frozen(sph_ctx *ctx, const int *flags);
  * rank is taken by id within the cell, which is the reference's insertion
  * order when its pointer array is in id order (a single process:
  * src/geometry.c:56 sets id = array index and nothing reorders the array;
- * the multi-rank exchange renumbers at src/communication.c:240, 428).  cap = 0 (the default) turns the cap off; SPH_REF_MAX_BUCKET is
+ * the multi-rank exchange renumbers at src/communication.c:240, 428).
+ * cap = 0 (the default) turns the cap off; SPH_REF_MAX_BUCKET is
  * the reference's value.  Applies to every scene of the context and to the
  * solver's walks (viscosity, density, relaxation, sph_read_neighbors); the
  * surrogate's learned step does not apply it.  A change applies at once:
@@ -265,7 +266,8 @@ int sph_set_bucket_cap(sph_ctx *ctx, int cap);
  * four tiles per CU (262,144); 1 and 4 force a shape.
  * Results are bit for bit the same either way: the lanes split a particle's
  * candidate tests and pair terms and apply the terms in the same order.  Any
- * other value is SPH_EINVAL. */
+ * other value is SPH_EINVAL; a call that finds no device memory is SPH_ENOMEM
+ * and leaves the context's shape as it was. */
 int sph_set_gather_lanes(sph_ctx *ctx, int lanes);
 /* Sloshing clock offset of one scene: its forcing is evaluated at
  * t = (steps since the last upload or load + steps) * dt, so a scene loaded
@@ -462,9 +464,9 @@ sph_ctx *sph_shim_context(void);
  *   d = 4 dt v + 10 dt^2 a + 0.05 out          (a: sloshing and gravity).
  * BF16 weights and activations on MFMA with FP32 accumulation; FP32 master
  * weights and Adam.  The parameter vector (sph_surrogate_num_params floats)
- * is laid out as W1[64][16] (columns 0-4 features, 5 bias, rest zero),
+ * is laid out as W1[64][16] (columns 0-4 features, 5 bias, the rest unused),
  * W2[64][64], b2[64], W3[64][80] (columns 0-63 sum, 64-67 node features,
- * 68 bias, rest zero), W4[2][64], b4[2].
+ * 68 bias, the rest unused), W4[2][64], b4[2].
  * Arrays "by id" are in caller order (scene offset + id), 2 floats each.
  * ---------------------------------------------------------------------- */
 typedef struct sph_surrogate sph_surrogate;
@@ -489,7 +491,8 @@ int sph_surrogate_backward(sph_surrogate *m, sph_ctx *ctx, const float *target_b
 int sph_surrogate_adam(sph_surrogate *m, float lr, float beta1, float beta2, float eps);
 /* Move every unfrozen scene by the last prediction (x += d with the box
  * clamp, v = d / (4 dt) + 1.5 a dt with the velocity clamp); the state is
- * unhashed afterwards and the clock advances by four steps. */
+ * unhashed afterwards and the clock advances by four steps.  A context larger
+ * than any the network has predicted for is SPH_ESTATE. */
 int sph_surrogate_apply(sph_surrogate *m, sph_ctx *ctx);
 /* One judged macro-step of every scene (see sph_mlp.hip); flags (optional,
  * nscenes ints) marks the scenes re-taken by four plain steps: 1 judged

@@ -19,8 +19,8 @@
 //
 // Work layout: one wavefront per 16 consecutive particles everywhere (the
 // solver context's sorted slots).  The edge passes compact the group's edges
-// into LDS, 16 per MFMA tile.  Every product is taken with the weights as the
-// A operand and the particles (or the edge sums) as columns, because the
+// into LDS, 16 per MFMA tile.  Every product of the node layers is taken with the
+// weights as the A operand and the particles as columns, because the
 // 16x16x16 MFMA returns, per lane, rows 4 (l / 16) .. + 3 of column l % 16: the
 // very layout its B operand takes.  So the layers chain in registers, forward
 // and backward, and where a product needs the other layout (the weight
